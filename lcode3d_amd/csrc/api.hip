@@ -42,15 +42,15 @@ struct lcode_workspace {
     double* zero64 = nullptr;      // N * N FP64 zeros (MIXED: the RHS's
                                    // stand-in for a missing beam array)
     DenseGeom dense{};             // LCODE_SOLVER_DENSE*: matrices, scratch
-    void* tab_mixed = nullptr;     // [M][N]   (DST index, DCT index)
-    void* tab_mixed_t = nullptr;   // [N][M]
-    void* tab_dir = nullptr;       // [M][M]
-    void* tab_neu = nullptr;       // [N][N]
+    double* tab_mixed = nullptr;   // dense: multipliers [M][N] (DST index, DCT index)
+    double* tab_mixed_t = nullptr; // [N][M]
+    double* tab_dir = nullptr;     // [M][M]
+    double* tab_neu = nullptr;     // [N][N]
+    double* tri[4] = {};           // FFT: pass B's tables, rows ld long: sine
+                                   // along i ([M]) and cosine ([N]) with the
+                                   // trick term, then both without it
     double* colsum = nullptr;      // [N]
-    double* lam_i = nullptr;       // [M] eigenvalues k = 1 .. N - 2 (DST)
-    double* lam_j = nullptr;       // [N] eigenvalues k = 0 .. N - 1 (DCT)
-    double lam_add = 0, lam_norm = 1;
-    void* T = nullptr;             // 6 * N * (N + 1) transform scratch (S)
+    void* T = nullptr;             // 6 * N * ld transform scratch (S)
     double* partial = nullptr;     // [N]
     double* p1[5] = {};            // predictor particles (nc * nc)
     double* p2[5] = {};            // corrector particles
@@ -220,11 +220,32 @@ int upload(lcode_workspace* ws, T** dst, const std::vector<T>& src) {
     return LCODE_OK;
 }
 
-// Eigenvalue table in the workspace's transform precision.
-int upload_table(lcode_workspace* ws, void** dst, const std::vector<double>& v) {
-    if (!ws->fp32) return upload(ws, reinterpret_cast<double**>(dst), v);
-    std::vector<float> f(v.begin(), v.end());
-    return upload(ws, reinterpret_cast<float**>(dst), f);
+// Pass B's multipliers of one operator (fields.hip): [rows][ld] values of s =
+// 1 - l for the lines of spectral index k0 .. k0 + lines - 1, eliminated in
+// long double.  dirichlet: zero beyond both ends (M rows); else the cosine
+// transform's ends (N rows), whose last multiplier is the inverse of the last
+// pivot sigma / 2 + s (0 for sigma = 0, where that unknown is set to 0).
+std::vector<double> tri_table(int N, int ld, double h, bool dirichlet, int k0, int lines,
+                              int add) {
+    const int rows = dirichlet ? N - 2 : N;
+    std::vector<double> t((size_t)rows * ld, .5);
+    const long double pi = 3.14159265358979323846264338327950288L;
+    std::vector<long double> sigma(lines), s(lines);
+    for (int c = 0; c < lines; ++c) {
+        const long double w = std::sin((k0 + c) * pi / (2 * (N - 1)));
+        sigma[c] = 4 * w * w + (long double)h * h * add;
+    }
+    for (int i = 0; i < rows; ++i)
+        for (int c = 0; c < lines; ++c) {
+            const bool first = i == 0, last = !dirichlet && i == rows - 1;
+            const long double v = first ? (dirichlet ? sigma[c] + 1 : sigma[c] / 2)
+                                  : last ? sigma[c] / 2 + s[c] : sigma[c] + s[c];
+            // pivot 1 + v, at the last cosine row v itself
+            if (last) s[c] = v > 0 ? 1 - 1 / v : 1;
+            else s[c] = v / (1 + v);
+            t[(size_t)i * ld + c] = (double)s[c];
+        }
+    return t;
 }
 
 bool factor_radices(int L, FftPlan& plan) {
@@ -289,38 +310,35 @@ FieldPlan plan_for(lcode_workspace* ws, int kind, int slot) {
     FieldPlan p{};
     p.kind = kind;
     p.T = static_cast<char*>(ws->T) +
-          (size_t)slot * N * (N + 1) * (ws->fp32 ? sizeof(float) : sizeof(double));
+          (size_t)slot * N * ws->geom.ld * (ws->fp32 ? sizeof(float) : sizeof(double));
+    p.tri_scale = ws->h * ws->h / (2 * (N - 1));
     switch (kind) {
         case F_EY:
         case F_BX:  // DST along x (rows 1..N-2), DCT along y (lcode.py:275-286)
             p.rowsA0 = 1; p.rowsA = M;
             p.xfA = XF_DCT; p.lenA = N; p.colA0 = 0;
-            p.xfB = XF_DST; p.table = ws->tab_mixed_t;
-            p.lamL = ws->lam_j; p.lamK = ws->lam_i; p.lam_add = ws->lam_add;
+            p.xfB = XF_DST; p.table = ws->tab_mixed_t; p.tri = ws->tri[0];
             break;
         case F_EX:
         case F_BY:  // solved on the transposed RHS (lcode.py:287-288)
             p.rowsA0 = 0; p.rowsA = N;
             p.xfA = XF_DST; p.lenA = M; p.colA0 = 1;
-            p.xfB = XF_DCT; p.table = ws->tab_mixed;
-            p.lamL = ws->lam_i; p.lamK = ws->lam_j; p.lam_add = ws->lam_add;
+            p.xfB = XF_DCT; p.table = ws->tab_mixed; p.tri = ws->tri[1];
             break;
         case F_EZ:  // DST-I both ways on the interior (lcode.py:166-182)
             p.rowsA0 = 1; p.rowsA = M;
             p.xfA = XF_DST; p.lenA = M; p.colA0 = 1;
-            p.xfB = XF_DST; p.table = ws->tab_dir;
-            p.lamL = ws->lam_i; p.lamK = ws->lam_i;
+            p.xfB = XF_DST; p.table = ws->tab_dir; p.tri = ws->tri[2];
             break;
         default:    // F_BZ: DCT-I both ways, zero mode dropped (:339-362)
             p.rowsA0 = 0; p.rowsA = N;
             p.xfA = XF_DCT; p.lenA = N; p.colA0 = 0;
-            p.xfB = XF_DCT; p.table = ws->tab_neu;
-            p.lamL = ws->lam_j; p.lamK = ws->lam_j; p.zero_mode = 1;
+            p.xfB = XF_DCT; p.table = ws->tab_neu; p.tri = ws->tri[3];
+            p.zero_mode = 1;
             p.colsum = ws->colsum;
             p.partial = ws->partial;
             break;
     }
-    p.lam_norm = ws->lam_norm;
     return p;
 }
 
@@ -456,27 +474,43 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
         g.costab32 = ws->costab32;
     }
 
-    // Eigenvalue tables, normalisation 1 / (2 (N - 1))^2 folded in
-    // (lcode.py:144-157, :215-231, :316-330).
-    const double norm = (double)(2 * (N - 1)) * (2 * (N - 1));
-    std::vector<double> li(M), lj(N);
-    for (int k = 1; k <= M; ++k) li[k - 1] = lam(k, N, ws->h);
-    for (int k = 0; k < N; ++k) lj[k] = lam(k, N, ws->h);
-    const double add = ws->trick_on ? 1 : 0;
-    std::vector<double> mixed((size_t)M * N), mixed_t((size_t)N * M);
-    for (int a = 0; a < M; ++a)
-        for (int b = 0; b < N; ++b) {
-            const double v = 1 / (li[a] + lj[b] + add) / norm;
-            mixed[(size_t)a * N + b] = v;
-            mixed_t[(size_t)b * M + a] = v;
-        }
-    std::vector<double> dir((size_t)M * M), neu((size_t)N * N);
-    for (int a = 0; a < M; ++a)
-        for (int b = 0; b < M; ++b)
-            dir[(size_t)a * M + b] = 1 / (li[a] + li[b]) / norm;
-    for (int a = 0; a < N; ++a)
-        for (int b = 0; b < N; ++b)
-            neu[(size_t)a * N + b] = (a == 0 && b == 0) ? 0. : 1 / (lj[a] + lj[b]) / norm;
+    const int add = ws->trick_on ? 1 : 0;
+    g.ld = (N + 15) / 16 * 16;   // whole 128-byte lines of FP64 spectra
+    if (ws->solver == LCODE_SOLVER_DENSE64 || ws->solver == LCODE_SOLVER_DENSE_BF16X3) {
+        // Eigenvalue tables, normalisation 1 / (2 (N - 1))^2 folded in
+        // (lcode.py:144-157, :215-231, :316-330).
+        const double norm = (double)(2 * (N - 1)) * (2 * (N - 1));
+        std::vector<double> li(M), lj(N);
+        for (int k = 1; k <= M; ++k) li[k - 1] = lam(k, N, ws->h);
+        for (int k = 0; k < N; ++k) lj[k] = lam(k, N, ws->h);
+        std::vector<double> mixed((size_t)M * N), mixed_t((size_t)N * M);
+        for (int a = 0; a < M; ++a)
+            for (int b = 0; b < N; ++b) {
+                const double v = 1 / (li[a] + lj[b] + add) / norm;
+                mixed[(size_t)a * N + b] = v;
+                mixed_t[(size_t)b * M + a] = v;
+            }
+        std::vector<double> dir((size_t)M * M), neu((size_t)N * N);
+        for (int a = 0; a < M; ++a)
+            for (int b = 0; b < M; ++b)
+                dir[(size_t)a * M + b] = 1 / (li[a] + li[b]) / norm;
+        for (int a = 0; a < N; ++a)
+            for (int b = 0; b < N; ++b)
+                neu[(size_t)a * N + b] = (a == 0 && b == 0) ? 0. : 1 / (lj[a] + lj[b]) / norm;
+        if ((rc = upload(ws, &ws->tab_mixed, mixed)) ||
+            (rc = upload(ws, &ws->tab_mixed_t, mixed_t)) ||
+            (rc = upload(ws, &ws->tab_dir, dir)) || (rc = upload(ws, &ws->tab_neu, neu)))
+            return fail(rc);
+    } else {
+        // the spectral index of pass B's lines is the transform along j:
+        // cosine (k = 0 .. N - 1) where i takes the sine, and the other way
+        // round; Ez sine both ways, Bz cosine both ways
+        if ((rc = upload(ws, &ws->tri[0], tri_table(N, g.ld, ws->h, true, 0, N, add))) ||
+            (rc = upload(ws, &ws->tri[1], tri_table(N, g.ld, ws->h, false, 1, M, add))) ||
+            (rc = upload(ws, &ws->tri[2], tri_table(N, g.ld, ws->h, true, 1, M, 0))) ||
+            (rc = upload(ws, &ws->tri[3], tri_table(N, g.ld, ws->h, false, 0, N, 0))))
+            return fail(rc);
+    }
     // Column sums of the final DCT-I of Bz: the mean of Bz is
     // sum_k colsum[k] sum_i T[k][i] / N^2.
     std::vector<double> colsum(N);
@@ -487,15 +521,7 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
         const long double c = (k == 0 || k == N - 1) ? 1 : 2;
         colsum[k] = (double)(c * s);
     }
-    if ((rc = upload_table(ws, &ws->tab_mixed, mixed))) return fail(rc);
-    if ((rc = upload_table(ws, &ws->tab_mixed_t, mixed_t))) return fail(rc);
-    if ((rc = upload_table(ws, &ws->tab_dir, dir))) return fail(rc);
-    if ((rc = upload_table(ws, &ws->tab_neu, neu))) return fail(rc);
     if ((rc = upload(ws, &ws->colsum, colsum))) return fail(rc);
-    if ((rc = upload(ws, &ws->lam_i, li))) return fail(rc);
-    if ((rc = upload(ws, &ws->lam_j, lj))) return fail(rc);
-    ws->lam_add = add;
-    ws->lam_norm = norm;
 
     {
         // zn diagnostic taps (scipy.ndimage.gaussian_filter1d: truncate 4)
@@ -532,13 +558,11 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
             }
         DenseGeom& d = ws->dense;
         d.prec = ws->solver == LCODE_SOLVER_DENSE64 ? DENSE_F64 : DENSE_BF16X3;
-        double *pS, *pC, *pCT, *pm, *pmt;
+        double *pS, *pC, *pCT;
         if ((rc = upload(ws, &pS, Sd))) return fail(rc);
         if ((rc = upload(ws, &pC, Cd))) return fail(rc);
         if ((rc = upload(ws, &pCT, CdT))) return fail(rc);
-        if ((rc = upload(ws, &pm, mixed))) return fail(rc);
-        if ((rc = upload(ws, &pmt, mixed_t))) return fail(rc);
-        d.Sd = pS; d.Cd = pC; d.CdT = pCT; d.mixed = pm; d.mixed_t = pmt;
+        d.Sd = pS; d.Cd = pC; d.CdT = pCT; d.mixed = ws->tab_mixed; d.mixed_t = ws->tab_mixed_t;
         d.colsum = ws->colsum;
         if ((rc = dev_alloc(ws, (void**)&d.mean, sizeof(double)))) return fail(rc);
         if (d.prec == DENSE_F64) {
@@ -571,8 +595,8 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     }
 
     const size_t n2 = (size_t)N * N, np = (size_t)cfg->nc * cfg->nc;
-    // six N x (N + 1) slots: the wave FFT keeps rows N + 1 long (even)
-    if ((rc = dev_alloc(ws, &ws->T, 6 * (n2 + N) * (ws->fp32 ? sizeof(float) : sizeof(double)))))
+    // the spectra of six fields, [N][ld] each
+    if ((rc = dev_alloc(ws, &ws->T, 6 * (size_t)N * g.ld * (ws->fp32 ? sizeof(float) : sizeof(double)))))
         return fail(rc);
     if ((rc = dev_alloc(ws, (void**)&ws->partial, N * sizeof(double)))) return fail(rc);
     for (int k = 0; k < 5; ++k) {

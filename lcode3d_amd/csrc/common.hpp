@@ -490,15 +490,12 @@ struct FieldPlan {
     int rowsA0, rowsA;        // rows i of the RHS transformed along j
     int xfA, lenA, colA0;     // transform along j: type, length, first j
     int xfB;                  // transform along i (length rowsA)
-    const void* table;        // [lenA][rowsA] spectral multiplier (S)
-    // the same multiplier as 1 / (lamL[line] + lamK[k] + lam_add) / lam_norm
-    // (0 at line = k = 0 when zero_mode): the eigenvalues of the two
-    // transforms, the trick term and the normalisation
-    const double *lamL, *lamK;
-    double lam_add, lam_norm;
-    int zero_mode;
-    void* T;                  // scratch spectra (S): [lenA][rowsA]; in the wave
-                              // FFT [lenA][N + 1], indexed by grid row
+    const double* table;      // dense solvers: [lenA][rowsA] spectral multiplier
+    const double* tri;        // FFT solvers: s = 1 - l of the tridiagonal
+                              // elimination, [rowsA][ld] (pass B)
+    double tri_scale;         // h^2 / (2 (N - 1)): of the right-hand side there
+    int zero_mode;            // Bz: drop the zero mode
+    void* T;                  // scratch spectra (S), [N][ld] by grid row
     const double* colsum;     // Bz only: column sums of the last DCT
     double* partial;          // Bz only: [lenA] mean partials
     const double* prevF;      // Variant A / averaging source (or NULL)
@@ -602,6 +599,7 @@ int launch_diag_zn(const double* ro, const double* w, int r, int N, double* tmp,
 
 struct SolverGeom {
     int N;
+    int ld;                   // row length of the spectra and of pass B's tables
     FftPlan fft;
     const double* costab;     // cos(2 pi r / L), r in [0, L / 4]
     const double2* stage_tw;  // per-stage twiddles of the static plan

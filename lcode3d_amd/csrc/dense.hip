@@ -632,7 +632,7 @@ int launch_solve_bf16x3(int N, const DenseGeom& d, const SolveBatch& b,
         o2.mode = BF_TAB_ROWS; o2.Ch = Xh; o2.Cl = Xl;
         o2.tab = kind == F_EY || kind == F_BX ? d.mixed
                : kind == F_EX || kind == F_BY ? d.mixed_t
-               : static_cast<const double*>(fp.table);
+               : fp.table;
         o2.ldt = C;
         if (kind == F_BZ) { o2.colsum = d.colsum; o2.mean_acc = d.mean; }
         g2.op[f] = o2;
@@ -733,7 +733,7 @@ int launch_solve_dense(int N, const DenseGeom& d, const SolveBatch& b,
         double* Y = d.Y + f * n2;
         const double* tab = fp.kind == F_EY || fp.kind == F_BX ? d.mixed
                           : fp.kind == F_EX || fp.kind == F_BY ? d.mixed_t
-                          : static_cast<const double*>(fp.table);
+                          : fp.table;
         GemmOp o{};
         o.a_off = 0; o.b_off = 0;
         // P1 = T_B R

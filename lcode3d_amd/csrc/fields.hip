@@ -1,25 +1,28 @@
 // Field solves of the xi step (lcode.py:122-364) on gfx950.
 //
-// Every solve is out = T_x T_y (Mat o (T_y T_x rhs)) with T_x, T_y type-1
-// sine or cosine transforms along x (i) and y (j).  The transforms commute,
-// so a solve runs as three passes over lines, batched over all fields:
+// Every solve inverts a five-point operator whose boundary conditions make
+// it diagonal under a type-1 sine or cosine transform along each axis.  Along
+// j the solve transforms; along i it does not: after the transform along j
+// every line k is a tridiagonal system, which two first-order recurrences
+// solve directly (the same matrix, without a forward and an inverse transform
+// along i).  Three passes, batched over all fields:
 //
-//   pass A  one RHS row i per line: assemble the RHS on the fly, transform
-//           along j, store transposed: T[k][i]
-//   pass B  one row k of T per line: transform along i, multiply by the
-//           eigenvalue table, transform along i again, store back in place
-//   pass C  one output row i per line: gather the column T[.][i], transform
-//           along j, then the epilogue (Bz mean, Variant A, averaging)
+//   pass A  RHS rows i: assemble the RHS on the fly, transform along j, store
+//           the spectra row by row, T[i][k]
+//   pass B  the tridiagonal systems along i, in place, a group of lines k per
+//           block
+//   pass C  output rows i: transform T[i][.] along j, then the epilogue (Bz
+//           mean, Variant A, averaging)
 //
-// Each type-1 transform of length n is one complex FFT of length
-// L = 2 (n + 1) (sine) or 2 (n - 1) (cosine) of the odd or even extension;
-// two real lines ride in one complex FFT (real and imaginary parts).  All
-// six fields of a step share L = 2 (N - 1).  The FFT is a mixed-radix
-// (4, 2, 3, 5) Stockham transform in LDS.
+// A type-1 transform of length n is one complex FFT of length L = 2 (n + 1)
+// (sine) or 2 (n - 1) (cosine) of the odd or even extension; two real lines
+// ride in one complex FFT (real and imaginary parts).  All six fields of a
+// step share L = 2 (N - 1).  The FFT is a mixed-radix (4, 2, 3, 5) Stockham
+// transform in LDS.
 //
-// The transforms, the spectra T and the eigenvalue tables are in S = double
-// (plain path) or S = float (mixed-precision path); the RHS assembly, the
-// Bz mean and the epilogue are FP64 in both.
+// The transforms and the spectra T are in S = double (plain path) or S =
+// float (mixed-precision path); the RHS assembly, the recurrences of pass B
+// and their tables, the Bz mean and the epilogue are FP64 in both.
 
 #include "common.hpp"
 
@@ -371,7 +374,6 @@ template <> struct TwSrc<float> {
 template <int L, bool TW_LDS, typename S>
 __device__ __forceinline__ Tw<S> load_twiddles(typename Vec<S>::T* lds,
                                                const SolverGeom& g) {
-    using V = typename Vec<S>::T;
     Tw<S> r{nullptr, nullptr};
     if constexpr (L == 0) {
         S* ct = reinterpret_cast<S*>(lds + (size_t)g.P * padded_len(g.fft.L));
@@ -694,154 +696,196 @@ pass_a_kernel(SolverGeom g, SolveBatch b) {
     for (int k = t; k < fp.lenA; k += Tp) {
         double a, c;
         get_ext(z, fp.xfA, k, a, c);
-        if (va) T[(size_t)k * lines + ra] = (S)a;
-        if (vb) T[(size_t)k * lines + rb] = (S)c;
+        if (va) T[(size_t)(fp.rowsA0 + ra) * g.ld + k] = (S)a;
+        if (vb) T[(size_t)(fp.rowsA0 + rb) * g.ld + k] = (S)c;
     }
 }
 
-constexpr int kMaxPerThread = 4;
-
-// 1: pass B evaluates the spectral multipliers from the eigenvalues (two
-// FP64 divisions per point, no table traffic); 0: it reads the
-// precomputed tables.  Measured at 641^2: pass B 43.9 us evaluated, 41.7 us
-// read, so 0 by default.
-#ifndef LCODE_FFT_TABLE_INLINE
-#define LCODE_FFT_TABLE_INLINE 0
-#endif
-
-// LCODE_PASS_B_WAVES: waves per SIMD the register allocation must allow
-// (6: at most 80 VGPRs; at 641^2 a CU holds three 8-wave FP64 blocks or two
-// 12-wave FP32 blocks, and at 8 the FP64 pass spills).
-#ifndef LCODE_PASS_B_WAVES
-#define LCODE_PASS_B_WAVES 6
-#endif
-template <int L_, bool TW_LDS, typename S>
+// Pass B: the tridiagonal systems along i.  With g = h^2 f / (2 (N - 1)) (the
+// normalisation of the transform along j and its inverse) and sigma = h^2
+// (lambda_k + trick), line k reads
+//   -u(i-1) + (2 + sigma) u(i) - u(i+1) = g(i)
+// with u = 0 beyond both ends (sine along i) or with (1 + sigma / 2) u - u' =
+// g / 2 at them (cosine along i).  Elimination from the top leaves the
+// multipliers l(i) = 1 / (2 + sigma - l(i-1)), all in (0, 1], and
+//   y(i) = g(i) + l(i-1) y(i-1),    u(i) = l(i) (y(i) + u(i+1)).
+// The table holds s = 1 - l, rounded once from long double: where l is near
+// 1 (the smooth lines) 1 - l carries the decay, and y - s y keeps its
+// relative accuracy where l y would not.  No step subtracts like-sized
+// numbers, so the error is that of the transforms it replaces: relative 2-norm
+// 1.5e-16 .. 2.5e-16 against 1.6e-16 .. 2.7e-16 (FFT) for smooth lines at
+// N = 361 .. 1281.
+//
+// A block takes CB lines; lane = (chunk, line) with 64 / CB chunks of R
+// consecutive rows per wave, so a load reads 64 / CB runs of CB values.  Every chunk solves its rows from a zero carry in registers,
+// carries are combined within the wave by shuffles and across the waves
+// through LDS (a carry enters as v + c - S c, S = 1 - prod l of the rows
+// between), and each row then takes its carry.  Bound: HBM and Infinity
+// Cache traffic (8 N^2 values in, and 6 N^2 out per six fields: the
+// multipliers of Ey, Bx and of Ex, By are shared) against a round trip of
+// latency each way; the arithmetic is about 20 FP64 operations per value.
+// Six fields, us per launch, against the transform along i, multiplier and
+// transform back that this replaced: 361^2 28.6 -> 9.4, 641^2 23.4 -> 13.7,
+// 1281^2 122 -> 62, 641^2 with FP32 spectra 17.5 -> 12.9.
+template <int R, int CB, typename S>
 __global__ void __launch_bounds__(1024)
-__attribute__((amdgpu_waves_per_eu(LCODE_PASS_B_WAVES)))
 pass_b_kernel(SolverGeom g, SolveBatch b) {
-    using V = typename Vec<S>::T;
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    V* lds = reinterpret_cast<V*>(lds_raw);
-    __shared__ double red[2][16];
+    constexpr int kChunks = 64 / CB;      // chunks per wave
+    __shared__ double2 agg[2][16][CB];    // (S, v) of each wave, both sweeps
+    __shared__ double red[16][CB];
     if (!gate_open(b.gate)) return;
-    constexpr int kPts = L_ != 0 ? points_per_thread(L_, std::is_same<S, float>::value) : kMaxPerThread;
-    const BlockPos bp = xcd_block();
+    // the fields of one line group adjacent: Ey and Bx (Ex and By) read the
+    // same multipliers
+    const BlockPos bp = xcd_block_rows();
     const FieldPlan& fp = b.f[bp.field];
-    const int Tp = g.Tp, L = g.fft.L;
-    const int lines = fp.lenA, len = fp.rowsA, xf = fp.xfB;
-    if (bp.block * g.P * 2 >= lines) return;
-    const int pair = threadIdx.x / Tp, t = threadIdx.x - pair * Tp;
-    V* z = lds + (size_t)pair * padded_len(L);
-    const Tw<S> tw = load_twiddles<L_, TW_LDS, S>(lds, g);
-    const int la = (bp.block * g.P + pair) * 2, lb = la + 1;
-    const bool va = la < lines, vb = lb < lines;
-    S* rowa = static_cast<S*>(fp.T) + (size_t)la * len;
-    S* rowb = static_cast<S*>(fp.T) + (size_t)lb * len;
+    const int n = fp.rowsA, k0 = bp.block * CB;
+    if (k0 >= fp.lenA) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int col = lane % CB, chunk = wave * kChunks + lane / CB, r0 = chunk * R;
+    const int k = k0 + col, kc = min(k, fp.lenA - 1);
+    const bool neumann = fp.xfB == XF_DCT;
+    S* const T = static_cast<S*>(fp.T) + (size_t)fp.rowsA0 * g.ld;
+    const double* const tab = fp.tri;
+    // (32-bit offsets from uniform bases: a field has at most 2^24 values)
+    auto at = [&](int row) { return (unsigned)(min(max(row, 0), n - 1) * g.ld + kc); };
 
-    if constexpr (L_ != 0) {
-        constexpr int kPer = points_per_thread(L_, std::is_same<S, float>::value);
-        const S* T = static_cast<const S*>(fp.T);
-        const size_t oa = (size_t)(va ? la : 0) * len, ob = (size_t)(vb ? lb : 0) * len;
-        S xa[kPer], xb[kPer];
+    // all loads first, rows clamped in bounds; the rows from n on become
+    // zero rows (s = 1) whose solution is 0
+    double y[R], s[R];
 #pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int nc = min(t + u * Tp, len - 1);
-            xa[u] = T[oa + nc];
-            xb[u] = T[ob + nc];
-        }
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = t + u * Tp;
-            if (n < len)
-                put_ext(z, xf, n, len, L, va ? (double)xa[u] : 0., vb ? (double)xb[u] : 0.);
-        }
-    } else {
-        for (int n = t; n < len; n += Tp)
-            put_ext(z, xf, n, len, L, va ? (double)rowa[n] : 0., vb ? (double)rowb[n] : 0.);
+    for (int i = 0; i < R; ++i) {
+        y[i] = (double)T[at(r0 + i)];
+        s[i] = tab[at(r0 + i)];
     }
-    put_ext_zeros(z, xf, len, t);
-    __syncthreads();
-    fft_any<L_, S>(z, g, tw, t);
-    // the spectral multipliers of this thread's points, all loaded before
-    // their first use (rows and points clamped in bounds, unused values
-    // dropped); loading them before the first transform instead keeps 12
-    // more VGPRs live across it, which spill under the 64-VGPR budget
-    S ta[kPts], tb[kPts];
-    if (LCODE_FFT_TABLE_INLINE) {
-        // evaluated as the tables are built on the host, operation for
-        // operation (the same values, none of the table's HBM traffic)
-        const double lla = fp.lamL[va ? la : 0], llb = fp.lamL[vb ? lb : 0];
+    const double s_before = tab[at(r0 - 1)];
 #pragma unroll
-        for (int u = 0; u < kPts; ++u) {
-            const int kc = min(t + u * Tp, len - 1);
-            const double lk = fp.lamK[kc];
-            const double a = 1 / (lla + lk + fp.lam_add) / fp.lam_norm;
-            const double c = 1 / (llb + lk + fp.lam_add) / fp.lam_norm;
-            ta[u] = (S)(fp.zero_mode && la == 0 && kc == 0 ? 0. : a);
-            tb[u] = (S)c;
-        }
-    } else {
-        const size_t oa = (size_t)(va ? la : 0) * len, ob = (size_t)(vb ? lb : 0) * len;
-        const S* tab = static_cast<const S*>(fp.table);
+    for (int i = 0; i < R; ++i) {
+        const int row = r0 + i;
+        y[i] = row < n ? y[i] * fp.tri_scale : 0.;
+        if (neumann && (row == 0 || row == n - 1)) y[i] *= .5;
+        if (row >= n) s[i] = 1.;
+    }
+    // sum over the rows of column `col` (every thread of the block calls it)
+    auto column_sum = [&](double v) {
 #pragma unroll
-        for (int u = 0; u < kPts; ++u) {
-            const int kc = min(t + u * Tp, len - 1);
-            ta[u] = tab[oa + kc];
-            tb[u] = tab[ob + kc];
-        }
-    }
-
-    S ha[kPts], hb[kPts];
-#pragma unroll
-    for (int u = 0; u < kPts; ++u) {
-        const int k = t + u * Tp;
-        ha[u] = hb[u] = 0;
-        if (k < len) {
-            double a, c;
-            get_ext(z, xf, k, a, c);
-            if (va) ha[u] = (S)a * ta[u];
-            if (vb) hb[u] = (S)c * tb[u];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kPts; ++u) {
-        const int k = t + u * Tp;
-        if (k < len) put_ext(z, xf, k, len, L, (double)ha[u], (double)hb[u]);
-    }
-    put_ext_zeros(z, xf, len, t);
-    __syncthreads();
-    fft_any<L_, S>(z, g, tw, t);
-
-    double sa = 0., sb = 0.;
-    for (int k = t; k < len; k += Tp) {
-        double a, c;
-        get_ext(z, xf, k, a, c);
-        if (va) rowa[k] = (S)a;
-        if (vb) rowb[k] = (S)c;
-        sa += a;
-        sb += c;
-    }
-    if (fp.partial) {
-        // Bz mean: the sum of all Bz equals sum_k colsum[k] * sum_i T[k][i].
-        const int wave = threadIdx.x >> 6;
-        sa = wave_sum(sa);
-        sb = wave_sum(sb);
-        if ((threadIdx.x & 63) == 0) {
-            red[0][wave] = sa;
-            red[1][wave] = sb;
-        }
+        for (int d = CB; d < 64; d *= 2) v += __shfl_xor(v, d, 64);
         __syncthreads();
-        if (t == 0) {
-            const int w0 = (pair * Tp) >> 6, nw = Tp >> 6;
-            double ta = 0., tb = 0.;
-            for (int w = 0; w < nw; ++w) {
-                ta += red[0][w0 + w];
-                tb += red[1][w0 + w];
-            }
-            if (va) fp.partial[la] = fp.colsum[la] * ta;
-            if (vb) fp.partial[lb] = fp.colsum[lb] * tb;
+        if (lane < CB) red[wave][col] = v;
+        __syncthreads();
+        double t = 0.;
+        for (int w = 0; w < waves; ++w) t += red[w][col];
+        return t;
+    };
+    // Bz, k = 0: the operator has the constants as its null space; the zero
+    // mode of the right-hand side and of the solution is dropped (weights
+    // 1/2 at the ends, as the cosine transform sums)
+    const bool zero = fp.zero_mode && k0 == 0;   // (block-uniform)
+    if (zero) {
+        double t = 0.;
+#pragma unroll
+        for (int i = 0; i < R; ++i) t += y[i];
+        t = column_sum(t) / (n - 1);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int row = r0 + i;
+            if (k == 0 && row < n) y[i] -= (row == 0 || row == n - 1) ? .5 * t : t;
         }
+    }
+
+    // forward sweep
+    double v = 0., P = 0., sp = s_before;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        v = fma(-sp, v, y[i] + v);
+        P = fma(sp, 1. - P, P);
+        y[i] = v;
+        sp = s[i];
+    }
+#pragma unroll
+    for (int d = CB; d < 64; d *= 2) {
+        const double Po = __shfl_up(P, d, 64), vo = __shfl_up(v, d, 64);
+        if (lane >= d) {
+            v = fma(-P, vo, v + vo);
+            P = fma(P, 1. - Po, Po);
+        }
+    }
+    if (lane >= 64 - CB) agg[0][wave][col] = make_double2(P, v);
+    P = __shfl_up(P, CB, 64);
+    v = __shfl_up(v, CB, 64);
+    if (lane < CB) P = v = 0.;
+    __syncthreads();
+    double carry = 0.;
+    for (int w = 0; w < wave; ++w) {
+        const double2 a = agg[0][w][col];
+        carry = fma(-a.x, carry, a.y + carry);
+    }
+    carry = fma(-P, carry, v + carry);
+    P = 0.;
+    sp = s_before;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        P = fma(sp, 1. - P, P);
+        y[i] = fma(-P, carry, y[i] + carry);
+        sp = s[i];
+    }
+
+    // backward sweep
+    v = P = 0.;
+#pragma unroll
+    for (int i = R - 1; i >= 0; --i) {
+        const double t = y[i] + v;
+        v = fma(-s[i], t, t);
+        P = fma(s[i], 1. - P, P);
+        y[i] = v;
+    }
+#pragma unroll
+    for (int d = CB; d < 64; d *= 2) {
+        const double Po = __shfl_down(P, d, 64), vo = __shfl_down(v, d, 64);
+        if (lane < 64 - d) {
+            v = fma(-P, vo, v + vo);
+            P = fma(P, 1. - Po, Po);
+        }
+    }
+    if (lane < CB) agg[1][wave][col] = make_double2(P, v);
+    P = __shfl_down(P, CB, 64);
+    v = __shfl_down(v, CB, 64);
+    if (lane >= 64 - CB) P = v = 0.;
+    __syncthreads();
+    carry = 0.;
+    for (int w = waves - 1; w > wave; --w) {
+        const double2 a = agg[1][w][col];
+        carry = fma(-a.x, carry, a.y + carry);
+    }
+    carry = fma(-P, carry, v + carry);
+    P = 0.;
+#pragma unroll
+    for (int i = R - 1; i >= 0; --i) {
+        P = fma(s[i], 1. - P, P);
+        y[i] = fma(-P, carry, y[i] + carry);
+    }
+    if (zero) {
+        double t = 0.;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int row = r0 + i;
+            if (row < n) t += (row == 0 || row == n - 1) ? .5 * y[i] : y[i];
+        }
+        t = column_sum(t) / (n - 1);
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (k == 0) y[i] -= t;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+        if (r0 + i < n && k < fp.lenA) T[at(r0 + i)] = (S)y[i];
+    if (fp.partial) {
+        // Bz mean: the sum of all Bz equals sum_k colsum[k] sum_i T[i][k]
+        double t = 0.;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (r0 + i < n) t += y[i];
+        t = column_sum(t);
+        if (wave == 0 && lane < CB && k < fp.lenA) fp.partial[k] = fp.colsum[k] * t;
     }
 }
 
@@ -872,19 +916,19 @@ pass_c_kernel(SolverGeom g, SolveBatch b) {
     const int ca = ra - fp.rowsA0, cb = rb - fp.rowsA0;
     const bool ha = ra < N && ca >= 0 && ca < fp.rowsA;
     const bool hb = rb < N && cb >= 0 && cb < fp.rowsA;
-    const int stride = fp.rowsA;
-    const S* T = static_cast<const S*>(fp.T);
+    // (rows without data read a valid row, and are dropped)
+    const S* Ta = static_cast<const S*>(fp.T) + (size_t)(ha ? ra : fp.rowsA0) * g.ld;
+    const S* Tb = static_cast<const S*>(fp.T) + (size_t)(hb ? rb : fp.rowsA0) * g.ld;
     if constexpr (L_ != 0) {
-        // every column load of the thread first (addresses clamped in
-        // bounds, unused values dropped), then the LDS stores
+        // every load of the thread first (columns clamped in bounds, unused
+        // values dropped), then the LDS stores
         constexpr int kPer = points_per_thread(L_, std::is_same<S, float>::value);
-        const int cac = ha ? ca : 0, cbc = hb ? cb : 0;
         S xa[kPer], xb[kPer];
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const S* col = T + (size_t)min(t + u * Tp, fp.lenA - 1) * stride;
-            xa[u] = col[cac];
-            xb[u] = col[cbc];
+            const int n = min(t + u * Tp, fp.lenA - 1);
+            xa[u] = Ta[n];
+            xb[u] = Tb[n];
         }
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
@@ -894,11 +938,8 @@ pass_c_kernel(SolverGeom g, SolveBatch b) {
                         hb ? (double)xb[u] : 0.);
         }
     } else {
-        for (int n = t; n < fp.lenA; n += Tp) {
-            const S* col = T + (size_t)n * stride;
-            put_ext(z, fp.xfA, n, fp.lenA, L, ha ? (double)col[ca] : 0.,
-                    hb ? (double)col[cb] : 0.);
-        }
+        for (int n = t; n < fp.lenA; n += Tp)
+            put_ext(z, fp.xfA, n, fp.lenA, L, ha ? (double)Ta[n] : 0., hb ? (double)Tb[n] : 0.);
     }
     put_ext_zeros(z, fp.xfA, fp.lenA, t);
     __syncthreads();
@@ -1081,9 +1122,6 @@ guess_kernel(GuessArgs p) {
 // across lanes, so the passes read and write global memory coalesced.
 // Against the radix-4/5 plan above: four LDS exchanges per transform instead
 // of six, no barrier across waves at L = 1280, a quarter less VALU work.
-// Between the passes the spectra are kept in grid-row order, rows N + 1
-// long, so a pass-A or pass-C line pair (two grid rows) is one aligned
-// 16-byte element per k.
 // ---------------------------------------------------------------------------
 
 // LCODE_FFT_WAVE_POINTS_1280: points per lane at L = 1280, 20 (one wave per
@@ -1285,20 +1323,6 @@ __device__ __forceinline__ void wext_out(const V (&x)[LCODE_WAVE_R1], int xf,
 // lanes): 40 / R1 with FP64 points (two at 20 points per lane, four at 10),
 // twice that with FP32 (three asked for: 168 registers, where the FP32
 // passes of L = 1280 spill at most 6; those of L = 2560 are not launched).
-// LCODE_FFT_WAVE_PAIRS (4): line pairs per block of the wave pass C: a block
-// reads the spectra of P consecutive row pairs together, P 16-byte elements
-// per k in one wave-wide access (pass C 24.2 -> 22.6 us at 641^2 with 4; the
-// same for pass A's stores cost it 26.4 -> 30.0 us: the block barriers of the
-// transform tie its waves' long right-hand-side loads together).
-// At L = 2560 one pair per block: four would take all of a CU's LDS (the
-// 1281^2 step 717 -> 712 xi-steps/s).
-#ifndef LCODE_FFT_WAVE_PAIRS
-#define LCODE_FFT_WAVE_PAIRS 4
-#endif
-template <int L> struct WavePairs {
-    static constexpr int P = L == 1280 ? LCODE_FFT_WAVE_PAIRS : 1;
-};
-
 #define LCODE_WAVE_ATTR(S) \
     __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? 40 / WaveLanes<L>::R1 : 3)))
 
@@ -1326,8 +1350,7 @@ pass_a_wave_kernel(SolverGeom g, SolveBatch b) {
     const BlockPos bp = xcd_block_rows();
     const FieldPlan& fp = b.f[bp.field];
     const int N = g.N, lane = threadIdx.x;
-    // grid rows ga (even) and ga + 1; the spectra keep grid row order with
-    // rows N + 1 long, so the pair is one 16-byte element per k
+    // grid rows ga (even) and ga + 1
     const int ga = bp.block * 2, gb = ga + 1;
     const int ta = ga - fp.rowsA0, tb = gb - fp.rowsA0;   // rows of the transform
     const bool va = ta >= 0 && ta < fp.rowsA, vb = tb >= 0 && tb < fp.rowsA;
@@ -1349,10 +1372,11 @@ pass_a_wave_kernel(SolverGeom g, SolveBatch b) {
     wext_load<L>(z, fp.xfA, lane, x);
     __syncthreads();
     wave_fft<L>(z, x, g.wave_tw, lane);
-    V* Tsp = static_cast<V*>(fp.T);
-    const int rowp = (N + 1) / 2;   // pairs per row of the spectra
+    S* const Ta = static_cast<S*>(fp.T) + (size_t)ga * g.ld;
+    S* const Tb = Ta + g.ld;
     wext_out<L>(x, fp.xfA, lane, [&](int, int k, double a, double c) {
-        Tsp[(size_t)k * rowp + ga / 2] = mk<V>((S)a, (S)c);
+        if (va) Ta[k] = (S)a;
+        if (vb) Tb[k] = (S)c;
     });
 }
 
@@ -1364,39 +1388,9 @@ pass_a_wave_kernel(SolverGeom g, SolveBatch b) {
 #define LCODE_WAVE_C_ATTR(S) \
     __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? 40 / WaveLanes<L>::R1 : LCODE_WAVE_C_F32_WAVES)))
 
-// LCODE_WAVE_TABLE_INLINE (0): the wave pass B evaluates its spectral
-// multipliers instead of reading the table.  LCODE_WAVE_TABLE_EARLY: it
-// loads them before its first transform.
-#ifndef LCODE_WAVE_TABLE_INLINE
-#define LCODE_WAVE_TABLE_INLINE 0
-#endif
-#ifndef LCODE_WAVE_TABLE_EARLY
-#define LCODE_WAVE_TABLE_EARLY 0
-#endif
-
-// Waves per SIMD the FP64 wave pass B at L = 2560 is compiled for (build
-// option): 2 (the other passes' budget, 256 registers: 41 spill to
-// scratch) or 1 (up to 512: 256 VGPRs and 45 AGPRs, no scratch, half the
-// waves).  The 1281^2 plain run: 707.6-708.9 xi-steps/s with 2, 711.5-711.7
-// with 1 (A/B on one box, two runs each).
-#ifndef LCODE_WAVE_B2560_WAVES
-#define LCODE_WAVE_B2560_WAVES 1
-#endif
-// Waves per SIMD of the FP32 wave pass B (build option): 3, as the other
-// FP32 passes, spills 6 registers at L = 1280; 2 (184 VGPRs) spills none:
-// the mixed six-field solve 61.5 -> 59.7-59.9 us at 641^2 (A/B on one
-// box, two runs each).
-#ifndef LCODE_WAVE_B_F32_WAVES
-#define LCODE_WAVE_B_F32_WAVES 2
-#endif
-#define LCODE_WAVE_B_ATTR(S)                                                        \
-    __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? (L == 2560 ? LCODE_WAVE_B2560_WAVES \
-                                                                    : 40 / WaveLanes<L>::R1) \
-                                                      : LCODE_WAVE_B_F32_WAVES)))
-
-template <int L, typename S>
-__global__ void __launch_bounds__(WaveLanes<L>::T) LCODE_WAVE_B_ATTR(S)
-pass_b_wave_kernel(SolverGeom g, SolveBatch b) {
+template <int L, typename S, typename G>
+__global__ void __launch_bounds__(WaveLanes<L>::T) LCODE_WAVE_C_ATTR(S)
+pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
     using V = typename Vec<S>::T;
     constexpr int T = WaveLanes<L>::T;
     constexpr int kPer = (L / 2 + 1 + T - 1) / T;
@@ -1404,146 +1398,38 @@ pass_b_wave_kernel(SolverGeom g, SolveBatch b) {
     if (!gate_open(b.gate)) return;
     const BlockPos bp = xcd_block();
     const FieldPlan& fp = b.f[bp.field];
-    const int lines = fp.lenA, len = fp.rowsA, xf = fp.xfB, lane = threadIdx.x;
-    const int la = bp.block * 2, lb = la + 1;
-    if (la >= lines) return;
-    const bool vb = lb < lines;
-    // spectra rows N + 1 long in grid row order: line k's transform inputs
-    // start at grid row rowsA0
-    const size_t stride = (size_t)g.N + 1;
-    S* rowa = static_cast<S*>(fp.T) + (size_t)la * stride + fp.rowsA0;
-    S* rowb = static_cast<S*>(fp.T) + (size_t)(vb ? lb : la) * stride + fp.rowsA0;
+    const int N = g.N, lane = threadIdx.x;
+    const int ra = bp.block * 2, rb = ra + 1;
+    auto has = [&](int r) { return r < N && r - fp.rowsA0 >= 0 && r - fp.rowsA0 < fp.rowsA; };
+    const bool ha = has(ra), hb = has(rb);
     {
+        // (rows without data read a valid row, and are dropped)
+        const S* Ta = static_cast<const S*>(fp.T) + (size_t)(ha ? ra : fp.rowsA0) * g.ld;
+        const S* Tb = static_cast<const S*>(fp.T) + (size_t)(hb ? rb : fp.rowsA0) * g.ld;
         S xa[kPer], xb[kPer];
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int n = min(lane + u * T, len - 1);
-            xa[u] = rowa[n];
-            xb[u] = rowb[n];
+            const int n = min(lane + u * T, fp.lenA - 1);
+            xa[u] = Ta[n];
+            xb[u] = Tb[n];
         }
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             const int n = lane + u * T;
-            if (n < len) z[n] = mk<V>(xa[u], vb ? xb[u] : (S)0);
-        }
-    }
-    // the spectral multipliers of this lane's outputs (or,
-    // LCODE_WAVE_TABLE_INLINE, evaluated from the eigenvalues as the host
-    // builds the table: the same correctly rounded divisions); with
-    // LCODE_WAVE_TABLE_EARLY their loads are in flight during the first
-    // transform
-    S ma[LCODE_WAVE_R1], mb[LCODE_WAVE_R1];
-    auto multipliers = [&]() {
-        if (LCODE_WAVE_TABLE_INLINE) {
-            const double lla = fp.lamL[la], llb = fp.lamL[vb ? lb : la];
-            wext_index<L>(xf, lane, [&](int u, int k) {
-                const double lk = fp.lamK[k];
-                const double va = 1 / (lla + lk + fp.lam_add) / fp.lam_norm;
-                ma[u] = (S)(fp.zero_mode && la == 0 && k == 0 ? 0. : va);
-                mb[u] = (S)(1 / (llb + lk + fp.lam_add) / fp.lam_norm);
-            });
-        } else {
-            const S* tab = static_cast<const S*>(fp.table);
-            const S* ta = tab + (size_t)la * len;
-            const S* tb = tab + (size_t)(vb ? lb : la) * len;
-            wext_index<L>(xf, lane, [&](int u, int k) {
-                ma[u] = ta[k];
-                mb[u] = tb[k];
-            });
-        }
-    };
-    if (LCODE_WAVE_TABLE_EARLY) multipliers();
-    __syncthreads();
-    V x[LCODE_WAVE_R1];
-    wext_load<L>(z, xf, lane, x);
-    __syncthreads();
-    wave_fft<L>(z, x, g.wave_tw, lane);
-    {
-        if (!LCODE_WAVE_TABLE_EARLY) multipliers();
-        wext_out<L>(x, xf, lane, [&](int u, int k, double a, double c) {
-            z[k] = mk<V>((S)a * ma[u], vb ? (S)c * mb[u] : (S)0);
-        });
-    }
-    __syncthreads();
-    wext_load<L>(z, xf, lane, x);
-    __syncthreads();
-    wave_fft<L>(z, x, g.wave_tw, lane);
-    double sa = 0., sb = 0.;
-    wext_out<L>(x, xf, lane, [&](int, int k, double a, double c) {
-        rowa[k] = (S)a;
-        if (vb) rowb[k] = (S)c;
-        sa += a;
-        sb += c;
-    });
-    if (fp.partial) {
-        // Bz mean: the sum of all Bz equals sum_k colsum[k] * sum_i T[k][i]
-        double* scratch = reinterpret_cast<double*>(z);
-        sa = block_sum_waves(sa, scratch);
-        sb = block_sum_waves(sb, scratch);
-        if (lane == 0) {
-            fp.partial[la] = fp.colsum[la] * sa;
-            if (vb) fp.partial[lb] = fp.colsum[lb] * sb;
-        }
-    }
-}
-
-template <int L, typename S, typename G>
-__global__ void __launch_bounds__(WaveLanes<L>::T * WavePairs<L>::P) LCODE_WAVE_C_ATTR(S)
-pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
-    using V = typename Vec<S>::T;
-    constexpr int T = WaveLanes<L>::T, P = WavePairs<L>::P, NT = T * P;
-    constexpr int kPer = (L / 2 + 1 + T - 1) / T;
-    constexpr int kZ = T * LCODE_WAVE_R1;   // LDS points per line pair
-    // pair p's staged inputs start kStage p points into its LDS (64 bytes
-    // apart: the four lanes storing one k hit different banks)
-    constexpr int kStage = P > 1 ? 4 : 0;
-    static_assert(L / 2 + 1 + kStage * (P - 1) <= kZ, "staged inputs fit the pair's LDS");
-    __shared__ V zall[P * kZ];
-    if (!gate_open(b.gate)) return;
-    const BlockPos bp = xcd_block();
-    const FieldPlan& fp = b.f[bp.field];
-    const int N = g.N, w = threadIdx.x / T, lane = threadIdx.x % T;
-    V* z = zall + w * kZ;
-    // this wave's pair of output rows; a pair beyond the grid (the last
-    // block) runs through the barriers and emits nothing
-    const int ra = (bp.block * P + w) * 2, rb = ra + 1;
-    const bool live = ra < N;
-    auto has = [&](int r) { return r < N && r - fp.rowsA0 >= 0 && r - fp.rowsA0 < fp.rowsA; };
-    const bool ha = has(ra), hb = has(rb);
-    {
-        // the block's P pairs of grid rows are P consecutive 16-byte
-        // elements per k of the spectra (rows N + 1 long, grid row order):
-        // the block reads them together, 16 k per wave-wide load, into each
-        // pair's LDS; rows without data hold stale values and are dropped
-        const V* Tsp = static_cast<const V*>(fp.T);
-        const int rowp = (N + 1) / 2;
-        V xv[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int idx = threadIdx.x + u * NT;
-            const int k = min(idx / P, fp.lenA - 1), pr = bp.block * P + idx % P;
-            xv[u] = Tsp[(size_t)k * rowp + min(pr, rowp - 1)];
-        }
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int idx = threadIdx.x + u * NT;
-            const int k = idx / P, p = idx % P, r0 = (bp.block * P + p) * 2;
-            if (k < fp.lenA && r0 < N)
-                zall[p * kZ + kStage * p + k] =
-                    mk<V>(has(r0) ? xv[u].x : (S)0, has(r0 + 1) ? xv[u].y : (S)0);
+            if (n < fp.lenA) z[n] = mk<V>(ha ? xa[u] : (S)0, hb ? xb[u] : (S)0);
         }
     }
     __syncthreads();
     V x[LCODE_WAVE_R1];
-    wext_load<L>(z + kStage * w, fp.xfA, lane, x);
+    wext_load<L>(z, fp.xfA, lane, x);
     __syncthreads();
     wave_fft<L>(z, x, g.wave_tw, lane);
 
     double mean = 0.;
     if (fp.partial) {
         double s = 0.;
-        for (int k = threadIdx.x; k < fp.lenA; k += NT) s += fp.partial[k];
-        mean = block_sum_waves(s, reinterpret_cast<double*>(zall)) / ((double)N * N);
+        for (int k = lane; k < fp.lenA; k += T) s += fp.partial[k];
+        mean = block_sum_waves(s, reinterpret_cast<double*>(z)) / ((double)N * N);
     }
     const bool transverse = fp.kind == F_EX || fp.kind == F_EY ||
                             fp.kind == F_BX || fp.kind == F_BY;
@@ -1587,7 +1473,7 @@ pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
         if (!ha) va = 0.;
         if (!hb) vb = 0.;
     };
-    if (live) {
+    {
         constexpr int kOut = LCODE_WAVE_R1 / 2;   // registers with q < R / 2
         G pa[kOut], pb[kOut], qa[kOut], qb[kOut];
 #pragma unroll
@@ -1615,7 +1501,7 @@ pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
             if (rb < N) emit(rb, j, vb, pb[s], qb[s]);
         }
     }
-    if (live && lane == 0) {
+    if (lane == 0) {
         double va, vb;
         value(R / 2, H, va, vb);
         emit(ra, H, va, prevF ? (double)prevF[oa + H] : 0., guess ? (double)guess[oa + H] : 0.);
@@ -1623,7 +1509,7 @@ pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
             emit(rb, H, vb, prevF ? (double)prevF[ob + H] : 0., guess ? (double)guess[ob + H] : 0.);
     }
     if (b.resid) {
-        double* scratch = reinterpret_cast<double*>(zall);
+        double* scratch = reinterpret_cast<double*>(z);
         r_num = block_sum_waves(r_num, scratch);
         r_den = block_sum_waves(r_den, scratch);
         if (threadIdx.x == 0) {
@@ -1636,10 +1522,44 @@ pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
 
 }  // namespace
 
+// Pass B's shape: 8 lines per block (a wave reads runs of 64 bytes) and 12
+// rows per thread, while 16 waves of 8 chunks hold a line (1536 rows); 6 rows
+// on short lines, where the chain of one thread is the whole time; beyond
+// 1536 rows 4 lines and 16 rows, for 4096 rows (more than any transform length
+// that fits LDS).  Six fields at 129^2 / 361^2 / 641^2 / 1281^2, us per launch
+// (rows x lines): 6 x 8 5.9 / 9.3 / 18.5 / -, 12 x 8 6.6 / 9.5 / 13.7 / 61.6,
+// 16 x 8 7.4 / 10.0 / 19.6 / -, 24 x 8 8.3 / 11.3 / 14.8 / 63.1 (fewer rows:
+// more carries to combine; more: too few waves); 12 x 16 6.8 / 9.8 / 16.4 / -,
+// 12 x 4 6.3 / 9.6 / 15.8 / 79.6 (longer and shorter runs).
+template <typename S>
+static int launch_pass_b(const SolverGeom& g, const SolveBatch& b, hipStream_t s,
+                         Profiler* prof) {
+    int rows = 0, lines = 0;
+    for (int f = 0; f < b.nfields; ++f) {
+        rows = rows > b.f[f].rowsA ? rows : b.f[f].rowsA;
+        lines = lines > b.f[f].lenA ? lines : b.f[f].lenA;
+    }
+    ProfScope ps(prof, "solve_pass_b", s, true);
+    auto go = [&](auto kernel, int R, int CB) {
+        const int per_wave = R * (64 / CB);
+        launch_timed(ps, kernel, dim3((lines + CB - 1) / CB, b.nfields),
+                     dim3(64 * ((rows + per_wave - 1) / per_wave)), 0, s, g, b);
+    };
+    if (rows <= 192) go(pass_b_kernel<6, 8, S>, 6, 8);
+    else if (rows <= 1536) go(pass_b_kernel<12, 8, S>, 12, 8);
+    else if (rows <= 4096) go(pass_b_kernel<16, 4, S>, 16, 4);
+    else {
+        set_error("internal: line too long for the tridiagonal pass");
+        return LCODE_E_UNSUPPORTED;
+    }
+    LCODE_HIP(hipGetLastError());
+    return LCODE_OK;
+}
+
 template <int L_, bool TW_LDS, typename S, typename G>
 static int launch_passes(const SolverGeom& g, const SolveBatch& b,
                          hipStream_t s, Profiler* prof, size_t lds,
-                         dim3 ga, dim3 gb, dim3 gc) {
+                         dim3 ga, dim3 gc) {
     const dim3 block(g.P * g.Tp);
     {
         ProfScope ps(prof, "solve_pass_a", s, true);
@@ -1647,10 +1567,9 @@ static int launch_passes(const SolverGeom& g, const SolveBatch& b,
     }
     LCODE_HIP(hipGetLastError());
     {
-        ProfScope ps(prof, "solve_pass_b", s, true);
-        launch_timed(ps, pass_b_kernel<L_, TW_LDS, S>, gb, block, lds, s, g, b);
+        const int rc = launch_pass_b<S>(g, b, s, prof);
+        if (rc) return rc;
     }
-    LCODE_HIP(hipGetLastError());
     {
         ProfScope ps(prof, "solve_pass_c", s, true);
         launch_timed(ps, pass_c_kernel<L_, TW_LDS, S, G>, gc, block, lds, s, g, b);
@@ -1705,10 +1624,8 @@ bool solver_static_length(int L) {
 
 template <int L, typename S, typename G>
 static int launch_wave_passes(const SolverGeom& g, const SolveBatch& b,
-                              hipStream_t s, Profiler* prof, int max_b) {
+                              hipStream_t s, Profiler* prof) {
     const dim3 block(WaveLanes<L>::T);
-    constexpr int PC = WavePairs<L>::P;
-    const int nblk_c = ((g.N + 1) / 2 + PC - 1) / PC;
     {
         ProfScope ps(prof, "solve_pass_a", s, true);
         // one block per pair of grid rows
@@ -1717,15 +1634,13 @@ static int launch_wave_passes(const SolverGeom& g, const SolveBatch& b,
     }
     LCODE_HIP(hipGetLastError());
     {
-        ProfScope ps(prof, "solve_pass_b", s, true);
-        launch_timed(ps, pass_b_wave_kernel<L, S>, dim3((max_b + 1) / 2, b.nfields),
-                     block, 0, s, g, b);
+        const int rc = launch_pass_b<S>(g, b, s, prof);
+        if (rc) return rc;
     }
-    LCODE_HIP(hipGetLastError());
-    const dim3 gc(nblk_c, b.nfields);
+    const dim3 gc((g.N + 1) / 2, b.nfields);
     {
         ProfScope ps(prof, "solve_pass_c", s, true);
-        launch_timed(ps, pass_c_wave_kernel<L, S, G>, gc, dim3(WaveLanes<L>::T * PC), 0, s,
+        launch_timed(ps, pass_c_wave_kernel<L, S, G>, gc, block, 0, s,
                      g, b);
     }
     LCODE_HIP(hipGetLastError());
@@ -1746,11 +1661,8 @@ static int launch_solve_t(const SolverGeom& g, const SolveBatch& b,
                           hipStream_t s, Profiler* prof) {
     const size_t lds = (size_t)solver_lds_bytes(g);
     const int per_block = 2 * g.P;
-    int max_a = 0, max_b = 0;
-    for (int f = 0; f < b.nfields; ++f) {
-        max_a = max_a > b.f[f].rowsA ? max_a : b.f[f].rowsA;
-        max_b = max_b > b.f[f].lenA ? max_b : b.f[f].lenA;
-    }
+    int max_a = 0;
+    for (int f = 0; f < b.nfields; ++f) max_a = max_a > b.f[f].rowsA ? max_a : b.f[f].rowsA;
     // the wave FFT runs the FP64 transforms and, with LCODE_FFT_WAVE_FP32, the
     // FP32 ones of L = 1280 (the workspace sets wave_tw only then)
     if constexpr (std::is_same<S, double>::value || LCODE_FFT_WAVE_FP32) if (g.wave_tw) {
@@ -1758,31 +1670,29 @@ static int launch_solve_t(const SolverGeom& g, const SolveBatch& b,
         // (or line) 0 and a sine transform of N - 2 from 1
         for (int f = 0; f < b.nfields; ++f) {
             const FieldPlan& p = b.f[f];
-            const bool ok_a = p.xfA == XF_DCT ? p.lenA == g.N && p.colA0 == 0
-                                              : p.lenA == g.N - 2 && p.colA0 == 1;
-            const bool ok_b = p.rowsA == (p.xfB == XF_DCT ? g.N : g.N - 2);
-            if (!ok_a || !ok_b) {
+            const bool ok = p.xfA == XF_DCT ? p.lenA == g.N && p.colA0 == 0
+                                            : p.lenA == g.N - 2 && p.colA0 == 1;
+            if (!ok) {
                 set_error("internal: field plan outside the wave FFT layout");
                 return LCODE_E_INVALID;
             }
         }
-        if (g.fft.L == 1280) return launch_wave_passes<1280, S, G>(g, b, s, prof, max_b);
-        if (g.fft.L == 2560) return launch_wave_passes<2560, S, G>(g, b, s, prof, max_b);
+        if (g.fft.L == 1280) return launch_wave_passes<1280, S, G>(g, b, s, prof);
+        if (g.fft.L == 2560) return launch_wave_passes<2560, S, G>(g, b, s, prof);
     }
     const dim3 ga((max_a + per_block - 1) / per_block, b.nfields);
-    const dim3 gb((max_b + per_block - 1) / per_block, b.nfields);
     const dim3 gc((g.N + per_block - 1) / per_block, b.nfields);
 #define LCODE_CASE(LL)                                                          \
     case LL:                                                                    \
         return g.tw_lds                                                         \
-                   ? launch_passes<LL, true, S, G>(g, b, s, prof, lds, ga, gb, gc) \
-                   : launch_passes<LL, false, S, G>(g, b, s, prof, lds, ga, gb, gc);
+                   ? launch_passes<LL, true, S, G>(g, b, s, prof, lds, ga, gc) \
+                   : launch_passes<LL, false, S, G>(g, b, s, prof, lds, ga, gc);
     switch (g.static_L) {
         LCODE_CASE(32) LCODE_CASE(64) LCODE_CASE(128) LCODE_CASE(256)
         LCODE_CASE(512) LCODE_CASE(640) LCODE_CASE(1024) LCODE_CASE(1280)
         LCODE_CASE(2048) LCODE_CASE(2560)
         default:
-            return launch_passes<0, false, S, G>(g, b, s, prof, lds, ga, gb, gc);
+            return launch_passes<0, false, S, G>(g, b, s, prof, lds, ga, gc);
     }
 #undef LCODE_CASE
 }
