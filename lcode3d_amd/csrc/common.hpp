@@ -656,6 +656,18 @@ struct UnetWgradArgs {
     float* partial;           // [tiles][9 cout_pad 32 nin + cout_pad]
 };
 
+// Weight packing of every layer: FP32 masters w[cout][cin][3][3] to the
+// convolutions' bfloat16 layouts (bwd NULL: no input gradient needed).
+constexpr int kUnetLayers = 8;
+struct UnetPackLayer {
+    const float* w;
+    int cout, cin, cout_pad, cinp;
+    uint16_t *fwd, *bwd;
+};
+struct UnetPackArgs {
+    UnetPackLayer layer[kUnetLayers];
+};
+
 // Planes of the network from the step's fields (FP64 or FP32 grids).
 struct UnetIoArgs {
     const void *f1[6], *f2[6], *f3[6];   // fields of slices n-1, n-2, n-3
@@ -680,8 +692,7 @@ int unet_tiles(int H, int W);
 int launch_unet_conv(const UnetConvArgs& a, hipStream_t s);
 int launch_unet_wgrad(const UnetWgradArgs& a, int cout, int cin, float* grad,
                       hipStream_t s);
-int launch_unet_pack(const float* w, int cout, int cin, int cout_pad, int cinp,
-                     uint16_t* fwd, uint16_t* bwd, hipStream_t s);
+int launch_unet_pack(const UnetPackArgs& a, hipStream_t s);
 int launch_unet_adam(float* p, const float* g, float* m, float* v, int n,
                      float lr, int t, hipStream_t s);
 int launch_unet_pool(const uint16_t* x, int H, int W, uint16_t* y, hipStream_t s);

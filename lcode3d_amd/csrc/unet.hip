@@ -260,24 +260,45 @@ unet_wgrad_kernel(UnetWgradArgs a) {
     }
 }
 
-// Sums the per-block partials in block order and writes the gradient in
+// Sums the per-block partials in a fixed order and writes the gradient in
 // the master layout w[co][ci][tap] (co < cout, ci < cin real), then b[co].
+// Bound: reading the partials once (18 MB for the 64-channel layers at S =
+// 161).  A block takes 64 consecutive values of a partial, its four waves
+// every fourth partial each with kAhead loads in flight; one thread per value
+// walking all partials in turn left the chain of their latencies (37 us a
+// layer on average at S = 161, now 4.8 us).
 __global__ void __launch_bounds__(256)
 unet_wgrad_reduce_kernel(const float* partial, int nblocks, int cout_pad,
                          int cinp, int cout, int cin, float* grad) {
+    constexpr int kAhead = 8;
+    __shared__ float red[4][64];
     const int per = 9 * cout_pad * cinp + cout_pad;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= cout * cin * 9 + cout) return;
-    int src;
-    if (k < cout * cin * 9) {
-        const int co = k / (cin * 9), ci = (k / 9) % cin, tap = k % 9;
-        src = (tap * cout_pad + co) * cinp + ci;
-    } else {
-        src = 9 * cout_pad * cinp + (k - cout * cin * 9);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int k = blockIdx.x * 64 + lane;
+    const float* src = partial + min(k, per - 1);
+    float s[kAhead] = {};
+    for (int b0 = wave; b0 < nblocks; b0 += 4 * kAhead) {
+        float v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            v[u] = src[(size_t)min(b0 + 4 * u, nblocks - 1) * per];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) s[u] += b0 + 4 * u < nblocks ? v[u] : 0.f;
     }
-    float s = 0.f;
-    for (int b = 0; b < nblocks; ++b) s += partial[(size_t)b * per + src];
-    grad[k] = s;
+#pragma unroll
+    for (int d = kAhead / 2; d > 0; d /= 2)
+#pragma unroll
+        for (int u = 0; u < d; ++u) s[u] += s[u + d];
+    red[wave][lane] = s[0];
+    __syncthreads();
+    if (wave != 0 || k >= per) return;
+    const float sum = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    if (k < 9 * cout_pad * cinp) {
+        const int tap = k / (cout_pad * cinp), co = (k / cinp) % cout_pad, ci = k % cinp;
+        if (co < cout && ci < cin) grad[((size_t)co * cin + ci) * 9 + tap] = sum;
+    } else if (k - 9 * cout_pad * cinp < cout) {
+        grad[cout * cin * 9 + k - 9 * cout_pad * cinp] = sum;
+    }
 }
 
 // One Adam step t >= 1 (Kingma & Ba 2015, Algorithm 1, bias-corrected).
@@ -302,17 +323,20 @@ unet_adam_kernel(float* p, const float* g, float* m, float* v, int n, float lr,
 // (cinp = cin padded to the input tensor's 32-channel chunks) and the
 // input-gradient form bwd[tap'][cin][32] with bwd[t][ci][co] =
 // w[co][ci][8 - t]; zeros for co >= cout and ci >= cin.
+// All layers in one launch (blockIdx.y): eight small launches in a row cost
+// 4.7 us each.
 __global__ void __launch_bounds__(256)
-unet_pack_kernel(const float* w, int cout, int cin, int cout_pad, int cinp,
-                 uint16_t* fwd, uint16_t* bwd) {
+unet_pack_kernel(UnetPackArgs a) {
+    const UnetPackLayer& L = a.layer[blockIdx.y];
+    const int cout = L.cout, cin = L.cin, cout_pad = L.cout_pad, cinp = L.cinp;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < 9 * cout_pad * cinp) {
         const int tap = k / (cout_pad * cinp), co = (k / cinp) % cout_pad, ci = k % cinp;
-        fwd[k] = co < cout && ci < cin ? f2bf(w[((size_t)co * cin + ci) * 9 + tap]) : 0;
+        L.fwd[k] = co < cout && ci < cin ? f2bf(L.w[((size_t)co * cin + ci) * 9 + tap]) : 0;
     }
-    if (bwd && k < 9 * cin * kC) {
+    if (L.bwd && k < 9 * cin * kC) {
         const int tap = k / (cin * kC), ci = (k / kC) % cin, co = k % kC;
-        bwd[k] = co < cout ? f2bf(w[((size_t)co * cin + ci) * 9 + (8 - tap)]) : 0;
+        L.bwd[k] = co < cout ? f2bf(L.w[((size_t)co * cin + ci) * 9 + (8 - tap)]) : 0;
     }
 }
 
@@ -578,17 +602,18 @@ int launch_unet_wgrad(const UnetWgradArgs& a, int cout, int cin, float* grad,
     }
 #undef LCODE_WG
     LCODE_HIP(hipGetLastError());
-    const int n = cout * cin * 9 + cout;
-    unet_wgrad_reduce_kernel<<<nblk(n), 256, 0, s>>>(a.partial, (int)grid.x, a.cout_pad,
-                                                      a.nin * kC, cout, cin, grad);
+    const int per = 9 * a.cout_pad * a.nin * kC + a.cout_pad;
+    unet_wgrad_reduce_kernel<<<(per + 63) / 64, 256, 0, s>>>(a.partial, (int)grid.x, a.cout_pad,
+                                                              a.nin * kC, cout, cin, grad);
     LCODE_HIP(hipGetLastError());
     return LCODE_OK;
 }
 
-int launch_unet_pack(const float* w, int cout, int cin, int cout_pad, int cinp,
-                     uint16_t* fwd, uint16_t* bwd, hipStream_t s) {
-    const int n = max(9 * cout_pad * cinp, bwd ? 9 * cin * kC : 0);
-    unet_pack_kernel<<<nblk(n), 256, 0, s>>>(w, cout, cin, cout_pad, cinp, fwd, bwd);
+int launch_unet_pack(const UnetPackArgs& a, hipStream_t s) {
+    int n = 0;
+    for (const UnetPackLayer& L : a.layer)
+        n = max(n, max(9 * L.cout_pad * L.cinp, L.bwd ? 9 * L.cin * kC : 0));
+    unet_pack_kernel<<<dim3(nblk(n), kUnetLayers), 256, 0, s>>>(a);
     LCODE_HIP(hipGetLastError());
     return LCODE_OK;
 }
@@ -668,7 +693,7 @@ struct LayerShape {
 };
 
 // C0 .. C7 (see the header): 14 input planes read as one 32-channel chunk
-constexpr LayerShape kLayers[8] = {
+constexpr LayerShape kLayers[kUnetLayers] = {
     {32, 14, 32, 32, 0}, {32, 32, 32, 32, 1}, {32, 32, 32, 32, 2}, {32, 32, 32, 32, 3},
     {32, 64, 32, 64, 2}, {32, 64, 32, 64, 1}, {32, 64, 32, 64, 0}, {6, 32, 16, 32, 0}};
 
@@ -753,14 +778,14 @@ static int check_net(const lcode_unet* n) {
 int lcode_unet_pack(const lcode_unet* n, hipStream_t stream) {
     int rc = check_net(n);
     if (rc) return rc;
-    for (int k = 0; k < 8; ++k) {
+    UnetPackArgs a{};
+    for (int k = 0; k < kUnetLayers; ++k) {
         const LayerShape& L = kLayers[k];
-        if ((rc = launch_unet_pack(n->params + param_offset(k), L.cout, L.cin, L.cout_pad,
-                                   L.cinp, n->wpack + pack_offset(k, false),
-                                   k ? n->wpack + pack_offset(k, true) : nullptr, stream)))
-            return rc;
+        a.layer[k] = UnetPackLayer{n->params + param_offset(k), L.cout, L.cin, L.cout_pad, L.cinp,
+                                   n->wpack + pack_offset(k, false),
+                                   k ? n->wpack + pack_offset(k, true) : nullptr};
     }
-    return LCODE_OK;
+    return launch_unet_pack(a, stream);
 }
 
 static uint16_t* T(const lcode_unet* n, int t) { return n->act + tensor_offset(n->S, t); }
