@@ -65,12 +65,13 @@ struct lcode_workspace {
     int* regions = nullptr;        // the same bound per deposition tile:
                                    // two slots of region_n^2 ints
     int region_n = 0;              // tiles per side (0: no per-tile bounds)
-    int* tile_order = nullptr;     // deposition tiles, centre first
-    // deposition tiles taken by two blocks: split_tile[s] for s < nsplit,
-    // then the slot of each tile (-1: not split); the two parts' sums
-    // (nsplit x 2 x 4 x tile^2 doubles) and a count per slot
+    DepositPlan dep_plan{};        // tiles of the deposition
+    int cus = 0;                   // compute units of the device
+    unsigned* tile_order = nullptr;   // what each deposition block takes
+                                   // (dep_entry)
+    // deposition tiles taken by two blocks: the two parts' sums (nsplit x 2 x 4
+    // x tile^2 doubles) and a count per slot
     int nsplit = 0;
-    int* split_tile = nullptr;
     double* split_part = nullptr;
     int* split_count = nullptr;
     int bound_slot = 0;            // slot the next push raises
@@ -120,12 +121,6 @@ namespace {
 #define LCODE_SOLVER_MAX_LDS 65536
 #endif
 
-// Cells a fine particle may move from its initial cell and still be
-// deposited through the LDS tiles (beyond: the spill list, deposited with
-// device atomics by a grid-wide kernel).  The adaptive halo is the pushes'
-// displacement bound, so small displacements keep small tiles; 6 covers the
-// nonlinear 1281^2 case (up to ~4.4 cells) within the LDS tables.
-constexpr int kDepositHalo = 6;
 // 1: per-tile displacement bounds size each deposition tile's halo; 0: the
 // largest bound over all particles sizes every tile's halo (build option)
 #ifndef LCODE_DEP_REGIONS
@@ -166,12 +161,6 @@ constexpr int kDepOrder = LCODE_DEP_ORDER;
 #endif
 constexpr int kDepResident = 3;   // tile blocks per CU (158 VGPRs, 4 waves) when
                                   // the runtime reports none
-
-// The deposition stages each tile's coarse rectangle in LDS: it has at
-// most ext / coarseness + 3 rows (ext: the tile and its largest halo).
-static bool deposit_staged(const lcode_config* cfg) {
-    return (kDepTile + 2 * kDepositHalo + 2) / cfg->plasma_coarseness + 3 <= kDepCoarseMax;
-}
 
 // Side of the XCD clusters of the tile order (tile_order.hpp).
 #ifndef LCODE_DEP_CLUSTER
@@ -281,8 +270,6 @@ int check_cfg(const lcode_config* c) {
                   "plasma_coarseness and plasma_fineness must be positive");
     LCODE_REQUIRE(c->plasma_fineness <= 3,
                   "plasma_fineness > 3 is not supported (deposition tile tables)");
-    LCODE_REQUIRE(c->plasma_fineness * (kDepTile + 2 * kDepositHalo + 2) <= kDepFineMax,
-                  "plasma_fineness too large for this build's deposition tiles");
     LCODE_REQUIRE(c->solver == LCODE_SOLVER_FFT64 || c->solver == LCODE_SOLVER_FFT32 ||
                       c->solver == LCODE_SOLVER_DENSE64 ||
                       c->solver == LCODE_SOLVER_DENSE_BF16X3 ||
@@ -631,53 +618,51 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     // particle within the largest halo + 1 cells of the tile interpolates
     // from when 2 coarseness + 10 <= tile side (a fine particle lies within
     // 2 coarseness + 2 cells of its coarse neighbours, at the plasma edge)
-    const int nt = (N + kDepTile - 1) / kDepTile;
-    if (kDepRegions && 2 * cfg->plasma_coarseness + kDepositHalo + 4 <= kDepTile) {
-        ws->region_n = nt;
-        if ((rc = dev_alloc(ws, (void**)&ws->regions, 2 * (size_t)nt * nt * sizeof(int))))
-            return fail(rc);
-    }
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws->device) !=
         hipSuccess) {
         set_error("hipDeviceGetAttribute (multiprocessor count) failed");
         return fail(LCODE_E_HIP);
     }
-    int resident = deposit_blocks_per_cu(deposit_staged(cfg));
-    if (resident <= 0) resident = kDepResident;
-    if (kDepOrder) {
-        std::vector<int> order((size_t)nt * nt);
-        for (int k = 0; k < nt * nt; ++k) order[k] = k;
-        if (kDepOrder == 2) {
-            order = xcd_cluster_order(nt, LCODE_DEP_CLUSTER);
-            // (when every tile block is resident at once: one round)
-            if (LCODE_DEP_BALANCE && cus >= 8 && cus % 8 == 0 &&
-                (LCODE_DEP_BALANCE == 2 || nt * nt <= resident * cus))
-                balance_xcd_slots(order, nt, cus / 8);
-        } else {
-            const double mid = (nt - 1) / 2.;
-            auto dist = [&](int k) {
-                return std::max(std::fabs(k / nt - mid), std::fabs(k % nt - mid));
-            };
-            std::stable_sort(order.begin(), order.end(),
-                             [&](int u, int v) { return dist(u) < dist(v); });
-        }
-        if ((rc = dev_alloc(ws, (void**)&ws->tile_order, order.size() * sizeof(int))) ||
-            (rc = hipMemcpy(ws->tile_order, order.data(), order.size() * sizeof(int),
-                            hipMemcpyHostToDevice) == hipSuccess ? LCODE_OK : LCODE_E_HIP)) {
-            if (rc == LCODE_E_HIP) set_error("hipMemcpy of the tile order failed");
+    ws->cus = cus;
+    ws->dep_plan = deposit_plan(N, cfg->plasma_coarseness, cfg->plasma_fineness, cus);
+    const int nt = ws->dep_plan.nt;
+    if (kDepRegions && 2 * cfg->plasma_coarseness + kDepositHalo + 4 <= ws->dep_plan.tile) {
+        ws->region_n = nt;
+        if ((rc = dev_alloc(ws, (void**)&ws->regions, 2 * (size_t)nt * nt * sizeof(int))))
             return fail(rc);
-        }
+    }
+    int resident = deposit_blocks_per_cu(ws->dep_plan);
+    if (resident <= 0) resident = kDepResident;
+    std::vector<int> order((size_t)nt * nt);
+    for (int k = 0; k < nt * nt; ++k) order[k] = k;
+    if (kDepOrder == 2) {
+        order = xcd_cluster_order(nt, LCODE_DEP_CLUSTER);
+        // (when every tile block is resident at once: one round)
+        if (LCODE_DEP_BALANCE && cus >= 8 && cus % 8 == 0 &&
+            (LCODE_DEP_BALANCE == 2 || nt * nt <= resident * cus))
+            balance_xcd_slots(order, nt, cus / 8);
+    } else if (kDepOrder == 1) {
+        const double mid = (nt - 1) / 2.;
+        auto dist = [&](int k) {
+            return std::max(std::fabs(k / nt - mid), std::fabs(k % nt - mid));
+        };
+        std::stable_sort(order.begin(), order.end(),
+                         [&](int u, int v) { return dist(u) < dist(v); });
     }
     {
         const int free_slots = std::max(resident * cus - nt * nt, 0);
         const int ns = std::min(LCODE_DEP_SPLIT < 0 ? free_slots : LCODE_DEP_SPLIT, nt * nt);
+        // (split_tile_table: the tile of each slot, then the slot of each tile)
+        const std::vector<int> tab = split_tile_table(nt, ns);
+        std::vector<unsigned> entries((size_t)nt * nt + ns);
+        for (int k = 0; k < nt * nt; ++k) entries[k] = dep_entry(order[k], tab[ns + order[k]], 0);
+        for (int k = 0; k < ns; ++k) entries[(size_t)nt * nt + k] = dep_entry(tab[k], k, 1);
+        if ((rc = upload(ws, &ws->tile_order, entries))) return fail(rc);
         if (ns > 0) {
-            const std::vector<int> tab = split_tile_table(nt, ns);
             ws->nsplit = ns;
-            const size_t part = 2 * 4 * (size_t)kDepTile * kDepTile;
-            if ((rc = upload(ws, &ws->split_tile, tab)) ||
-                (rc = dev_alloc(ws, (void**)&ws->split_part, ns * part * sizeof(double))) ||
+            const size_t part = 2 * 4 * (size_t)ws->dep_plan.tile * ws->dep_plan.tile;
+            if ((rc = dev_alloc(ws, (void**)&ws->split_part, ns * part * sizeof(double))) ||
                 (rc = dev_alloc(ws, (void**)&ws->split_count, ns * sizeof(int))))
                 return fail(rc);
             if (hipMemset(ws->split_count, 0, ns * sizeof(int)) != hipSuccess) {
@@ -865,7 +850,7 @@ static int do_push(lcode_workspace* ws, const lcode_config* cfg,
     if (ws->regions) {
         a.region_max = ws->regions + (size_t)ws->bound_slot * ws->region_n * ws->region_n;
         a.region_n = ws->region_n;
-        a.region_t = kDepTile;
+        a.region_t = ws->dep_plan.tile;
     }
     a.host_flag = ws->host_flag;
     a.grid32 = ws->grid32;
@@ -902,7 +887,7 @@ static DepositArgs deposit_args(const lcode_config* cfg,
                                 const double* q, const double* px,
                                 const double* py, const double* pz,
                                 const lcode_virt_params* vp,
-                                double* const out[4]) {
+                                double* const out[4], const DepositPlan& plan) {
     DepositArgs a{};
     a.nf = cfg->nf;
     a.nc = cfg->nc;
@@ -917,11 +902,20 @@ static DepositArgs deposit_args(const lcode_config* cfg,
     a.ro_initial = ro_initial;
     a.ro = out[0]; a.jx = out[1]; a.jy = out[2]; a.jz = out[3];
     a.halo = kDepositHalo;
-    a.ntx = (a.N + kDepTile - 1) / kDepTile;
-    a.staged = deposit_staged(cfg);
+    a.tile = plan.tile;
+    a.waves = plan.waves;
+    a.ntx = plan.nt;
+    a.fine_max = plan.fine_max;
+    a.coarse_max = plan.coarse_max;
+    a.staged = plan.staged;
     a.group = cfg->plasma_fineness;
     return a;
 }
+
+// What a deposition sizes its tiles' halo by: the largest halo, the bounds the
+// workspace's pushes raised, or the bound of its own offsets (a deposition on
+// its own, whose particles may come from anywhere).
+enum HaloBound { HALO_LARGEST, HALO_OF_PUSHES, HALO_OF_OFFSETS };
 
 static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
                       const double* ro_initial, const double* xo,
@@ -929,9 +923,12 @@ static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
                       const double* px, const double* py, const double* pz,
                       const lcode_virt_params* vp, double* const out[4],
                       hipStream_t stream, Gate gate = Gate{nullptr, 0.},
-                      bool adaptive_halo = false) {
+                      HaloBound halo = HALO_LARGEST) {
+    // (a workspace may serve other coarseness and fineness values than its own)
+    const DepositPlan plan = deposit_plan(ws->N, cfg->plasma_coarseness, cfg->plasma_fineness,
+                                          ws->cus);
     DepositArgs a = deposit_args(cfg, ro_initial, xo, yo, m, q, px, py, pz,
-                                 vp, out);
+                                 vp, out, plan);
     a.grid32 = ws->grid32;
     a.fault = ws->fault;
     a.spill = ws->spill;
@@ -940,8 +937,6 @@ static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
     a.spill_next = ws->spill_ctr + (1 - ws->spill_slot);
     a.tile_order = ws->tile_order;
     a.nsplit = ws->nsplit;
-    a.split_tile = ws->split_tile;
-    a.split_slot = ws->split_tile ? ws->split_tile + ws->nsplit : nullptr;
     a.split_part = ws->split_part;
     a.split_count = ws->split_count;
     // the spill list is deposited by the tile kernel's last block, unless
@@ -961,20 +956,25 @@ static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
     // after a push of this workspace: a halo of the pushes' displacement
     // bound, read from the slot the pushes raised; the deposition zeroes
     // the other slot, which the next pushes raise
-    if (adaptive_halo) {
+    if (halo != HALO_LARGEST) {
         a.halo_cells = ws->spill_ctr + 2 + ws->bound_slot;
         a.halo_next = ws->spill_ctr + 2 + (1 - ws->bound_slot);
         if (ws->regions) {
             const size_t nr = (size_t)ws->region_n * ws->region_n;
-            a.halo_regions = ws->regions + ws->bound_slot * nr;
+            if (halo == HALO_OF_PUSHES) a.halo_regions = ws->regions + ws->bound_slot * nr;
             a.halo_regions_next = ws->regions + (1 - ws->bound_slot) * nr;
         }
     }
     a.gate = gate;
     LCODE_REQUIRE(cfg->nf <= ws->nf, "workspace was built for fewer fine particles");
-    const int rc = launch_deposit(a, stream, &ws->prof);
+    // (on top of what pushes may have raised the slot to: a larger bound only
+    // makes larger halos)
+    int rc = LCODE_OK;
+    if (halo == HALO_OF_OFFSETS)
+        rc = launch_deposit_bound(a, ws->spill_ctr + 2 + ws->bound_slot, stream, &ws->prof);
+    if (rc == LCODE_OK) rc = launch_deposit(a, stream, &ws->prof);
     if (rc == LCODE_OK) ws->spill_slot = 1 - ws->spill_slot;
-    if (rc == LCODE_OK && adaptive_halo) ws->bound_slot = 1 - ws->bound_slot;
+    if (rc == LCODE_OK && halo != HALO_LARGEST) ws->bound_slot = 1 - ws->bound_slot;
     return rc;
 }
 
@@ -1028,7 +1028,7 @@ int lcode_deposit(lcode_workspace* ws, const lcode_config* cfg,
     LCODE_REQUIRE(virt_params && out, "NULL virt_params/out");
     for (int k = 0; k < 4; ++k) LCODE_REQUIRE(out[k], "NULL output");
     return do_deposit(ws, cfg, ro_initial, x_offt, y_offt, m, q, px, py, pz,
-                      virt_params, out, stream);
+                      virt_params, out, stream, Gate{nullptr, 0.}, HALO_OF_OFFSETS);
 }
 
 }  // extern "C"
@@ -1094,8 +1094,11 @@ int lcode_deposit_noalloc(const lcode_config* cfg, const double* ro_initial,
                   "(the spill list of its fixed scratch holds 2048^2)");
     int* s = nullptr;
     if ((rc = scratch_on_current_device(&s))) return rc;
+    // (whatever the tile order, one round of blocks or several)
     DepositArgs a = deposit_args(cfg, ro_initial, x_offt, y_offt, m, q, px, py,
-                                 pz, virt_params, out);
+                                 pz, virt_params, out,
+                                 deposit_plan(cfg->grid_steps, cfg->plasma_coarseness,
+                                              cfg->plasma_fineness, 256));
     int* ctr = s + kNoAllocSpillCap;
     a.spill = s;
     a.spill_count = ctr;
@@ -1237,7 +1240,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     // 3: deposit (lcode.py:856-859)
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p1[0], ws->p1[1], c->m,
                          c->q, ws->p1[2], ws->p1[3], ws->p1[4], vp, ws->dep,
-                         stream, Gate{nullptr, 0.}, true)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     // 4: fields with prev fields in the trick term; only the averages are
     // used afterwards (lcode.py:862-881)
@@ -1260,7 +1263,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     // 6: deposit (lcode.py:890-891)
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, Gate{nullptr, 0.}, true)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     // 7: fields with the pass-1 averages in the trick term; the solved
     // fields are the step's output (lcode.py:893-911, :927-928).  The
@@ -1284,7 +1287,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     double* const outD[4] = {out->ro, out->jx, out->jy, out->jz};
     return do_deposit(ws, cfg, c->ro_initial, out->x_offt, out->y_offt, c->m,
                       c->q, out->px, out->py, out->pz, vp, outD, stream,
-                      Gate{nullptr, 0.}, true);
+                      Gate{nullptr, 0.}, HALO_OF_PUSHES);
 }
 
 static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
@@ -1343,7 +1346,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
         return rc;
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, Gate{nullptr, 0.}, true)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     if ((rc = field_pass(ws, cfg, prev, trick_avg, beam_ro, beam_scalar,
                          ws->dep, outF, ws->favg, stream, Gate{nullptr, 0.},
@@ -1370,7 +1373,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
         return rc;
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, fallback, true)))
+                         stream, fallback, HALO_OF_PUSHES)))
         return rc;
     if ((rc = field_pass(ws, cfg, prev, trick_avg, beam_ro, beam_scalar,
                          ws->dep, outF, ws->favg, stream, fallback)))
@@ -1385,7 +1388,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
     double* const outD[4] = {out->ro, out->jx, out->jy, out->jz};
     return do_deposit(ws, cfg, c->ro_initial, out->x_offt, out->y_offt, c->m,
                       c->q, out->px, out->py, out->pz, vp, outD, stream,
-                      Gate{nullptr, 0.}, true);
+                      Gate{nullptr, 0.}, HALO_OF_PUSHES);
 }
 
 // ws->grid32 for the duration of one call

@@ -112,48 +112,12 @@ __device__ __forceinline__ bool gate_open(const Gate& g) {
     return !(num <= g.thr2 * den);
 }
 
-// Deposition tile side in cells and threads per tile block (build options).
-// At 641^2, coarseness 3, with grouped particles, 256 threads per block
-// (165 VGPRs: three blocks per CU), in the developed wake (slices 420-719,
-// HIP events on a sample of the launches, three boxes): 24 cells (729
-// tiles, all resident at once) 43.0-43.2 us per launch, 28 cells (529
-// tiles) 43.7-47.8 us, 30-36 cells 49-58 us, 16-22 cells 44-51 us (more
-// tiles than block slots); 512 threads 54-59 us.  With the central tiles
-// split over the free block slots: 24 cells 39.3 us, 25 cells 39.8, 26
-// cells (143 split tiles) 42.5, 27 cells 43.3.
-#ifndef LCODE_DEP_TILE
-#define LCODE_DEP_TILE 24
-#endif
-#ifndef LCODE_DEP_BLOCK
-#define LCODE_DEP_BLOCK 256
-#endif
-constexpr int kDepTile = LCODE_DEP_TILE;
-// LDS sizes of a deposition tile: fine indices per side (at least fineness
-// (kDepTile + 2 halo + 2) for fineness <= 3, halo <= 6) and coarse
-// particles per side of the staged coarse rectangle (a tile whose rectangle
-// is larger takes the unstaged kernel).
-#ifndef LCODE_DEP_FINE_MAX
-#define LCODE_DEP_FINE_MAX 128
-#endif
-#ifndef LCODE_DEP_COARSE_MAX
-#define LCODE_DEP_COARSE_MAX 18
-#endif
-constexpr int kDepFineMax = LCODE_DEP_FINE_MAX;
-constexpr int kDepCoarseMax = LCODE_DEP_COARSE_MAX;
-// 1: each deposition thread takes a group of fine particles (fineness x
-// fineness, one initial cell) and sums successive particles with a common
-// stencil centre in registers before the LDS atomics (43.8 us per launch at
-// 641^2); 0: one thread per fine particle (57.7 us).
-#ifndef LCODE_DEP_GROUP
-#define LCODE_DEP_GROUP 1
-#endif
-// 1: the lanes of a deposition wave take groups a prime stride apart
-// instead of adjacent ones (build option; at 641^2 39.6 -> 44.7 us per
-// launch: adjacent lanes' LDS reads of the staged tables lose their
-// locality)
-#ifndef LCODE_DEP_SPREAD
-#define LCODE_DEP_SPREAD 0
-#endif
+// Cells a fine particle may move from its initial cell and still be
+// deposited through the LDS tiles (beyond: the spill list, deposited with
+// device atomics by a grid-wide kernel).  The adaptive halo is the pushes'
+// displacement bound, so small displacements keep small tiles; 6 covers the
+// nonlinear 1281^2 case (up to ~4.4 cells) within the LDS tables.
+constexpr int kDepositHalo = 6;
 
 // XCD-aware block order.  Workgroups go to the 8 XCDs round-robin by linear
 // id and each XCD has its own L2: map linear id `lin` of `total` to a
@@ -321,21 +285,21 @@ struct DepositArgs {
     // next pushes' per-tile slots, each zeroed by its tile
     const int* halo_regions;
     int* halo_regions_next;
-    // NULL, or the tile each of the first ntx * ntx blocks takes (a
-    // permutation of the row-major tile indices)
-    const int* tile_order;
+    // NULL (block = row-major tile), or what each of the ntx * ntx + nsplit
+    // blocks takes: dep_entry()
+    const unsigned* tile_order;
+    int tile;                      // cells per tile side
+    int waves;                     // waves per SIMD of the tile kernel's form
+    int fine_max, coarse_max;      // LDS tables: fine indices and staged coarse
+                                   // particles per side, at most
     int ntx;                       // tiles per side; the tile kernel runs
                                    // ntx * ntx + nsplit one-dimensional blocks
-    // split tiles (nsplit 0: none).  Block ntx * ntx + s is the second part
-    // of tile split_tile[s], and split_slot[tile] is s for that tile (-1 for
-    // the others).  The two parts of a split tile each deposit half of its
-    // particle groups and write their sums to split_part (2 x 4 x tile^2
-    // doubles per slot); the second to finish, counted in split_count[s]
-    // (zero between calls: that block resets it), adds the other's sums to
-    // its own and stores the tile.
+    // split tiles (nsplit 0: none), numbered by slots.  The two parts of a
+    // split tile each deposit half of its particle groups and write their sums
+    // to split_part (2 x 4 x tile^2 doubles per slot); the second to finish,
+    // counted in split_count[slot] (zero between calls: that block resets it),
+    // adds the other's sums to its own and stores the tile.
     int nsplit;
-    const int* split_tile;
-    const int* split_slot;
     double* split_part;
     int* split_count;
     // 1: no spill kernel follows; when a particle may spill (the pushes'
@@ -352,13 +316,29 @@ struct DepositArgs {
     Gate gate;
 };
 
+// A block of the tile kernel: its tile, the slot of a split tile (or -1) and
+// which part of it.
+inline unsigned dep_entry(int tile, int slot, int part) {
+    return (unsigned)tile | (unsigned)(slot + 1) << 16 | (unsigned)part << 31;
+}
+
 int launch_estimate(const EstimateArgs& a, hipStream_t s, Profiler* prof);
 int launch_push(const PushArgs& a, hipStream_t s, Profiler* prof);
 int launch_deposit(const DepositArgs& a, hipStream_t s, Profiler* prof);
+// Raises *bound to the displacement bound of a's coarse offsets (in cells, at
+// most a.halo + 1).
+int launch_deposit_bound(const DepositArgs& a, int* bound, hipStream_t s, Profiler* prof);
+// The deposition's tiles for a grid and plasma.
+struct DepositPlan {
+    int tile, nt;                  // cells per tile side, tiles per side
+    int waves;                     // of the tile kernel per SIMD
+    int fine_max, coarse_max;      // LDS tables (DepositArgs)
+    int staged;                    // the coarse rectangle is staged in LDS
+};
+DepositPlan deposit_plan(int N, int coarseness, int fineness, int cus);
 // Tile blocks of the deposition one CU holds at once (the smaller of its
-// FP64- and FP32-grid forms, staged or not), or 0 when the runtime cannot
-// say.
-int deposit_blocks_per_cu(bool staged);
+// FP64- and FP32-grid forms), or 0 when the runtime cannot say.
+int deposit_blocks_per_cu(const DepositPlan& p);
 // make_plasma (lcode.py:452-573) on the device.
 constexpr double kElectronMass = 1.;      // lcode.py:47
 constexpr double kElectronCharge = -1.;   // lcode.py:46

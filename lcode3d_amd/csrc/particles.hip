@@ -6,6 +6,8 @@
 
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace lcode {
 
 namespace {
@@ -16,6 +18,13 @@ constexpr int kBlock = 256;
 #define LCODE_SPILL_BLOCKS 256
 #endif
 constexpr int kSpillBlocks = LCODE_SPILL_BLOCKS;
+
+// A value that every lane of the wave holds alike, in a scalar register.
+__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ double scalar(double v) {
+    return __hiloint2double(scalar(__double2hiint(v)), scalar(__double2loint(v)));
+}
 
 __device__ __forceinline__ int clampi(int v, int n) {
     return v < 0 ? 0 : (v >= n ? n - 1 : v);
@@ -215,33 +224,18 @@ push_kernel(PushArgs a) {
     }
 }
 
-// Deposition values of a fine particle with mass m, charge q, momentum p
-// (lcode.py:651-655): dro = q / (1 - pz / gamma), dj = p dro / gamma,
-// evaluated with one division as dro = q gamma r, dj = q p r,
-// r = 1 / (gamma - pz) (the same quantities, rounded differently).
-// G = float: the FP32-grid form, in FP32 arithmetic.
-template <typename G>
-__device__ __forceinline__ void deposit_values(G m, G q, G px, G py, G pz,
-                                               G* v) {
-    const G gamma_m = sqrt(m * m + px * px + py * py + pz * pz);
-    const G qr = q / (gamma_m - pz);
-    v[0] = gamma_m * qr;
-    v[1] = px * qr;
-    v[2] = py * qr;
-    v[3] = pz * qr;
-}
-
 // Coarse->fine interpolation of fine particle (fi, fj) (lcode.py:591-621)
-// and its deposition values, reading everything from global memory.
-template <typename G>
+// and its deposition values (lcode.py:651-655): dro = q / (1 - pz / gamma), dj
+// = p dro / gamma, evaluated with one division as dro = q gamma r, dj = q p r,
+// r = 1 / (gamma - pz) (the same quantities, rounded differently).  Reads
+// everything from global memory.
 struct FineParticle {
-    double x, y;         // position (FP64 in every form)
-    G v[4];              // dro, djx, djy, djz
+    double x, y;         // position
+    double v[4];         // dro, djx, djy, djz
 };
 
-template <typename G>
-__device__ __forceinline__ void fine_particle(const DepositArgs& a, int fi,
-                                              int fj, FineParticle<G>& p) {
+__device__ __forceinline__ void fine_particle(const DepositArgs& a, int fi, int fj,
+                                              FineParticle& p) {
     const double ipi = a.ip[fi], ini = a.in[fi];
     const double ipj = a.ip[fj], inj = a.in[fj];
     const double A = ipi * ipj, B = ipi * inj, C = ini * ipj, D = ini * inj;
@@ -256,22 +250,19 @@ __device__ __forceinline__ void fine_particle(const DepositArgs& a, int fi,
     p.x = a.fg[fi] + LCODE_MIX(a.x_offt);
     p.y = a.fg[fj] + LCODE_MIX(a.y_offt);
     const double s = a.smallness;
-    deposit_values<G>((G)(s * LCODE_MIX(a.m)), (G)(s * LCODE_MIX(a.q)),
-                      (G)(s * LCODE_MIX(a.px)), (G)(s * LCODE_MIX(a.py)),
-                      (G)(s * LCODE_MIX(a.pz)), p.v);
+    const double m = s * LCODE_MIX(a.m), q = s * LCODE_MIX(a.q), px = s * LCODE_MIX(a.px),
+                 py = s * LCODE_MIX(a.py), pz = s * LCODE_MIX(a.pz);
 #undef LCODE_MIX
+    const double gamma = sqrt(m * m + px * px + py * py + pz * pz);
+    const double qr = q / (gamma - pz);
+    p.v[0] = gamma * qr;
+    p.v[1] = px * qr;
+    p.v[2] = py * qr;
+    p.v[3] = pz * qr;
 }
 
-// Tiles of the owner-computes deposition: a block owns kTile x kTile cells
-// and deposits, in LDS, every fine particle whose cell moved at most
-// a.halo cells from its initial cell and whose stencil touches the tile.
-constexpr int kTile = kDepTile;
-constexpr int kDepBlock = LCODE_DEP_BLOCK;
-#ifdef LCODE_DEP_WAVES
-#define LCODE_DEP_ATTR __attribute__((amdgpu_waves_per_eu(LCODE_DEP_WAVES, LCODE_DEP_WAVES)))
-#else
-#define LCODE_DEP_ATTR
-#endif
+
+constexpr int kDepBlock = 256;   // threads of a deposition tile's block
 
 // First fine index whose initial cell is >= c (fg is increasing).
 __device__ int first_fine_at_or_after(const double* fg, int nf, int c, int N,
@@ -284,80 +275,12 @@ __device__ int first_fine_at_or_after(const double* fg, int nf, int c, int N,
     return lo;
 }
 
-// deposit_kernel (lcode.py:626-663) as owner-computes tiles: each block
-// accumulates its kTile^2 cells of ro, jx, jy, jz in LDS (FP64 LDS atomics,
-// ds_add_f64), then stores them once, adding the ion background last
-// (lcode.py:687).  Every cell of the grid is written by exactly one block,
-// so the outputs need no zeroing.  A block visits the fine particles whose
-// initial cell lies within halo + 1 cells of its tile; their per-index
-// interpolation data and, when they fit, the coarse particles they
-// interpolate from are staged in LDS first; then one thread per fine
-// particle adds its 9 x 4 weighted values to the LDS tile.  A particle
-// displaced by more than a.halo cells from its initial cell is appended to
-// the spill list by its home tile (the tile owning its initial cell), and
-// deposit_spill_kernel, launched next, adds the list with device atomics
-// across the whole grid.  A non-finite particle deposits nothing: the tile
-// (or, when the pushes reported one, every tile) is written as NaN.
-// A split tile is deposited by two blocks, each over alternate runs of its
-// particle groups: the tiles with the most work then take about half as
-// long, using block slots the launch leaves free; the second block to
-// finish adds the first one's sums (published in global memory) and
-// stores the tile.
-constexpr int kFineMax = kDepFineMax;       // fine indices per side
-constexpr int kCoarseMax = kDepCoarseMax;   // coarse particles per side staged in LDS
-constexpr int kExtMax = kTile + 14;   // initial cells per side: kTile + 2 halo + 2, halo <= 6
-
-struct FineTab {                 // per fine index along one axis
-    double2 w[kFineMax];         // interpolation weights (ip, in)
-    double fg[kFineMax];         // initial position
-    int4 idx[kFineMax];          // coarse neighbours (P, Nn), initial cell, -
-};
-
-// First fine index whose initial cell is >= c, found by one wave (every
-// lane calls it): 64 samples narrow it to a stride, 64 more pin it down.
-__device__ int wave_first_fine(const double* fg, int nf, int c, int N,
-                               double h) {
-    const int lane = threadIdx.x & 63;
-    if (nf > 64 * 64) return first_fine_at_or_after(fg, nf, c, N, h);
-    const int stride = (nf + 63) / 64;
-    const int i1 = lane * stride;
-    const bool below1 = i1 < nf && cell_of(fg[i1], N, h) < c;
-    const int n1 = __popcll(__ballot(below1));
-    if (n1 == 0) return 0;
-    const int base = (n1 - 1) * stride;
-    const int i2 = base + lane;
-    const bool below2 = lane < stride && i2 < nf && cell_of(fg[i2], N, h) < c;
-    return base + __popcll(__ballot(below2));
-}
-
-// Adds v[c] * w[k] (or val[c][k]) to the stencil points of cell (i, j) that
-// lie in this block's tile.
 template <typename G>
-__device__ __forceinline__ void lds_deposit(double (*acc)[kTile][kTile],
-                                            int i, int j, int ci0, int cj0,
-                                            const G* v, const G* w,
-                                            const G (*val)[9]) {
-    const bool inside = i - 1 >= ci0 && i + 1 < ci0 + kTile &&
-                        j - 1 >= cj0 && j + 1 < cj0 + kTile;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        const int si = i + stencil_di(k) - ci0;
-        const int sj = j + stencil_dj(k) - cj0;
-        if (inside || (si >= 0 && si < kTile && sj >= 0 && sj < kTile)) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                atomicAdd(&acc[c][si][sj], (double)(val ? val[c][k] : v[c] * w[k]));
-        }
-    }
-}
-
-template <typename A, typename G>
-__device__ __forceinline__ void deposit_spill_one(const DepositArgs& a, int fk,
-                                                  int N) {
-    FineParticle<A> fp;
-    fine_particle<A>(a, fk / a.nf, fk % a.nf, fp);
-    TscT<A> t;
-    tsc_weights<A>(fp.x, fp.y, N, a.h, t, nullptr, 1. / a.h);
+__device__ __forceinline__ void deposit_spill_one(const DepositArgs& a, int fk, int N) {
+    FineParticle fp;
+    fine_particle(a, fk / a.nf, fk % a.nf, fp);
+    Tsc t;
+    tsc_weights<double>(fp.x, fp.y, N, a.h, t, nullptr, 1. / a.h);
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
         const size_t idx = (size_t)(t.i + stencil_di(k)) * N + (t.j + stencil_dj(k));
@@ -368,57 +291,173 @@ __device__ __forceinline__ void deposit_spill_one(const DepositArgs& a, int fk,
     }
 }
 
-// A: type of the per-particle arithmetic and register sums, G: storage
-// type of the output grids (double, double: the plain path; double,
-// float: the mixed form, whose density and currents are stored in FP32).
-// The LDS tile accumulates in FP64: at 641^2 FP32 LDS atomics (ds_add_f32)
-// kept the LDS pipeline 8x longer busy than FP64 ones (ds_add_f64) for the
-// same instruction count (148 against 35 us per launch).  FP32 arithmetic
-// (A = float) took the deposition from 49.8 to 47.9 us only (the kernel is
-// bound by latency, not by its VALU work) while its rounding, relative to
-// the background density 1, left the density response of a small beam
-// (amplitude 0.01) with relative errors up to 4e-4 in Ez; the mixed form
-// keeps FP64 arithmetic.
-template <bool STAGED, typename A, typename G>
-__device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
+// deposit_kernel (lcode.py:626-663) as owner-computes tiles: each block
+// accumulates its T^2 cells of ro, jx, jy, jz in LDS (FP64 LDS atomics,
+// ds_add_f64), then stores them once, adding the ion background last
+// (lcode.py:687).  Every cell of the grid is written by exactly one block, so
+// the outputs need no zeroing.  A block visits the fine particles whose initial
+// cell lies within halo + 1 cells of its tile; their per-index interpolation
+// data and, when they fit, the coarse particles they interpolate from are
+// staged in LDS first.  A particle displaced by more than a.halo cells from its
+// initial cell is appended to the spill list by its home tile (the tile owning
+// its initial cell), and deposit_spill_kernel, launched next, adds the list with
+// device atomics across the whole grid.  A non-finite particle deposits nothing:
+// the tile (or, when the pushes reported one, every tile) is written as NaN.  A
+// split tile is deposited by two blocks, each over half of the strips; the
+// second block to finish adds the first one's sums (published in global memory)
+// and stores the tile.
+//
+// One thread takes a group of fine particles (fineness x fineness, one initial
+// cell) and sums their 3 x 3 x 4 stencil values in registers while they share a
+// stencil centre; the sums go to LDS when the centre changes and after the group
+// (43.8 us per launch at 641^2 against 57.7 with one thread per particle).  The
+// group's second particle is the one that more likely stays in the first one's
+// cell.  Adjacent lanes hold adjacent cells, so the atomics of one instruction
+// fall on distinct addresses.
+//
+// What bounds it at 641^2: a tile's start and end take 10 us (three dependent
+// rounds of loads - bounds and the ends of the fine ranges, tables and coarse
+// rectangle, then the stores - and the launch), the rest is the chain of a
+// particle: two rounds of LDS reads and about 60 dependent FP64 operations, with
+// three waves per SIMD to overlap it (VALU issue 62 % of that time, LDS 40 %).
+// us per launch before / now: 129^2 25.3 / 12.4, 361^2 28.8 / 20.8, 641^2 39.9 /
+// 34.8, 1281^2 with fineness 3 231 / 182.  Tried at 641^2 and slower: strips of
+// particles along j whose sums slide with the centre (61 us: the lanes leave
+// their columns at different steps), 5 waves per block (44 - 65), 32-cell tiles
+// with 8 waves (35 - 52).
+template <int T>
+struct DepTile {
+    static constexpr int kPitch = T;                // LDS row of the sums
+    static constexpr int kComp = T * kPitch;        // one component
+    static constexpr int kExtMax = T + 14;          // initial cells per side: T + 2 halo + 2, halo <= 6
+};
+
+// LDS of a tile block: the sums, the fine-index tables of both axes (a.fine_max
+// entries each) and the staged coarse rectangle (a.coarse_max squared, or 0).
+// The staged particles lie in 16-byte pairs, so that one read brings two of a
+// corner's values: (x_offt, y_offt), (m, q), (px, py), pz.
+struct DepLds {
+    double2 *wi, *wj;          // interpolation weights (ip, in)
+    double2 *cpos, *cmq, *cpxy;
+    int4 *xi, *xj;             // coarse neighbours (P, Nn), initial cell, -
+    double *acc, *fi, *fj, *cpz;
+    __device__ DepLds(unsigned char* p, int acc_len, int fine_max, int coarse_max) {
+        auto take = [&](size_t bytes) {
+            unsigned char* q = p;
+            p += bytes;
+            return q;
+        };
+        const size_t f = fine_max, c = (size_t)coarse_max * coarse_max;
+        wi = (double2*)take(16 * f);
+        wj = (double2*)take(16 * f);
+        xi = (int4*)take(16 * f);
+        xj = (int4*)take(16 * f);
+        cpos = (double2*)take(16 * c);
+        cmq = (double2*)take(16 * c);
+        cpxy = (double2*)take(16 * c);
+        acc = (double*)take(8 * (size_t)acc_len);
+        fi = (double*)take(8 * f);
+        fj = (double*)take(8 * f);
+        cpz = (double*)take(8 * c);
+    }
+};
+
+inline size_t deposit_lds_bytes(int T, int fine_max, int coarse_max) {
+    return 8 * (size_t)(4 * T * T) + 80 * (size_t)fine_max +
+           56 * (size_t)coarse_max * coarse_max;
+}
+
+// First fine index whose initial cell is >= c (fg is increasing), from this
+// lane's sample of a 64-entry window at w0 (the cell of entry w0 + lane), else
+// by search.  Every lane of the wave calls it.
+__device__ __forceinline__ int wave_first_fine(const double* fg, int nf, int c, int N, double h,
+                                               int w0, int sample) {
+    const int lane = threadIdx.x & 63;
+    const int n = __popcll(__ballot(w0 + lane < nf && sample < c));
+    const bool open_left = n > 0 || w0 == 0, open_right = n < 64 || w0 + 64 >= nf;
+    if (open_left && open_right) return min(w0 + n, nf);
+    return first_fine_at_or_after(fg, nf, c, N, h);
+}
+
+// x / h + .5, its product rounded before the sum as the reference rounds its
+// quotient (lcode.py:404): far from the axis a product left unrounded moves the
+// weights by 1e-14 against it.
+__device__ __forceinline__ double in_cells(double x, double inv_h) {
+#pragma clang fp contract(off)
+    const double q = x * inv_h;
+    return q + .5;
+}
+
+// gamma = sqrt(s) and 1 / (gamma - pz) to about an ulp, without the compiler's
+// rescaling of tiny and huge arguments (gamma is a particle's energy): the
+// hardware's estimates refined by Newton's iteration.
+__device__ __forceinline__ void gamma_and_inverse(double s, double pz, double& gamma,
+                                                  double& inv) {
+    const double r0 = __builtin_amdgcn_rsq(s);
+    double g = s * r0, hh = .5 * r0;
+    double e = fma(-hh, g, .5);
+    g = fma(g, e, g);
+    hh = fma(hh, e, hh);
+    e = fma(-g, g, s);
+    g = fma(e, hh, g);
+    e = fma(-g, g, s);
+    gamma = fma(e, hh, g);
+    const double d = gamma - pz;
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.), r, r);
+    inv = fma(fma(-d, r, 1.), r, r);
+}
+
+// G: storage type of the output grids (float: the mixed form).  The arithmetic
+// and the sums are FP64 in both: at 641^2 FP32 LDS atomics (ds_add_f32) kept the
+// LDS pipeline 8x longer busy than FP64 ones, and FP32 arithmetic left the
+// density response of a small beam (amplitude 0.01) with relative errors up to
+// 4e-4 in Ez.
+template <int T, int W, bool STAGED, typename G>
+__global__ void __launch_bounds__(kDepBlock) __attribute__((amdgpu_waves_per_eu(W)))
+deposit_tile_kernel(DepositArgs a) {
     // the count slot of the next call is zeroed here (also when gated off)
     // unless a spill kernel follows, which does it
-    if (a.spill_in_tiles && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
-        *a.spill_next = 0;
+    if (a.spill_in_tiles && blockIdx.x == 0 && threadIdx.x == 0) *a.spill_next = 0;
     if (!gate_open(a.gate)) return;   // block-uniform: before any barrier
-    __shared__ double acc[4][kTile][kTile];
-    __shared__ int last_block, split_last;
-    __shared__ FineTab ti, tj;
-    // the staged coarse particles in 16-byte pairs where the arithmetic
-    // type allows, so that one LDS read brings two of a corner's values:
-    // (x_offt, y_offt), (m, q), (px, py), pz
-    using A2 = typename std::conditional<std::is_same<A, double>::value, double2, float2>::type;
-    __shared__ double2 cpos[kCoarseMax * kCoarseMax];
-    __shared__ A2 cmq[kCoarseMax * kCoarseMax], cpxy[kCoarseMax * kCoarseMax];
-    __shared__ A cpz[kCoarseMax * kCoarseMax];
-    __shared__ int range[4];
-    __shared__ int tile_nan;
+    using D = DepTile<T>;
+    // W = 3: the values ahead of the checks, where their latency overlaps the
+    // position's (151 registers); W = 4: after them (127)
+    constexpr bool kEarly = W < 4;
+    constexpr int kAcc = 4 * D::kComp;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const DepLds l(lds_raw, kAcc, a.fine_max, STAGED ? a.coarse_max : 0);
+    __shared__ int last_block, split_last, tile_nan;
+    __shared__ int range[4], corner[4];
     const int N = a.N;
-    const double inv_h = 1. / a.h;
-    // tile of this block: row-major, or the host's order in a.tile_order
-    // (which keeps neighbouring tiles on one XCD and gives each CU a mix of
-    // the wake's heavy tiles and light ones)
-    // A split tile's two parts (the tile's own block, part 0, and one of the
-    // nsplit blocks after the tiles, part 1) take alternate runs of
-    // blockDim.x particle groups.
-    const int ntx = a.ntx, ntiles = ntx * ntx, lin = blockIdx.x;
-    int tile, slot = -1, part = 0;
-    if (lin >= ntiles) {
-        slot = lin - ntiles;
-        tile = a.split_tile[slot];
-        part = 1;
-    } else {
-        tile = a.tile_order ? a.tile_order[lin] : lin;
-        if (a.nsplit) slot = a.split_slot[tile];
-    }
+    const double inv_h = scalar(1. / a.h);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // tile of this block: row-major, or from the host's table (which keeps
+    // neighbouring tiles on one XCD and gives each CU a mix of the wake's heavy
+    // tiles and light ones; its last nsplit entries are the second parts of the
+    // split tiles)
+    const int ntx = a.ntx, lin = blockIdx.x;
+    const unsigned entry = scalar(a.tile_order ? (int)a.tile_order[lin] : lin);
+    const int tile = entry & 0xFFFFu, slot = (int)((entry >> 16) & 0x7FFFu) - 1, part = entry >> 31;
     const int nparts = slot >= 0 ? 2 : 1;
     const int ty = tile / ntx, tx = tile - ty * ntx;
-    const int ci0 = ty * kTile, cj0 = tx * kTile;
+    const int ci0 = ty * T, cj0 = tx * T;
+    // the fine grid around this wave's end of a range (waves 0, 1: first and
+    // last row, 2, 3: column): a window of 64 about where an even grid of
+    // a.group points per cell has it, with the coarse neighbour there (the
+    // corners of the coarse rectangle), loaded while the bounds below arrive
+    static_assert(kDepBlock >= 256, "one wave per end of the two ranges");
+    const bool last_end = wave & 1;
+    const int end_cell = (wave < 2 ? ci0 : cj0) + (last_end ? T : -1);   // about
+    const int guess = (int)floor(((double)(end_cell - N / 2) - .5) * a.group + .5 * (a.nf - 1));
+    const int w0 = scalar(min(max(guess - 32, 0), max(a.nf - 64, 0)));
+    const int64_t* const neighbour = last_end ? a.Nn : a.P;
+    int sample = 0, sample_c = 0;
+    if (a.nf > 0) {
+        const int k = min(w0 + lane, a.nf - 1);
+        sample_c = (int)neighbour[k];
+        sample = cell_of(a.fg[k], N, a.h);
+    }
     // halo: the displacement bound of the last pushes when one is given.
     // A fine particle's offset is a convex mix of coarse offsets, so its
     // cell moved at most `bound` cells: with bound <= a.halo no particle
@@ -433,7 +472,7 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
     // a particle's stencil reaches has the particle's home tile in its
     // neighbourhood, so all of them visit it, or (beyond a.halo) none does
     // and its home tile lists it.
-    const int global = a.halo_cells ? max(*a.halo_cells, 0) : a.halo + 1;
+    const int global = scalar(a.halo_cells ? max(*a.halo_cells, 0) : a.halo + 1);
     // the pushes met a non-finite (or absurdly far) particle: the whole
     // deposition is NaN, with no particle visited (already reported)
     const bool nonfinite = global >= kNonFinite;
@@ -447,267 +486,322 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
                     bound = max(bound, a.halo_regions[r * ntx + c]);
             }
     }
-    const int halo = min(bound, a.halo);
-    const bool may_spill = bound > a.halo;
+    const int halo = scalar(min(bound, a.halo));
+    const bool may_spill = scalar(bound) > a.halo;
     if (threadIdx.x == 0 && part == 0) {
         // zero the slots the next pushes raise; nothing reads them here
         if (a.halo_next && tile == 0) *a.halo_next = 0;
         if (a.halo_regions_next) a.halo_regions_next[tile] = 0;
     }
     if (threadIdx.x == 0) tile_nan = 0;
-    const int ext = kTile + 2 * halo + 2;
-    const int ci_lo = ci0 - 1 - halo, cj_lo = cj0 - 1 - halo;
-    for (int k = threadIdx.x; k < 4 * kTile * kTile; k += blockDim.x)
-        (&acc[0][0][0])[k] = 0;
-    {
-        const int wave = threadIdx.x >> 6;
-        if (wave < 4) {
-            const int lo = (wave < 2) ? ci_lo : cj_lo;
-            const int r = wave_first_fine(a.fg, a.nf, lo + ((wave & 1) ? ext : 0), N, a.h);
-            if ((threadIdx.x & 63) == 0) range[wave] = r;
+    for (int k = threadIdx.x; k < kAcc; k += kDepBlock) l.acc[k] = 0;
+    const int ext = T + 2 * halo + 2;
+    if (wave < 4) {
+        const int lo = (wave < 2 ? ci0 : cj0) - 1 - halo;
+        const int r = wave_first_fine(a.fg, a.nf, lo + (last_end ? ext : 0), N, a.h, w0, sample);
+        // the coarse neighbour of the range's first (last) fine index
+        const int at = min(max(last_end ? r - 1 : r, 0), max(a.nf - 1, 0));
+        int c = __shfl(sample_c, at - w0, 64);
+        if (at < w0 || at >= w0 + 64) c = (int)neighbour[at];
+        if (lane == 0) {
+            range[wave] = r;
+            corner[wave] = clampi(c, a.nc);
         }
     }
     __syncthreads();
-    const int fi_a = range[0], ni = range[1] - range[0];
-    const int fj_a = range[2], nj = range[3] - range[2];
-    const bool overfull = ni > kFineMax || nj > kFineMax || ext > kExtMax;
+    const int fi_a = scalar(range[0]), ni = scalar(range[1]) - fi_a;
+    const int fj_a = scalar(range[2]), nj = scalar(range[3]) - fj_a;
+    const bool overfull = ni > a.fine_max || nj > a.fine_max || ext > D::kExtMax;
     if (overfull) {
         // denser fine grid than the host-checked fineness allows: flag the
         // tile as faulted and fill it with NaN rather than drop particles
         if (threadIdx.x == 0 && part == 0) atomicAdd(a.fault, 1);
-    } else if (!nonfinite) {
-        for (int k = threadIdx.x; k < ni + nj; k += blockDim.x) {
-            const bool isj = k >= ni;
-            const int f = isj ? fj_a + k - ni : fi_a + k;
-            FineTab& t = isj ? tj : ti;
-            const int s = isj ? k - ni : k;
-            t.w[s] = make_double2(a.ip[f], a.in[f]);
-            t.fg[s] = a.fg[f];
-            t.idx[s] = make_int4(clampi((int)a.P[f], a.nc), clampi((int)a.Nn[f], a.nc),
-                                 cell_of(a.fg[f], N, a.h), 0);
-        }
-        __syncthreads();
-        // coarse rectangle referenced by this block's fine particles
-        int cI0 = 0, cJ0 = 0, cW = 0;
+    } else if (!nonfinite && ni > 0 && nj > 0) {
+        // coarse rectangle referenced by this block's fine particles:
+        // indices_prev/next grow with the fine index, so it is [P[first],
+        // Nn[last]] on each axis; the host checked the fit
+        int cI0 = 0, cJ0 = 0, cH = a.nc, cW = a.nc;
         if constexpr (STAGED) {
-            // indices_prev/next grow with the fine index, so the rectangle
-            // is [P[first], Nn[last]] on each axis; the host checked the fit
-            cI0 = ni ? ti.idx[0].x : 0;
-            cJ0 = nj ? tj.idx[0].x : 0;
-            int cH = ni ? ti.idx[ni - 1].y - cI0 + 1 : 0;
-            cW = nj ? tj.idx[nj - 1].y - cJ0 + 1 : 0;
-            if (cH > kCoarseMax || cW > kCoarseMax || cH < 0 || cW < 0) {
+            cI0 = scalar(corner[0]);
+            cJ0 = scalar(corner[2]);
+            cH = scalar(corner[1]) - cI0 + 1;
+            cW = scalar(corner[3]) - cJ0 + 1;
+            if (cH > a.coarse_max || cW > a.coarse_max || cH < 0 || cW < 0) {
                 if (threadIdx.x == 0 && part == 0) atomicAdd(a.fault, 1);
-                cH = cH < 0 ? 0 : (cH > kCoarseMax ? kCoarseMax : cH);
-                cW = cW < 0 ? 0 : (cW > kCoarseMax ? kCoarseMax : cW);
+                cH = cH < 0 ? 0 : (cH > a.coarse_max ? a.coarse_max : cH);
+                cW = cW < 0 ? 0 : (cW > a.coarse_max ? a.coarse_max : cW);
             }
-            const double* src[7] = {a.x_offt, a.y_offt, a.m, a.q, a.px, a.py, a.pz};
-            for (int k = threadIdx.x; k < cH * cW; k += blockDim.x) {
-                const size_t g = (size_t)(cI0 + k / cW) * a.nc + cJ0 + k % cW;
-                cpos[k] = make_double2(src[0][g], src[1][g]);
-                cmq[k].x = (A)src[2][g];
-                cmq[k].y = (A)src[3][g];
-                cpxy[k].x = (A)src[4][g];
-                cpxy[k].y = (A)src[5][g];
-                cpz[k] = (A)src[6][g];
+        }
+        // the tables, their neighbour indices as offsets in the rectangle:
+        // rows scaled by its width, each clamped into it, so that a row part
+        // plus a column part is an in-bounds index
+        const int hmax = max(cH - 1, 0), wmax = max(cW - 1, 0);
+        // staged as shares of a fine particle (`sm` first: a plasma of coarseness^2
+        // masses then has an exact 1 / fineness^2, and a particle at rest exactly its
+        // charge); `same`: every particle has the first one's mass and charge
+        const double sm = a.smallness;
+        bool same = STAGED;
+        double m0 = 0., q0 = 0.;
+        struct Coarse {
+            double x, y, m, q, px, py, pz;
+        };
+        struct Fine {
+            double ip, in, fg;
+            int P, Nn;
+        };
+        auto coarse_load = [&](int r, int c) {
+            const size_t g = (size_t)(cI0 + r) * a.nc + cJ0 + c;
+            return Coarse{a.x_offt[g], a.y_offt[g], a.m[g], a.q[g], a.px[g], a.py[g], a.pz[g]};
+        };
+        auto coarse_store = [&](int r, int c, const Coarse& v) {
+            const int k = r * cW + c;
+            l.cpos[k] = make_double2(v.x, v.y);
+            l.cmq[k] = make_double2(sm * v.m, sm * v.q);
+            l.cpxy[k] = make_double2(sm * v.px, sm * v.py);
+            l.cpz[k] = sm * v.pz;
+            same = same && v.m == m0 && v.q == q0;
+        };
+        auto fine_load = [&](int k) {
+            const int f = k >= ni ? fj_a + k - ni : fi_a + k;
+            return Fine{a.ip[f], a.in[f], a.fg[f], clampi((int)a.P[f], a.nc),
+                        clampi((int)a.Nn[f], a.nc)};
+        };
+        auto fine_store = [&](int k, const Fine& v) {
+            const bool isj = k >= ni;
+            // (the j tables follow the i tables)
+            const int s = isj ? k - ni + a.fine_max : k, lo = isj ? cJ0 : cI0,
+                      hi = isj ? wmax : hmax, scale = isj ? 1 : cW;
+            l.wi[s] = make_double2(v.ip, v.in);
+            l.fi[s] = v.fg;
+            l.xi[s] = make_int4(min(max(v.P - lo, 0), hi) * scale,
+                                min(max(v.Nn - lo, 0), hi) * scale,
+                                cell_of(v.fg, N, a.h), 0);
+        };
+        // 16 x 16 threads over the rectangle; every thread's first entries of both
+        // tables on their way together, the rest (large ranges) in turn
+        const int tr = threadIdx.x >> 4, tc = threadIdx.x & 15;
+        const bool have_c = STAGED && tr < cH && tc < cW, have_f = (int)threadIdx.x < ni + nj;
+        Coarse first_c{};
+        Fine first_f{};
+        if (have_f) first_f = fine_load(threadIdx.x);
+        if constexpr (STAGED) {
+            if (have_c) first_c = coarse_load(tr, tc);
+            if (cH > 0 && cW > 0) {
+                const size_t first = (size_t)cI0 * a.nc + cJ0;
+                m0 = a.m[first];
+                q0 = a.q[first];
             }
-            // every thread has read the rectangle's corners: turn the
-            // neighbour indices into offsets in it, rows scaled by its
-            // width, each clamped into it, so that a row part plus a column
-            // part is an in-bounds index of cs
-            __syncthreads();
-            const int hmax = max(cH - 1, 0), wmax = max(cW - 1, 0);
-            for (int k = threadIdx.x; k < ni + nj; k += blockDim.x) {
-                if (k < ni) {
-                    ti.idx[k].x = min(max(ti.idx[k].x - cI0, 0), hmax) * cW;
-                    ti.idx[k].y = min(max(ti.idx[k].y - cI0, 0), hmax) * cW;
+        }
+        if (have_f) fine_store(threadIdx.x, first_f);
+        for (int k = threadIdx.x + kDepBlock; k < ni + nj; k += kDepBlock)
+            fine_store(k, fine_load(k));
+        if constexpr (STAGED) {
+            if (have_c) coarse_store(tr, tc, first_c);
+            for (int r = tr; r < cH; r += kDepBlock / 16)
+                for (int c = r == tr ? tc + 16 : tc; c < cW; c += 16)
+                    coarse_store(r, c, coarse_load(r, c));
+        }
+        const bool uniform = __syncthreads_and(same);
+        m0 = scalar(sm * m0);
+        q0 = scalar(sm * q0);
+        // can a particle's stencil centre lie outside [1, N - 2]?
+        const bool edge = ci0 < 2 * halo + 2 || ci0 + T + 2 * halo + 1 > N - 2 ||
+                          cj0 < 2 * halo + 2 || cj0 + T + 2 * halo + 1 > N - 2;
+        const int gs = a.group > 0 ? a.group : 1, gs2 = gs * gs;
+        const int ngi = (ni + gs - 1) / gs, ngj = (nj + gs - 1) / gs, ng = ngi * ngj;
+        const float per_row = 1.f / ngj;
+        // a particle at this offset in its cell (or above) is followed by one in
+        // the next cell within its group
+        const double roomy = scalar(.5 - (double)(gs - 1) / gs);
+        const int ih = N / 2;
+        constexpr int kNoCentre = -(1 << 20);
+        double pat[4][9];
+#pragma unroll
+        for (int k = 0; k < 36; ++k) (&pat[0][0])[k] = 0.;
+        // The last round of groups is rarely full, and wave w of every block sits
+        // on SIMD w: the blocks of a CU (256 apart in launch order) start the
+        // rounds at different waves, so that the extra ones spread over its SIMDs
+        const int start = (wave + (lin >> 8)) % (kDepBlock / 64) * 64 + lane + part * kDepBlock;
+#pragma unroll 1
+        for (int L = start; L < ng; L += nparts * kDepBlock) {
+            const int gi = (int)((L + .5f) * per_row), gj = L - gi * ngj;
+            int ai = kNoCentre, aj = kNoCentre;   // centre of the sums in pat
+            int qa = 0, qb = 0;     // particle of the group
+            bool swap = false;      // its rows first, then its columns
+            // the sums to the cells that are the tile's (none about kNoCentre)
+            auto flush = [&]() {
+                const int si = ai - 1 - ci0, sj = aj - 1 - cj0;
+                double* const p0 = l.acc + si * D::kPitch + sj;
+                bool in_i[3], in_j[3];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    in_i[r] = (unsigned)(si + r) < (unsigned)T;
+                    in_j[r] = (unsigned)(sj + r) < (unsigned)T;
+                }
+#pragma unroll
+                for (int k = 0; k < 9; ++k) {
+                    const int r = stencil_di(k) + 1, c = stencil_dj(k) + 1;
+                    if (in_i[r] & in_j[c]) {
+#pragma unroll
+                        for (int n = 0; n < 4; ++n)
+                            atomicAdd(p0 + r * D::kPitch + c + n * D::kComp, pat[n][k]);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 36; ++k) (&pat[0][0])[k] = 0.;
+            };
+#pragma unroll 1
+            for (int q = 0; q < gs2; ++q) {
+                // (opaque in the loop, or the compiler makes a copy of the whole
+                // loop for each value of the block's flags, with more registers)
+                int is_uniform = scalar(uniform), is_edge = scalar(edge);
+                asm volatile("" : "+s"(is_uniform), "+s"(is_edge));
+                const int li = gi * gs + (swap ? qb : qa), lj = gj * gs + (swap ? qa : qb);
+                if (++qb == gs) {
+                    qb = 0;
+                    ++qa;
+                }
+                if (li >= ni || lj >= nj) continue;
+                // coarse->fine interpolation (lcode.py:591-621), then TSC centre and
+                // offset in the cell (lcode.py:404-407)
+                const double2 wi = l.wi[li], wj = l.wj[lj];
+                const int4 xi = l.xi[li], xj = l.xj[lj];
+                const double wA = wi.x * wj.x, wB = wi.x * wj.y, wC = wi.y * wj.x,
+                             wD = wi.y * wj.y;
+                const int pp = xi.x + xj.x, pn = xi.x + xj.y;
+                const int np = xi.y + xj.x, nn = xi.y + xj.y;
+                double x, y;
+                if constexpr (STAGED) {
+                    const double2 cA = l.cpos[pp], cB = l.cpos[pn], cC = l.cpos[np],
+                                  cD = l.cpos[nn];
+                    x = l.fi[li] + (wA * cA.x + wB * cB.x + wC * cC.x + wD * cD.x);
+                    y = l.fj[lj] + (wA * cA.y + wB * cB.y + wC * cC.y + wD * cD.y);
                 } else {
-                    const int s = k - ni;
-                    tj.idx[s].x = min(max(tj.idx[s].x - cJ0, 0), wmax);
-                    tj.idx[s].y = min(max(tj.idx[s].y - cJ0, 0), wmax);
+#define LCODE_MIX(arr) (wA * arr[pp] + wB * arr[pn] + wC * arr[np] + wD * arr[nn])
+                    x = l.fi[li] + LCODE_MIX(a.x_offt);
+                    y = l.fj[lj] + LCODE_MIX(a.y_offt);
                 }
-            }
-        }
-        __syncthreads();
-        const A sm = (A)a.smallness;
-        // coarse->fine interpolation of tile-local fine particle (li, lj)
-        // (lcode.py:591-621): its position, and apart from it (only for the
-        // particles whose stencil reaches the tile) its deposition values
-        // (lcode.py:651-655)
-        auto position = [&](int li, int lj, double& x, double& y) {
-            const double2 wi = ti.w[li], wj = tj.w[lj];
-            const int4 xi = ti.idx[li], xj = tj.idx[lj];
-            const double wA = wi.x * wj.x, wB = wi.x * wj.y;
-            const double wC = wi.y * wj.x, wD = wi.y * wj.y;
-            if constexpr (STAGED) {
-                // row offset + column offset (both clamped into the staged
-                // rectangle above)
-                const int pp = xi.x + xj.x, pn = xi.x + xj.y;
-                const int np = xi.y + xj.x, nn = xi.y + xj.y;
-                const double2 cA = cpos[pp], cB = cpos[pn], cC = cpos[np], cD = cpos[nn];
-#define LCODE_MIXP(c) (wA * cA.c + wB * cB.c + wC * cC.c + wD * cD.c)
-                x = ti.fg[li] + LCODE_MIXP(x);
-                y = tj.fg[lj] + LCODE_MIXP(y);
-#undef LCODE_MIXP
-            } else {
-                const int nc = a.nc;
-                const int pp = xi.x * nc + xj.x, pn = xi.x * nc + xj.y;
-                const int np = xi.y * nc + xj.x, nn = xi.y * nc + xj.y;
-#define LCODE_MIXP(arr) (wA * arr[pp] + wB * arr[pn] + wC * arr[np] + wD * arr[nn])
-                x = ti.fg[li] + LCODE_MIXP(a.x_offt);
-                y = tj.fg[lj] + LCODE_MIXP(a.y_offt);
-#undef LCODE_MIXP
-            }
-        };
-        auto values = [&](int li, int lj, A* v) {
-            const double2 wi = ti.w[li], wj = tj.w[lj];
-            const int4 xi = ti.idx[li], xj = tj.idx[lj];
-            const A Ag = (A)(wi.x * wj.x), Bg = (A)(wi.x * wj.y);
-            const A Cg = (A)(wi.y * wj.x), Dg = (A)(wi.y * wj.y);
-            if constexpr (STAGED) {
-                const int pp = xi.x + xj.x, pn = xi.x + xj.y;
-                const int np = xi.y + xj.x, nn = xi.y + xj.y;
-                const A2 mA = cmq[pp], mB = cmq[pn], mC = cmq[np], mD = cmq[nn];
-                const A2 pA = cpxy[pp], pB = cpxy[pn], pC = cpxy[np], pD = cpxy[nn];
-#define LCODE_MIX(a, b, c, d) (Ag * (a) + Bg * (b) + Cg * (c) + Dg * (d))
-                deposit_values<A>(sm * LCODE_MIX(mA.x, mB.x, mC.x, mD.x),
-                                  sm * LCODE_MIX(mA.y, mB.y, mC.y, mD.y),
-                                  sm * LCODE_MIX(pA.x, pB.x, pC.x, pD.x),
-                                  sm * LCODE_MIX(pA.y, pB.y, pC.y, pD.y),
-                                  sm * LCODE_MIX(cpz[pp], cpz[pn], cpz[np], cpz[nn]), v);
-#undef LCODE_MIX
-            } else {
-                const int nc = a.nc;
-                const int pp = xi.x * nc + xj.x, pn = xi.x * nc + xj.y;
-                const int np = xi.y * nc + xj.x, nn = xi.y * nc + xj.y;
-#define LCODE_MIX(arr) (Ag * (A)arr[pp] + Bg * (A)arr[pn] + Cg * (A)arr[np] + Dg * (A)arr[nn])
-                deposit_values<A>(sm * LCODE_MIX(a.m), sm * LCODE_MIX(a.q),
-                                  sm * LCODE_MIX(a.px), sm * LCODE_MIX(a.py),
-                                  sm * LCODE_MIX(a.pz), v);
-#undef LCODE_MIX
-            }
-        };
-        // does the 3 x 3 stencil around centre (i, j) reach this tile?
-        auto reaches = [&](int i, int j) {
-            return i + 1 >= ci0 && i - 1 < ci0 + kTile && j + 1 >= cj0 && j - 1 < cj0 + kTile;
-        };
-        // TSC centre and weights of the particle; false when it moved more
-        // than the halo from its initial cell (its home tile lists it)
-        auto locate = [&](int li, int lj, double x, double y, TscT<A>& t) {
-            const int ci = ti.idx[li].z, cj = tj.idx[lj].z;   // initial cell
-            const bool home = ci >= ci0 && ci < ci0 + kTile &&
-                              cj >= cj0 && cj < cj0 + kTile;
-            if (!(fabs(x) <= kFarCells * a.h && fabs(y) <= kFarCells * a.h)) {
-                // non-finite or absurdly far particle (a deposition called
-                // without the pushes' bound): its home tile becomes NaN
-                if (home) {
-                    tile_nan = 1;
-                    if (a.host_flag)
-                        __hip_atomic_store(a.host_flag, 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_SYSTEM);
-                }
-                return false;
-            }
-            tsc_weights<A>(x, y, N, a.h, t, home ? a.fault : nullptr, inv_h);
-            if (abs(t.i - ci) > halo || abs(t.j - cj) > halo) {
-                // (beyond a bound the pushes reported: cannot happen; counted
-                // as a fault rather than listed for a pass that does not run)
-                if (home) {
-                    if (may_spill) {
-                        a.spill[atomicAdd(a.spill_count, 1)] = (fi_a + li) * a.nf + fj_a + lj;
-                        if (a.host_spill)
-                            __hip_atomic_store(a.host_spill, 1, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_SYSTEM);
+                // the deposition values (lcode.py:651-655) from the mixed mass,
+                // charge and momentum: dro = q gamma r, dj = q p r with r = 1 /
+                // (gamma - pz)
+                double v[4];
+                auto values = [&]() {
+                    double m, qq, px, py, pz;
+                    if (STAGED && is_uniform) {
+                        const double w = (wA + wB) + (wC + wD);
+                        m = w * m0;
+                        qq = w * q0;
+                    } else if constexpr (STAGED) {
+                        const double2 mA = l.cmq[pp], mB = l.cmq[pn], mC = l.cmq[np], mD = l.cmq[nn];
+                        m = wA * mA.x + wB * mB.x + wC * mC.x + wD * mD.x;
+                        qq = wA * mA.y + wB * mB.y + wC * mC.y + wD * mD.y;
                     } else {
-                        atomicAdd(a.fault, 1);
+                        m = sm * LCODE_MIX(a.m);
+                        qq = sm * LCODE_MIX(a.q);
                     }
-                }
-                return false;
-            }
-            return true;
-        };
-#if LCODE_DEP_GROUP
-        // One thread per group of gs x gs fine particles with consecutive
-        // indices (the tile's fine range starts at a cell edge, so with gs =
-        // fineness a group is the particles of one initial cell).  The
-        // thread sums the 3 x 3 x 4 stencil values of successive particles
-        // with a common stencil centre in registers and adds them to LDS
-        // when the centre changes and after the group's last particle.
-        // Adjacent lanes hold adjacent cells, so the atomics of one
-        // instruction hit distinct LDS addresses.
-        const int gs = a.group > 0 ? a.group : 1;
-        const int ngi = (ni + gs - 1) / gs, ngj = (nj + gs - 1) / gs;
-        // With LCODE_DEP_SPREAD the lanes of a wave take groups kSpread
-        // apart (g = L * stride mod n, the stride a prime that does not
-        // divide n, so the map is a permutation): where the wake compresses
-        // the plasma, adjacent groups' particles share cells, and adjacent
-        // lanes would then add to the same LDS addresses in one instruction.
-        const int ng = ngi * ngj;
-        int stride = 1;
-        if (LCODE_DEP_SPREAD) {
-            constexpr int kPrimes[6] = {13, 17, 19, 23, 29, 31};
-            stride = kPrimes[5];
-#pragma unroll
-            for (int u = 5; u >= 0; --u)
-                if (ng % kPrimes[u] != 0) stride = kPrimes[u];
-        }
-        for (int L = threadIdx.x + part * blockDim.x; L < ng; L += nparts * blockDim.x) {
-            const int g = LCODE_DEP_SPREAD ? (int)((long long)L * stride % ng) : L;
-            const int gi = g / ngj, gj = g - gi * ngj;
-            A pat[4][9];
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int k = 0; k < 9; ++k) pat[c][k] = 0;
-            int ai = -1, aj = -1;   // centre of the sums in pat (-1: none)
-            int qi = 0, qj = 0;     // particle (qi, qj) of the group
-            for (int q = 0; q <= gs * gs; ++q) {
-                const int li = gi * gs + qi, lj = gj * gs + qj;
-                if (++qj == gs) {
-                    qj = 0;
-                    ++qi;
-                }
-                A v[4] = {0, 0, 0, 0};
-                TscT<A> t;
-                t.i = t.j = -1;
-                if (q < gs * gs && li < ni && lj < nj) {
-                    double x, y;
-                    position(li, lj, x, y);
-                    if (!locate(li, lj, x, y, t) || !reaches(t.i, t.j)) t.i = -1;
-                    else values(li, lj, v);
-                }
-                if (ai >= 0 && (t.i != ai || t.j != aj)) {
-                    if (q == gs * gs || t.i >= 0) {
-                        lds_deposit<A>(acc, ai, aj, ci0, cj0, nullptr, nullptr, pat);
-#pragma unroll
-                        for (int c = 0; c < 4; ++c)
-#pragma unroll
-                            for (int k = 0; k < 9; ++k) pat[c][k] = 0;
-                        ai = -1;
+                    if constexpr (STAGED) {
+                        const double2 pA = l.cpxy[pp], pB = l.cpxy[pn], pC = l.cpxy[np],
+                                      pD = l.cpxy[nn];
+                        px = wA * pA.x + wB * pB.x + wC * pC.x + wD * pD.x;
+                        py = wA * pA.y + wB * pB.y + wC * pC.y + wD * pD.y;
+                        pz = wA * l.cpz[pp] + wB * l.cpz[pn] + wC * l.cpz[np] + wD * l.cpz[nn];
+                    } else {
+                        px = sm * LCODE_MIX(a.px);
+                        py = sm * LCODE_MIX(a.py);
+                        pz = sm * LCODE_MIX(a.pz);
+#undef LCODE_MIX
                     }
+                    double gamma, inv;
+                    gamma_and_inverse(m * m + px * px + py * py + pz * pz, pz, gamma, inv);
+                    const double qr = qq * inv;
+                    v[0] = gamma * qr;
+                    v[1] = px * qr;
+                    v[2] = py * qr;
+                    v[3] = pz * qr;
+                };
+                if constexpr (kEarly) values();
+                const double xh = in_cells(x, inv_h), yh = in_cells(y, inv_h);
+                const double fx = floor(xh), fy = floor(yh);
+                const double xl = xh - fx - .5, yl = yh - fy - .5;
+                // (.5 + x)^2 / 2, (.5 - x)^2 / 2 and .75 - x^2
+                const double wxP = fma(xl, fma(xl, .5, .5), .125), wxM = fma(xl, fma(xl, .5, -.5), .125);
+                const double wyP = fma(yl, fma(yl, .5, .5), .125), wyM = fma(yl, fma(yl, .5, -.5), .125);
+                const double wx[3] = {wxM, fma(-xl, xl, .75), wxP};
+                const double wy[3] = {wyP, fma(-yl, yl, .75), wyM};   // stencil order
+                int ti = (int)fx + ih, tj = (int)fy + ih;
+                const int ci = xi.z, cj = xj.z;   // initial cell
+                const bool home = ((unsigned)(ci - ci0) < (unsigned)T) &
+                                  ((unsigned)(cj - cj0) < (unsigned)T);
+                // (NaN where the position is not finite)
+                const bool odd = __builtin_isunordered(xl, yl);
+                if (is_edge && !odd && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2)) {
+                    if (home) atomicAdd(a.fault, 1);
+                    ti = min(max(ti, 1), N - 2);
+                    tj = min(max(tj, 1), N - 2);
                 }
-                if (t.i >= 0) {
-                    ai = t.i;
-                    aj = t.j;
+                if (q == 0) swap = yl >= roomy;
+                if (odd | ((unsigned)(ti - ci + halo) > 2u * halo) |
+                    ((unsigned)(tj - cj + halo) > 2u * halo)) {
+                    if (home) {
+                        if (odd || !(fabs(xh) <= kFarCells && fabs(yh) <= kFarCells)) {
+                            // non-finite or absurdly far particle (a deposition
+                            // called without the pushes' bound): its home tile
+                            // becomes NaN
+                            tile_nan = 1;
+                            if (a.host_flag)
+                                __hip_atomic_store(a.host_flag, 1, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_SYSTEM);
+                        } else {
+                            // moved more than the halo: its home tile lists it
+                            // (beyond a bound the pushes reported: cannot happen;
+                            // counted as a fault rather than listed for a pass
+                            // that does not run)
+                            if (!is_edge && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2))
+                                atomicAdd(a.fault, 1);
+                            if (may_spill) {
+                                a.spill[atomicAdd(a.spill_count, 1)] =
+                                    (fi_a + li) * a.nf + fj_a + lj;
+                                if (a.host_spill)
+                                    __hip_atomic_store(a.host_spill, 1, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_SYSTEM);
+                            } else {
+                                atomicAdd(a.fault, 1);
+                            }
+                        }
+                    }
+                    continue;
+                }
+                // does the 3 x 3 stencil reach this tile?
+                if (((unsigned)(ti + 1 - ci0) >= (unsigned)(T + 2)) |
+                    ((unsigned)(tj + 1 - cj0) >= (unsigned)(T + 2)))
+                    continue;
+                if ((ti != ai) | (tj != aj)) {
+                    if (ai != kNoCentre) flush();   // another centre
+                    ai = ti;
+                    aj = tj;
+                }
+                if constexpr (!kEarly) values();
 #pragma unroll
-                    for (int k = 0; k < 9; ++k)
+                for (int k = 0; k < 9; ++k) {
+                    const double w = wx[k % 3] * wy[k / 3];
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) pat[c][k] += v[c] * t.w[k];
+                    for (int n = 0; n < 4; ++n) pat[n][k] += v[n] * w;
                 }
             }
+            flush();
         }
-#else
-        for (int p = threadIdx.x + part * blockDim.x; p < ni * nj; p += nparts * blockDim.x) {
-            const int li = p / nj, lj = p - li * nj;
-            double x, y;
-            A v[4];
-            position(li, lj, x, y);
-            TscT<A> t;
-            if (!locate(li, lj, x, y, t) || !reaches(t.i, t.j)) continue;
-            values(li, lj, v);
-            lds_deposit<A>(acc, t.i, t.j, ci0, cj0, v, t.w, nullptr);
-        }
-#endif
+    }
+    // the ion background of this thread's cells, on its way while the block's
+    // other waves finish
+    constexpr int kOut = (T * T + kDepBlock - 1) / kDepBlock;
+    double base[kOut];
+#pragma unroll
+    for (int u = 0; u < kOut; ++u) {
+        const int k = threadIdx.x + u * kDepBlock;
+        const int i = ci0 + k / T, j = cj0 + k % T;
+        base[u] = 0.;
+        if (k < T * T && i < N && j < N && a.ro_initial)
+            base[u] = a.ro_initial[(size_t)i * N + j];
     }
     __syncthreads();
     // a split tile: both parts publish their sums (all NaN from a part that
@@ -715,8 +809,6 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
     // second to finish adds the other's sums to its own and stores the tile
     bool store = true;
     if (nparts == 2) {
-        constexpr int kAcc = 4 * kTile * kTile;
-        double* const sums = &acc[0][0][0];
         double* const mine = a.split_part + ((size_t)slot * 2 + part) * kAcc;
         const double* const other = a.split_part + ((size_t)slot * 2 + 1 - part) * kAcc;
         // The sums travel as device-scope atomic stores and loads (written
@@ -726,8 +818,8 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
         // stores).  A device-scope fence instead writes back and invalidates
         // the whole L2 of the XCD, under every other block there (measured:
         // 40.7 -> 58.6 us per launch with 39 split tiles).
-        for (int k = threadIdx.x; k < kAcc; k += blockDim.x)
-            __hip_atomic_store(mine + k, tile_nan ? __builtin_nan("") : sums[k],
+        for (int k = threadIdx.x; k < kAcc; k += kDepBlock)
+            __hip_atomic_store(mine + k, tile_nan ? __builtin_nan("") : l.acc[k],
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_s_waitcnt(0);   // vmcnt, expcnt and lgkmcnt all zero
         __syncthreads();
@@ -735,33 +827,21 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
         __syncthreads();
         store = split_last;
         if (store) {
-            for (int k = threadIdx.x; k < kAcc; k += blockDim.x)
-                sums[k] += __hip_atomic_load(other + k, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
+            for (int k = threadIdx.x; k < kAcc; k += kDepBlock)
+                l.acc[k] += __hip_atomic_load(other + k, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
             if (threadIdx.x == 0) a.split_count[slot] = 0;
             __syncthreads();
         }
     }
-    // store the tile, adding the ion background to ro last (lcode.py:687);
-    // all background loads are issued before the first store
-    constexpr int kOut = (kTile * kTile + kDepBlock - 1) / kDepBlock;
+    // store the tile, adding the ion background to ro last (lcode.py:687)
     if (store) {
-        double base[kOut];
 #pragma unroll
         for (int u = 0; u < kOut; ++u) {
             const int k = threadIdx.x + u * kDepBlock;
-            const int r = k / kTile, c = k % kTile;
+            const int r = k / T, c = k % T;
             const int i = ci0 + r, j = cj0 + c;
-            base[u] = 0.;
-            if (k < kTile * kTile && i < N && j < N && a.ro_initial)
-                base[u] = a.ro_initial[(size_t)i * N + j];
-        }
-#pragma unroll
-        for (int u = 0; u < kOut; ++u) {
-            const int k = threadIdx.x + u * kDepBlock;
-            const int r = k / kTile, c = k % kTile;
-            const int i = ci0 + r, j = cj0 + c;
-            if (k >= kTile * kTile || i >= N || j >= N) continue;
+            if (k >= T * T || i >= N || j >= N) continue;
             const size_t idx = (size_t)i * N + j;
             G* const ro = gp<G>(a.ro);
             G* const jx = gp<G>(a.jx);
@@ -771,11 +851,12 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
                 ro[idx] = jx[idx] = jy[idx] = jz[idx] = (G)__builtin_nan("");
                 continue;
             }
+            const double* s = l.acc + r * D::kPitch + c;
             // the FP64 ion background is added in FP64, then rounded once
-            ro[idx] = (G)(a.ro_initial ? acc[0][r][c] + base[u] : acc[0][r][c]);
-            jx[idx] = (G)acc[1][r][c];
-            jy[idx] = (G)acc[2][r][c];
-            jz[idx] = (G)acc[3][r][c];
+            ro[idx] = (G)(a.ro_initial ? s[0] + base[u] : s[0]);
+            jx[idx] = (G)s[D::kComp];
+            jy[idx] = (G)s[2 * D::kComp];
+            jz[idx] = (G)s[3 * D::kComp];
         }
     }
     // a particle may have spilled somewhere (the bound every block read
@@ -785,14 +866,14 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
         __threadfence();   // every thread's stores visible at device scope
         __syncthreads();
         if (threadIdx.x == 0)
-            last_block = atomicAdd(a.done, 1) == (int)(gridDim.x * gridDim.y) - 1;
+            last_block = atomicAdd(a.done, 1) == (int)gridDim.x - 1;
         __syncthreads();
         if (last_block) {
             __threadfence();
             const int count = __hip_atomic_load(a.spill_count, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
-            for (int p = threadIdx.x; p < count; p += blockDim.x)
-                deposit_spill_one<A, G>(a, a.spill[p], N);
+            for (int p = threadIdx.x; p < count; p += kDepBlock)
+                deposit_spill_one<G>(a, a.spill[p], N);
             if (threadIdx.x == 0) *a.done = 0;
         }
     }
@@ -802,7 +883,7 @@ __device__ __forceinline__ void deposit_tile_body(const DepositArgs& a) {
 // halo, with device-scope atomics over the whole grid (after the tile
 // kernel's stores, which it follows on the stream), and zeroes the count
 // slot of the next call.  An empty list costs one load per block.
-template <typename A, typename G>
+template <typename G>
 __global__ void __launch_bounds__(kBlock)
 deposit_spill_kernel(DepositArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.spill_next = 0;
@@ -810,13 +891,35 @@ deposit_spill_kernel(DepositArgs a) {
     const int count = *a.spill_count;
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < count;
          p += gridDim.x * blockDim.x)
-        deposit_spill_one<A, G>(a, a.spill[p], a.N);
+        deposit_spill_one<G>(a, a.spill[p], a.N);
 }
 
-template <bool STAGED, typename A, typename G>
-__global__ void __launch_bounds__(kDepBlock) LCODE_DEP_ATTR
-deposit_tile_kernel(DepositArgs a) {
-    deposit_tile_body<STAGED, A, G>(a);
+// The displacement bound of a deposition without a push before it: raises
+// *bound to the cells that the coarse offsets move a particle at most, or to
+// halo + 1 (which sends the deposition to its largest halo and the spill list)
+// when an offset is not finite or larger, or when an interpolation weight would
+// let a fine particle move further than its coarse ones.  4 us at 641^2,
+// against the largest halo's three times as many particles per tile and a
+// device-wide fence in every block (lcode_deposit 122 -> 39 us).
+__global__ void __launch_bounds__(kBlock)
+deposit_bound_kernel(DepositArgs a, int* bound) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    int cells = 0;
+    if (k < a.nc * a.nc) {
+        // (rounded up by more than the interpolation's rounding)
+        const double d = fmax(fabs(a.x_offt[k]), fabs(a.y_offt[k])) * (1. + 1e-9) / a.h;
+        const bool finite = isfinite(a.x_offt[k]) && isfinite(a.y_offt[k]);
+        cells = finite && d <= a.halo ? (int)ceil(d) : a.halo + 1;
+    }
+    if (k < a.nf) {
+        const double p = a.ip[k], n = a.in[k];
+        if (!(p >= 0. && n >= 0. && p + n <= 1. + 1e-10)) cells = a.halo + 1;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) cells = max(cells, __shfl_xor(cells, off, 64));
+    if ((threadIdx.x & 63) == 0 &&
+        cells > __hip_atomic_load(bound, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(bound, cells);
 }
 
 __global__ void __launch_bounds__(64) zero_ints_kernel(int* p, int n) {
@@ -927,6 +1030,15 @@ int launch_make_plasma(const PlasmaArgs& a, hipStream_t s) {
     return LCODE_OK;
 }
 
+int launch_deposit_bound(const DepositArgs& a, int* bound, hipStream_t s, Profiler* prof) {
+    ProfScope ps(prof, "deposit_bound", s, true);
+    const int n = std::max(a.nc * a.nc, a.nf);
+    if (n > 0)
+        launch_timed(ps, deposit_bound_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, a, bound);
+    LCODE_HIP(hipGetLastError());
+    return LCODE_OK;
+}
+
 int launch_zero_ints(int* p, int n, hipStream_t s) {
     if (n <= 0) return LCODE_OK;
     zero_ints_kernel<<<1, 64, 0, s>>>(p, n);
@@ -934,54 +1046,81 @@ int launch_zero_ints(int* p, int n, hipStream_t s) {
     return LCODE_OK;
 }
 
-int deposit_blocks_per_cu(bool staged) {
-    int a = 0, b = 0;
-    hipError_t e1, e2;
-    if (staged) {
-        e1 = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &a, deposit_tile_kernel<true, double, double>, kDepBlock, 0);
-        e2 = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &b, deposit_tile_kernel<true, double, float>, kDepBlock, 0);
-    } else {
-        e1 = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &a, deposit_tile_kernel<false, double, double>, kDepBlock, 0);
-        e2 = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &b, deposit_tile_kernel<false, double, float>, kDepBlock, 0);
+// The tile kernel for a tile, its waves per SIMD and forms, or NULL.
+using DepKernel = void (*)(DepositArgs);
+template <int T, int W>
+static DepKernel deposit_kernel_of(bool staged, bool grid32) {
+    if (staged)
+        return grid32 ? deposit_tile_kernel<T, W, true, float> : deposit_tile_kernel<T, W, true, double>;
+    return grid32 ? deposit_tile_kernel<T, W, false, float> : deposit_tile_kernel<T, W, false, double>;
+}
+static DepKernel deposit_kernel_of(int tile, int waves, bool staged, bool grid32) {
+    switch (tile * 10 + waves) {
+        case 83: return deposit_kernel_of<8, 3>(staged, grid32);
+        case 163: return deposit_kernel_of<16, 3>(staged, grid32);
+        case 243: return deposit_kernel_of<24, 3>(staged, grid32);
+        case 244: return deposit_kernel_of<24, 4>(staged, grid32);
+        default: return nullptr;
     }
-    if (e1 != hipSuccess || e2 != hipSuccess) {
-        (void)hipGetLastError();   // leave no error behind for later checks
-        return 0;
+}
+
+int deposit_blocks_per_cu(const DepositPlan& p) {
+    int least = 0;
+    for (const bool grid32 : {false, true}) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &n, reinterpret_cast<const void*>(deposit_kernel_of(p.tile, p.waves, p.staged, grid32)),
+                kDepBlock, deposit_lds_bytes(p.tile, p.fine_max, p.staged ? p.coarse_max : 0)) !=
+            hipSuccess) {
+            (void)hipGetLastError();   // leave no error behind for later checks
+            return 0;
+        }
+        least = grid32 ? std::min(least, n) : n;
     }
-    return std::min(a, b);
+    return least;
+}
+
+// Small grids take small tiles: 24-cell ones would leave CUs idle (36 tiles at
+// 129^2) and the launch as long as the chain of one tile.  us per launch, 24 /
+// 16 / 8 cells: 129^2 25.3 / - / 12.3, 361^2 28.8 / 20.5 / -, 641^2 34.7 / 46.6 /
+// -; larger tiles than 24 leave too few blocks at 641^2 or too few registers
+// for the waves (32 cells with 8 waves 34.8 - 52).  In launches of several
+// rounds four waves per SIMD hide more of a tile's start than three (1281^2,
+// fineness 3: 190 -> 178), in one round they leave the same waves and fewer
+// registers (641^2: 34.7 -> 37.6).
+DepositPlan deposit_plan(int N, int coarseness, int fineness, int cus) {
+    DepositPlan p{};
+    p.tile = N <= 200 ? 8 : N <= 400 ? 16 : 24;
+    p.nt = (N + p.tile - 1) / p.tile;
+    p.waves = p.tile == 24 && p.nt * p.nt > 3 * cus ? 4 : 3;
+    const int ext = p.tile + 2 * kDepositHalo + 2;   // initial cells per side, at most
+    p.fine_max = std::max(fineness, 3) * ext;        // (a denser grid than configured fits too)
+    // the coarse rectangle of a tile has at most ext / coarseness + 3 rows;
+    // staged while three blocks share a CU's LDS
+    p.coarse_max = ext / coarseness + 3;
+    p.staged = deposit_lds_bytes(p.tile, p.fine_max, p.coarse_max) <= 53 * 1024;
+    return p;
 }
 
 int launch_deposit(const DepositArgs& a, hipStream_t s, Profiler* prof) {
-    LCODE_REQUIRE(a.ntx == (a.N + kTile - 1) / kTile, "deposition: tiles per side do not match N");
+    LCODE_REQUIRE(a.ntx == (a.N + a.tile - 1) / a.tile, "deposition: tiles per side do not match N");
     LCODE_REQUIRE(a.nsplit >= 0 && a.nsplit <= a.ntx * a.ntx &&
-                      (!a.nsplit || (a.split_tile && a.split_slot && a.split_part && a.split_count)),
+                      (!a.nsplit || (a.tile_order && a.split_part && a.split_count)),
                   "deposition: inconsistent split tiles");
-    const dim3 grid(a.ntx * a.ntx + a.nsplit);
+    const DepKernel kernel = deposit_kernel_of(a.tile, a.waves, a.staged, a.grid32);
+    LCODE_REQUIRE(kernel, "deposition: no kernel for this tile");
     {
         ProfScope ps(prof, "deposit_tile", s, true);
-        const dim3 block(kDepBlock);
-        if (a.grid32 && a.staged)
-            launch_timed(ps, deposit_tile_kernel<true, double, float>, grid, block, 0, s, a);
-        else if (a.grid32)
-            launch_timed(ps, deposit_tile_kernel<false, double, float>, grid, block, 0, s, a);
-        else if (a.staged)
-            launch_timed(ps, deposit_tile_kernel<true, double, double>, grid, block, 0, s, a);
-        else
-            launch_timed(ps, deposit_tile_kernel<false, double, double>, grid, block, 0, s, a);
+        launch_timed(ps, kernel, dim3(a.ntx * a.ntx + a.nsplit), dim3(kDepBlock),
+                     deposit_lds_bytes(a.tile, a.fine_max, a.staged ? a.coarse_max : 0), s, a);
     }
     LCODE_HIP(hipGetLastError());
     if (!a.spill_in_tiles) {
         ProfScope ps(prof, "deposit_spill", s, true);
         if (a.grid32)
-            launch_timed(ps, deposit_spill_kernel<double, float>, dim3(kSpillBlocks),
-                         dim3(kBlock), 0, s, a);
+            launch_timed(ps, deposit_spill_kernel<float>, dim3(kSpillBlocks), dim3(kBlock), 0, s, a);
         else
-            launch_timed(ps, deposit_spill_kernel<double, double>, dim3(kSpillBlocks),
-                         dim3(kBlock), 0, s, a);
+            launch_timed(ps, deposit_spill_kernel<double>, dim3(kSpillBlocks), dim3(kBlock), 0, s, a);
     }
     LCODE_HIP(hipGetLastError());
     return LCODE_OK;
