@@ -31,10 +31,7 @@ struct lcode_workspace {
     int trick_on = 0;
     int nc = 0, nf = 0;
     SolverGeom geom{};
-    double* costab = nullptr;      // quarter-wave cosine table
-    double2* stage_tw = nullptr;   // static-plan stage twiddles
-    double2* wave_tw = nullptr;    // wave FFT twiddles W_L^t
-    float* costab32 = nullptr;
+    double2* fft_tw = nullptr;     // roots of unity of the FFT's stages
     int fp32 = 0;                  // FP32 transforms (FFT32, MIXED)
     int solver = 0;                // LCODE_SOLVER_*
     int grid32 = 0;                // set for the duration of a mixed step:
@@ -97,29 +94,6 @@ struct lcode_workspace {
 };
 
 namespace {
-
-#ifndef LCODE_TW_LDS_OK
-#define LCODE_TW_LDS_OK 1
-#endif
-// Line pairs per FFT block (at most).  One pair per block measured best at
-// 641^2 (six-field solve FP64 79.6 -> 74.2 us, FP32 66.1 -> 61.3 us against
-// up to four): the same pairs per CU, a quarter or half the waves behind
-// each barrier, and a finer-grained last round of blocks.
-#ifndef LCODE_FFT_MAX_PAIRS_F64
-#define LCODE_FFT_MAX_PAIRS_F64 1
-#endif
-#ifndef LCODE_FFT_MAX_PAIRS_F32
-#define LCODE_FFT_MAX_PAIRS_F32 1
-#endif
-// Static-plan twiddle roots go to LDS when the block has at least this many
-// line pairs (else they are read through the caches).  With one pair per
-// block, LDS roots measured 74.0 -> 72.4 us (FP64) and 62.3 -> 60.2 us (FP32).
-#ifndef LCODE_TW_LDS_MIN_PAIRS
-#define LCODE_TW_LDS_MIN_PAIRS 1
-#endif
-#ifndef LCODE_SOLVER_MAX_LDS
-#define LCODE_SOLVER_MAX_LDS 65536
-#endif
 
 // 1: per-tile displacement bounds size each deposition tile's halo; 0: the
 // largest bound over all particles sizes every tile's halo (build option)
@@ -237,19 +211,11 @@ std::vector<double> tri_table(int N, int ld, double h, bool dirichlet, int k0, i
     return t;
 }
 
-bool factor_radices(int L, FftPlan& plan) {
-    plan.L = L;
-    plan.nstages = 0;
-    int rest = L;
-    const int radices[] = {4, 2, 3, 5};
-    for (int r : radices) {
-        while (rest % r == 0) {
-            if (plan.nstages == kMaxStages) return false;
-            plan.radix[plan.nstages++] = r;
-            rest /= r;
-        }
-    }
-    return rest == 1;
+// L = 2^a 3^b 5^c
+bool smooth_length(int L) {
+    for (int r : {2, 3, 5})
+        while (L % r == 0) L /= r;
+    return L == 1;
 }
 
 // Second-difference eigenvalues 4/h^2 sin^2(k pi / (2 (N - 1)))
@@ -340,6 +306,8 @@ RhsInputs rhs_base(const lcode_config* c) {
     in.trick = c->subtraction_trick;
     in.h = c->grid_step_size;
     in.dxi = c->xi_step_size;
+    in.inv_h2 = 1 / (c->grid_step_size * 2);
+    in.inv_dxi = 1 / c->xi_step_size;
     return in;
 }
 
@@ -379,87 +347,24 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     ws->solver = cfg->solver;
     ws->fp32 = cfg->solver == LCODE_SOLVER_FFT32 || cfg->solver == LCODE_SOLVER_MIXED;
     g.fp32 = ws->fp32;
-    const int cplx = ws->fp32 ? (int)sizeof(float2) : (int)sizeof(double2);
     const int L = 2 * (N - 1);
-    if (!factor_radices(L, g.fft)) {
+    if (!smooth_length(L)) {
         set_error("2 (grid_steps - 1) = " + std::to_string(L) +
                   " has a prime factor other than 2, 3, 5");
         return fail(LCODE_E_UNSUPPORTED);
     }
-    g.static_L = solver_static_length(L) ? L : 0;
-    g.Tp = solver_threads_per_pair(L, ws->fp32, g.static_L != 0);
-    const int max_lds = LCODE_SOLVER_MAX_LDS;   // per block, bytes
-    // line pairs per block: as many as 1024 threads and the LDS limit allow,
-    // at most LCODE_FFT_MAX_PAIRS_F64 / _F32
-    const int max_pairs = ws->fp32 ? LCODE_FFT_MAX_PAIRS_F32 : LCODE_FFT_MAX_PAIRS_F64;
-    auto pairs_for = [&](int fixed_bytes) {
-        int P = 1024 / g.Tp;
-        const int by_lds = (max_lds - fixed_bytes) / (solver_padded_len(L) * cplx);
-        if (by_lds < P) P = by_lds;
-        return P > max_pairs ? max_pairs : P;
-    };
-    int P;
-    if (g.static_L) {
-        // stage twiddles in LDS when the block keeps LCODE_TW_LDS_MIN_PAIRS pairs
-        P = pairs_for(solver_tw_count(L) * (int)sizeof(double2));   // FP64 roots
-        g.tw_lds = LCODE_TW_LDS_OK && P >= LCODE_TW_LDS_MIN_PAIRS;
-        if (!g.tw_lds) P = pairs_for(0);
-    } else {
-        g.tw_lds = 0;
-        P = pairs_for((L / 4 + 1) * cplx / 2);
-    }
-    if (P < 1) {
+    // (the largest lengths the solvers take)
+    if (L > (ws->fp32 ? 4096 : 3640)) {
         set_error("grid too large for one FFT line pair in 64 KiB of LDS");
         return fail(LCODE_E_UNSUPPORTED);
     }
-    g.P = P;
-    if ((N + g.Tp - 1) / g.Tp > 4) {
-        set_error("internal: too many points per thread");
+    if (!solver_fft_plan(L, &g.fft)) {
+        set_error("internal: no FFT plan for " + std::to_string(L) + " points");
         return fail(LCODE_E_UNSUPPORTED);
     }
-    if (g.static_L) {
-        // stage with span sp and radix R: exp(-2 pi i k / (sp R)), k < sp,
-        // after the entries of the earlier stages (the kernels form the
-        // powers q = 2 .. R - 1)
-        std::vector<double2> tw(solver_tw_count(L));
-        int off = 0;
-        for (int sp = 1, R = 1; sp < L; sp *= R) {
-            R = solver_static_radix(L / sp);
-            for (int k = 0; k < sp; ++k) {
-                const long double a = 2.0L * 3.14159265358979323846264338327950288L *
-                                      k / ((long double)sp * R);
-                tw[off + k] = make_double2((double)std::cos(a), (double)-std::sin(a));
-            }
-            off += sp;
-        }
-        if ((rc = upload(ws, &ws->stage_tw, tw))) return fail(rc);
-        g.stage_tw = ws->stage_tw;
-    }
-
-    g.wave_tw = nullptr;
-    if (solver_wave_length(L) && (!ws->fp32 || (LCODE_FFT_WAVE_FP32 && L == 1280))) {
-        // W_L^t = exp(-2 pi i t / L) for every t < L
-        std::vector<double2> wt(L);
-        for (int t = 0; t < L; ++t) {
-            const long double a = 2.0L * 3.14159265358979323846264338327950288L * t / L;
-            wt[t] = make_double2((double)std::cos(a), (double)-std::sin(a));
-        }
-        if ((rc = upload(ws, &ws->wave_tw, wt))) return fail(rc);
-        g.wave_tw = ws->wave_tw;
-    }
-
-    std::vector<double> costab(L / 4 + 1);
-    for (int r = 0; r <= L / 4; ++r) {
-        const long double a = 2.0L * 3.14159265358979323846264338327950288L * r / L;
-        costab[r] = (double)std::cos(a);
-    }
-    if ((rc = upload(ws, &ws->costab, costab))) return fail(rc);
-    g.costab = ws->costab;
-    if (ws->fp32) {
-        std::vector<float> c32(costab.begin(), costab.end());
-        if ((rc = upload(ws, &ws->costab32, c32))) return fail(rc);
-        g.costab32 = ws->costab32;
-    }
+    const std::vector<double2> tw = solver_fft_roots(g.fft);
+    if ((rc = upload(ws, &ws->fft_tw, tw))) return fail(rc);
+    g.tw = ws->fft_tw;
 
     const int add = ws->trick_on ? 1 : 0;
     g.ld = (N + 15) / 16 * 16;   // whole 128-byte lines of FP64 spectra
@@ -602,10 +507,8 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
         LCODE_HIP(hipMemset(ws->zero64, 0, n2 * sizeof(double)));
     }
     {
-        // last FFT pass: ceil(N / (2 P)) blocks per field (one line pair per
-        // block in the wave FFT), six fields: sized for P = 1, the most
-        const int per_block = 2;
-        const size_t nblk = (size_t)6 * ((N + per_block - 1) / per_block);
+        // last FFT pass: a block per field and pair of rows
+        const size_t nblk = (size_t)6 * ((N + 1) / 2);
         if ((rc = dev_alloc(ws, (void**)&ws->resid_part, 2 * nblk * sizeof(double))))
             return fail(rc);
     }

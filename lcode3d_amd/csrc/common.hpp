@@ -10,6 +10,7 @@
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "../../include/lcode3d_hip.h"
 
@@ -361,12 +362,30 @@ int launch_zero_ints(int* p, int n, hipStream_t s);
 enum FieldKind { F_EX = 0, F_EY = 1, F_EZ = 2, F_BX = 3, F_BY = 4, F_BZ = 5 };
 enum Xform { XF_DCT = 0, XF_DST = 1 };
 
-constexpr int kMaxStages = 24;
+constexpr int kMaxStages = 5;
+
+// The half-extension FFT of L = R1 T points (fields.hip): a first stage of
+// radix R1 on `lanes` lanes, then stages of product T over K columns.
+// Radix, span (product of the earlier stages' radices) and stride T / radix of a
+// stage in one word (5, 13, 14 bits).
+__host__ __device__ constexpr unsigned fft_word(int R, int span, int stride) {
+    return (unsigned)R | (unsigned)span << 5 | (unsigned)stride << 18;
+}
+__host__ __device__ constexpr int fft_word_radix(unsigned w) { return w & 31; }
+__host__ __device__ constexpr int fft_word_span(unsigned w) { return w >> 5 & 8191; }
+__host__ __device__ constexpr int fft_word_stride(unsigned w) { return w >> 18; }
 
 struct FftPlan {
     int L;                       // 2 (N - 1)
-    int nstages;
-    int radix[kMaxStages];
+    int R1, T;
+    int K, KP;                   // R1 / 2 + 1, made odd
+    int lanes;                   // T / 2 + 1
+    int threads;                 // of a block (one pair of rows)
+    unsigned k_inv;              // ceil(2^32 / K)
+    int nfirst, nroots;          // roots of the first stage, of the others
+    int nst;
+    unsigned word[kMaxStages];   // fft_word of each
+    unsigned span_inv[kMaxStages];   // ceil(2^32 / span), span > 1
 };
 
 // Sources of the right-hand sides (lcode.py:166-168, :258-268, :339-343).
@@ -378,6 +397,7 @@ struct RhsInputs {
     const double* beam;                   // NULL: beam_scalar everywhere
     double beam_scalar;
     double trick, h, dxi;
+    double inv_h2, inv_dxi;               // 1 / (2 h), 1 / dxi, rounded
     // FP32-grid form: an FP64 grid of N * N zeros read in place of a
     // missing beam array (the grid members above then point to floats)
     const double* zero64;
@@ -413,6 +433,17 @@ __device__ __forceinline__ double jz_src(const RhsInputs& in, size_t idx) {
     return r + beam_at<G>(in, idx);
 }
 
+// x / d with inv = 1 / d rounded to nearest: the product is within an ulp, the
+// remainder of the fused multiply-add exact, so the corrected quotient is the
+// rounded one (Markstein's theorem; d with an all-ones mantissa and results
+// near the smallest normals may be an ulp off).  The fixup gives division's
+// infinities, zeros and NaN.  (Pass A, division -> this: 641^2 with FP32 transforms
+// 18.4 -> 16.6 us, 1281^2 96.8 -> 94.1.)
+__device__ __forceinline__ double quotient(double x, double d, double inv) {
+    const double q = x * inv;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-q, d, x), inv, q), d, x);
+}
+
 // The right-hand side of field `kind` at (i, j).  Outside the interior the
 // derivative terms are zero; their neighbour offsets then collapse to the
 // point itself, so every load stays in bounds for any (i, j) of the grid.
@@ -422,33 +453,34 @@ __device__ __forceinline__ double rhs_value_k(int i, int j, int N,
     const size_t idx = (size_t)i * N + j;
     const bool inner = i >= 1 && i <= N - 2 && j >= 1 && j <= N - 2;
     const size_t oi = inner ? (size_t)N : 0, oj = inner ? 1 : 0;
-    const double h2 = in.h * 2;
+    auto over_h2 = [&](double x) { return quotient(x, in.h * 2, in.inv_h2); };
+    auto over_dxi = [&](double x) { return quotient(x, in.dxi, in.inv_dxi); };
     const G *jx = gp<G>(in.jx), *jy = gp<G>(in.jy);
     const G *jxp = gp<G>(in.jx_prev), *jyp = gp<G>(in.jy_prev);
     if constexpr (KIND == F_EX) {
-        const double d = (rho_src<G>(in, idx + oi) - rho_src<G>(in, idx - oi)) / h2;
-        const double dj = ((double)jxp[idx] - (double)jx[idx]) / in.dxi;
+        const double d = over_h2(rho_src<G>(in, idx + oi) - rho_src<G>(in, idx - oi));
+        const double dj = over_dxi((double)jxp[idx] - (double)jx[idx]);
         return -(((inner ? d : 0.) - dj) - (double)gp<G>(in.Ftrick[0])[idx] * in.trick);
     } else if constexpr (KIND == F_EY) {
-        const double d = (rho_src<G>(in, idx + oj) - rho_src<G>(in, idx - oj)) / h2;
-        const double dj = ((double)jyp[idx] - (double)jy[idx]) / in.dxi;
+        const double d = over_h2(rho_src<G>(in, idx + oj) - rho_src<G>(in, idx - oj));
+        const double dj = over_dxi((double)jyp[idx] - (double)jy[idx]);
         return -(((inner ? d : 0.) - dj) - (double)gp<G>(in.Ftrick[1])[idx] * in.trick);
     } else if constexpr (KIND == F_BX) {
-        const double d = (jz_src<G>(in, idx + oj) - jz_src<G>(in, idx - oj)) / h2;
-        const double dj = ((double)jyp[idx] - (double)jy[idx]) / in.dxi;
+        const double d = over_h2(jz_src<G>(in, idx + oj) - jz_src<G>(in, idx - oj));
+        const double dj = over_dxi((double)jyp[idx] - (double)jy[idx]);
         return +(((inner ? d : 0.) - dj) + (double)gp<G>(in.Ftrick[2])[idx] * in.trick);
     } else if constexpr (KIND == F_BY) {
-        const double d = (jz_src<G>(in, idx + oi) - jz_src<G>(in, idx - oi)) / h2;
-        const double dj = ((double)jxp[idx] - (double)jx[idx]) / in.dxi;
+        const double d = over_h2(jz_src<G>(in, idx + oi) - jz_src<G>(in, idx - oi));
+        const double dj = over_dxi((double)jxp[idx] - (double)jx[idx]);
         return -(((inner ? d : 0.) - dj) - (double)gp<G>(in.Ftrick[3])[idx] * in.trick);
     } else if constexpr (KIND == F_EZ) {
         // the interior only carries this right-hand side (zero elsewhere)
-        return -(((double)jx[idx + oi] - (double)jx[idx - oi]) +
-                 ((double)jy[idx + oj] - (double)jy[idx - oj])) / h2;
+        return over_h2(-(((double)jx[idx + oi] - (double)jx[idx - oi]) +
+                         ((double)jy[idx + oj] - (double)jy[idx - oj])));
     } else {  // F_BZ
         const double djx_dy = (double)jx[idx + oj] - (double)jx[idx - oj];
         const double djy_dx = (double)jy[idx + oi] - (double)jy[idx - oi];
-        return -((inner ? djx_dy : 0.) - (inner ? djy_dx : 0.)) / h2;
+        return over_h2(-((inner ? djx_dy : 0.) - (inner ? djy_dx : 0.)));
     }
 }
 
@@ -581,31 +613,16 @@ struct SolverGeom {
     int N;
     int ld;                   // row length of the spectra and of pass B's tables
     FftPlan fft;
-    const double* costab;     // cos(2 pi r / L), r in [0, L / 4]
-    const double2* stage_tw;  // per-stage twiddles of the static plan
-    const float* costab32;    // the same tables in FP32
-    int fp32;                 // transforms, spectra and tables in FP32
-    int static_L;             // L with a compile-time plan, else 0
-    int tw_lds;               // static plan: twiddles copied to LDS
-    int P, Tp;                // pairs of lines per block, threads per pair
-    const double2* wave_tw;   // wave FFT (L = 1280, 2560): W_L^t, t < L; else NULL
+    const double2* tw;        // roots of unity (solver_fft_roots)
+    int fp32;                 // transforms and spectra in FP32
 };
 
 int launch_solve(const SolverGeom& g, const SolveBatch& b, hipStream_t s,
                  Profiler* prof);
-bool solver_static_length(int L);
-bool solver_wave_length(int L);   // L has the wave FFT passes
-// LCODE_FFT_WAVE_FP32 (1): the FP32 transforms (FP32 and mixed solvers) of
-// L = 1280 run the wave FFT too (mixed six-field solve at 641^2 67.5 ->
-// 61.9 us); 0 keeps them on the radix-4/5 plan, as at L = 2560 always (there
-// the FP32 wave passes spill: the 1281^2 mixed step 871 -> 826 xi-steps/s).
-#ifndef LCODE_FFT_WAVE_FP32
-#define LCODE_FFT_WAVE_FP32 1
-#endif
-int solver_padded_len(int L);
-int solver_tw_count(int L);   // static plan: twiddle table entries
-int solver_threads_per_pair(int L, bool fp32, bool static_plan);   // threads of one line pair
-int solver_static_radix(int rem);   // static plan: radix of the next stage
+// The plan of a transform of L points; false where there is none.
+bool solver_fft_plan(int L, FftPlan* out);
+// Roots of unity of a plan's stages, in the order the kernels read them.
+std::vector<double2> solver_fft_roots(const FftPlan& p);
 int solver_lds_bytes(const SolverGeom& g);
 
 

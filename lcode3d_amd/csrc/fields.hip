@@ -17,8 +17,7 @@
 // A type-1 transform of length n is one complex FFT of length L = 2 (n + 1)
 // (sine) or 2 (n - 1) (cosine) of the odd or even extension; two real lines
 // ride in one complex FFT (real and imaginary parts).  All six fields of a
-// step share L = 2 (N - 1).  The FFT is a mixed-radix (4, 2, 3, 5) Stockham
-// transform in LDS.
+// step share L = 2 (N - 1).  The FFT keeps half of the extension (below).
 //
 // The transforms and the spectra T are in S = double (plain path) or S =
 // float (mixed-precision path); the RHS assembly, the recurrences of pass B
@@ -26,6 +25,8 @@
 
 #include "common.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace lcode {
@@ -51,29 +52,13 @@ template <typename V>
 __device__ __forceinline__ V cadd(V a, V b) { return mk<V>(a.x + b.x, a.y + b.y); }
 template <typename V>
 __device__ __forceinline__ V csub(V a, V b) { return mk<V>(a.x - b.x, a.y - b.y); }
+template <typename V>
+__device__ __forceinline__ V conj(V a) { return mk<V>(a.x, -a.y); }
+template <typename V>
+__device__ __forceinline__ V neg(V a) { return mk<V>(-a.x, -a.y); }
 // multiply by -i
 template <typename V>
 __device__ __forceinline__ V mul_mi(V a) { return mk<V>(a.y, -a.x); }
-
-// LDS layout of a pair's L complex points.  A 16-B point p sits in slot
-// p mod 16 of its 256-B group (all LDS banks once); the radix-4 stages
-// with span 1 and 4 store 16 lanes at points 4b + q and 16 (b / 4) +
-// (b mod 4) + 4 q, which hit only 4 slots.  XOR-ing the slot with
-// 5 ((p / 16) mod 4) (the group's low bits into both halves of the slot)
-// spreads both over the 16 slots, and leaves the consecutive accesses of
-// the other stages, the loads and the stores distinct (their group bits
-// are constant across 16 lanes).  Measured at 641^2 (FP64): pass B 43.2 us
-// with the XOR layout, 41.2 us with the identity layout (0, the default):
-// these conflicts are not what bounds the passes.
-#ifndef LCODE_FFT_SWIZZLE
-#define LCODE_FFT_SWIZZLE 0
-#endif
-__host__ __device__ constexpr int zi(int e) {
-    return LCODE_FFT_SWIZZLE ? (e & ~15) | ((e & 15) ^ (5 * ((e >> 4) & 3))) : e;
-}
-__host__ __device__ constexpr int padded_len(int L) {
-    return LCODE_FFT_SWIZZLE ? (L + 15) & ~15 : L;
-}
 
 // Forward DFT of R points held in registers: y_p = sum_q x_q e^{-2 pi i pq/R}.
 template <int R, typename V> struct Dft;
@@ -156,443 +141,488 @@ template <typename V> struct Dft<5, V> {
     }
 };
 
-// ---------------------------------------------------------------------------
-// Runtime plan (any L = 2^a 3^b 5^c): twiddles from a quarter-wave cosine
-// table ct[r] = cos(2 pi r / L), r in [0, L/4], held in LDS.
-// ---------------------------------------------------------------------------
-
-template <typename V>
-__device__ __forceinline__ V twiddle(const decltype(V::x)* ct, int t, int L) {
-    using S = decltype(V::x);
-    const int Q = L >> 2;
-    const int quad = t / Q, r = t - quad * Q;
-    const S c = ct[r], s = ct[Q - r];   // cos and sin of 2 pi r / L
-    S cs, sn;                           // of 2 pi t / L = quad pi / 2 + ...
-    switch (quad) {
-        case 0: cs = c; sn = s; break;
-        case 1: cs = -s; sn = c; break;
-        case 2: cs = -c; sn = -s; break;
-        default: cs = s; sn = -c; break;
-    }
-    return mk<V>(cs, -sn);
+// N1 N2 points (gcd 1) by Good-Thomas: n = (N2 n1 + N1 n2) mod R, k = (E1 k1 +
+// E2 k2) mod R with E1 = N2 (N2^-1 mod N1), E2 = N1 (N1^-1 mod N2), so that
+// W_R^(nk) = W_N1^(n1 k1) W_N2^(n2 k2): no twiddles between the two.
+constexpr int inverse_mod(int a, int n) {
+    for (int k = 1; k < n; ++k)
+        if (a * k % n == 1) return k;
+    return 0;
 }
 
-// One radix-R Stockham stage over the L points of this thread's pair.
-// Thread t of Tp handles butterflies t and t + Tp (Tp >= L / 4 makes two
-// enough for every radix >= 2).  span = product of the previous radices.
-template <int R, typename V>
-__device__ __forceinline__ void fft_stage(V* z, const decltype(V::x)* ct,
-                                          int L, int span, int t, int Tp) {
-    const int T = L / R;
-    const int tw = L / (span * R);
-    V v[2][R];
+template <int N1, int N2, typename V>
+__device__ __forceinline__ void dft_coprime(V* x) {
+    constexpr int R = N1 * N2, E1 = N2 * inverse_mod(N2 % N1, N1),
+                  E2 = N1 * inverse_mod(N1 % N2, N2);
+    V a[N2][N1];
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const int b = t + it * Tp;
-        if (b < T) {
-            const int k = b % span;
+    for (int n2 = 0; n2 < N2; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < N1; ++n1) a[n2][n1] = x[(N2 * n1 + N1 * n2) % R];
+        Dft<N1, V>::run(a[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < N1; ++k1) {
+        V b[N2];
+#pragma unroll
+        for (int n2 = 0; n2 < N2; ++n2) b[n2] = a[n2][k1];
+        Dft<N2, V>::run(b);
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2) x[(E1 * k1 + E2 * k2) % R] = b[k2];
+    }
+}
+
+template <typename V> struct Dft<6, V> {
+    static __device__ __forceinline__ void run(V* v) { dft_coprime<2, 3>(v); }
+};
+template <typename V> struct Dft<10, V> {
+    static __device__ __forceinline__ void run(V* v) { dft_coprime<2, 5>(v); }
+};
+template <typename V> struct Dft<12, V> {
+    static __device__ __forceinline__ void run(V* v) { dft_coprime<4, 3>(v); }
+};
+template <typename V> struct Dft<15, V> {
+    static __device__ __forceinline__ void run(V* v) { dft_coprime<3, 5>(v); }
+};
+template <typename V> struct Dft<20, V> {
+    static __device__ __forceinline__ void run(V* v) { dft_coprime<4, 5>(v); }
+};
+
+// M^2 points as M DFTs of stride M, the twiddles W^(n2 k1) and M DFTs across.
+template <int M, typename V, typename W>
+__device__ __forceinline__ void dft_square(V* x, W&& w) {
+    V a[M][M];
+#pragma unroll
+    for (int n2 = 0; n2 < M; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < M; ++n1) a[n2][n1] = x[M * n1 + n2];
+        Dft<M, V>::run(a[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < M; ++k1) {
+        V b[M];
+#pragma unroll
+        for (int n2 = 0; n2 < M; ++n2) b[n2] = n2 * k1 ? w(a[n2][k1], n2 * k1) : a[n2][k1];
+        Dft<M, V>::run(b);
+#pragma unroll
+        for (int k2 = 0; k2 < M; ++k2) x[k1 + M * k2] = b[k2];
+    }
+}
+
+template <typename V> struct Dft<9, V> {
+    static __device__ __forceinline__ void run(V* v) {
+        using S = decltype(V::x);
+        dft_square<3>(v, [](V a, int e) {   // W_9^e, e = 1, 2, 4
+            const S c = e == 1 ? (S)0.76604444311897803520 : e == 2 ? (S)0.17364817766693034885
+                                                                    : (S)-0.93969262078590838405;
+            const S s = e == 1 ? (S)0.64278760968653932632 : e == 2 ? (S)0.98480775301220805937
+                                                                    : (S)0.34202014332566873304;
+            return cmul(a, mk<V>(c, -s));
+        });
+    }
+};
+
+template <typename V> struct Dft<16, V> {
+    static __device__ __forceinline__ void run(V* v) {
+        using S = decltype(V::x);
+        constexpr S r = (S)0.70710678118654752440;
+        constexpr S c1 = (S)0.92387953251128675613, s1 = (S)0.38268343236508977173;
+        dft_square<4>(v, [](V a, int e) {   // W_16^e, e = 1, 2, 3, 4, 6, 9
+            switch (e) {
+                case 1: return cmul(a, mk<V>(c1, -s1));
+                case 2: return mk<V>(r * (a.x + a.y), r * (a.y - a.x));
+                case 3: return cmul(a, mk<V>(s1, -c1));
+                case 4: return mul_mi(a);
+                case 6: return mk<V>(r * (a.y - a.x), -r * (a.x + a.y));
+                default: return cmul(a, mk<V>(-c1, s1));   // 9
+            }
+        });
+    }
+};
+
+// ---------------------------------------------------------------------------
+// The FFT of an extension: x[L - p] = +x[p] (cosine) or -x[p] (sine), and so
+// X[L - k] = +-X[k].  With L = R1 T, n = l + T m and k = kappa + R1 k2,
+//   X[kappa + R1 k2] = sum_l W_T^(l k2) C_l[kappa],
+//   C_l[kappa] = W_L^(l kappa) A_l[kappa],  A_l = DFT_R1 of x[l + T m] over m,
+// and the symmetry halves the work twice: lane T - l's points are lane l's
+// mirrored, so lane l <= T / 2 writes both rows of C,
+//   C_(T-l)[kappa] = +-conj(W_L^(l kappa)) A_l[(R1 - kappa) mod R1],
+// and only the columns kappa <= R1 / 2 are transformed: the residues above hold
+// the mirror images of those below.  The first stage takes its points straight
+// from global memory (every point once: the lanes 0 .. T / 2 of
+// a row pair hold columns l + T m or L - l - T m), the K = R1 / 2 + 1 transforms of
+// length T run as Stockham stages in LDS, z[row KP + kappa] with kappa fastest
+// (KP = K made odd: the first stage's stores of consecutive rows then spread over all
+// banks), one butterfly per thread, and the last stage unfolds its outputs into
+// X[0 .. L / 2] in order, so that the passes store whole lines.  The host picks R1
+// and the radices (solver_fft_plan).
+//
+// Bound: the chain of a block (loads, three or four LDS exchanges, stores) with a few
+// wavefronts per SIMD on small grids, memory on large ones (1281^2: pass C 320 MB in
+// 67 us).  Six fields, passes A / C, us per launch, transforms of the whole extension
+// (radix 4 in LDS; 20 points per lane at 641^2 and 1281^2) -> of half of it:
+// 129^2 6.4 / 6.4 -> 6.2 / 6.2, 257^2 9.7 / 9.2 -> 8.8 / 8.2, 361^2 19.2 / 19.0 ->
+// 13.0 / 11.3, 641^2 23.8 / 21.2 -> 21.8 / 17.0, with FP32 transforms and grids 18.4 / 20.2
+// -> 15.1 / 15.0, 1281^2 96.8 / 80.3 -> 81.0 / 66.8.
+// ---------------------------------------------------------------------------
+
+// Roots held per butterfly of radix R: w^q, q = 1, 2, 3, 4, 8, 12 (below R).
+__host__ __device__ constexpr int root_count(int R) { return (R < 4 ? R : 4) - 1 + (R + 3) / 4 - 1; }
+
+// The plan of radices R1; r[0 .. nst).  A constant for the lengths with kernels of their
+// own (static_fft: powers of two and 5 times one, the usual grids), whose index
+// arithmetic then folds away.  A + C of six fields, us, the same plan from kernel
+// arguments and as a constant: 129^2 14.8 and 12.4, 257^2 19.9 and 17.1, 641^2 41.5 and 38.9.
+__host__ __device__ constexpr FftPlan make_plan(int L, int R1, int nst, const int* r) {
+    FftPlan p{};
+    p.L = L;
+    p.R1 = R1;
+    p.T = L / R1;
+    p.K = R1 / 2 + 1;
+    p.KP = p.K | 1;
+    p.lanes = p.T / 2 + 1;
+    p.nfirst = p.lanes * root_count(p.K);
+    p.nst = nst;
+    p.k_inv = (unsigned)((0x100000000ull + p.K - 1) / p.K);
+    int threads = p.lanes, span = 1;
+    for (int s = 0; s < nst; ++s) {
+        const int stride = p.T / r[s], tasks = p.K * stride;
+        p.word[s] = fft_word(r[s], span, stride);
+        if (span > 1) {
+            p.span_inv[s] = (unsigned)((0x100000000ull + span - 1) / span);
+            p.nroots += span * root_count(r[s]);
+        }
+        if (tasks > threads) threads = tasks;
+        span *= r[s];
+    }
+    p.threads = (threads + 63) / 64 * 64;
+    return p;
+}
+
+struct StaticFft {
+    int L, R1, nst, r[3];
+};
+constexpr StaticFft kStaticFft[] = {
+    {64, 4, 2, {4, 4}},    {128, 4, 2, {4, 8}},     {256, 4, 3, {4, 4, 4}},
+    {512, 4, 3, {4, 4, 8}}, {640, 4, 3, {4, 4, 10}}, {1024, 8, 2, {8, 16}},
+    {1280, 10, 2, {16, 8}}, {2048, 8, 2, {16, 16}},  {2560, 10, 2, {16, 16}},
+};
+constexpr int static_fft(int L) {   // index, or -1
+    for (int k = 0; k < (int)(sizeof(kStaticFft) / sizeof(kStaticFft[0])); ++k)
+        if (kStaticFft[k].L == L) return k;
+    return -1;
+}
+
+// n / d for n < 2^16 and 1 < d < 2^16, inv = ceil(2^32 / d).
+__device__ __forceinline__ int div_by(int n, unsigned inv) {
+    return (int)__umulhi((unsigned)n, inv);
+}
+
+// The roots w^q, q < R, of one butterfly, from the q = 1, 2, 3, 4, 8, 12 of a table
+// [root][stride] (the plan's order): the others, q = 4 a + c, are one product,
+// formed in FP64, and all are rounded once to the transform's precision.
+template <int R>
+struct Roots {
+    static constexpr int NL = R < 4 ? R : 4, NA = (R + 3) / 4;
+    double2 lo[4], hi[NA];
+    __device__ __forceinline__ void load(const double2* __restrict__ tw, int stride, int k) {
+#pragma unroll
+        for (int c = 1; c < NL; ++c) lo[c] = tw[(c - 1) * stride + k];
+#pragma unroll
+        for (int a = 1; a < NA; ++a) hi[a] = tw[(a + 2) * stride + k];
+    }
+    template <typename V>
+    __device__ __forceinline__ V at(int q) const {
+        const int a = q / 4, c = q % 4;
+        const double2 w = a == 0 ? lo[c] : c == 0 ? hi[a] : cmul(hi[a], lo[c]);
+        return mk<V>(w.x, w.y);
+    }
+};
+
+// The stages' roots, copied to LDS at the start of a block: loaded before the block's
+// inputs, stored after they are on their way.
+struct StageRoots {
+    static constexpr int kHeld = 2;
+    double2 v[kHeld];
+    __device__ __forceinline__ void load(const FftPlan& p, const double2* __restrict__ tw) {
+#pragma unroll
+        for (int u = 0; u < kHeld; ++u)
+            v[u] = tw[p.nfirst + min((int)(threadIdx.x + u * blockDim.x), p.nroots - 1)];
+    }
+    __device__ __forceinline__ void store(const FftPlan& p, const double2* __restrict__ tw,
+                                          double2* lds) const {
+#pragma unroll
+        for (int u = 0; u < kHeld; ++u) {
+            const int k = threadIdx.x + u * blockDim.x;
+            if (k < p.nroots) lds[k] = v[u];
+        }
+        for (int k = threadIdx.x + kHeld * blockDim.x; k < p.nroots; k += blockDim.x)
+            lds[k] = tw[p.nfirst + k];
+    }
+};
+
+// First stage, lane l: rows l and T - l of C from the points x.
+template <int R1, typename V>
+__device__ __forceinline__ void fft_first(V (&x)[R1], V* z, const FftPlan& p, bool sine, int l,
+                                          const Roots<R1 / 2 + 1>& w) {
+    constexpr int K = R1 / 2 + 1;
+    Dft<R1, V>::run(x);
+    V* const up = z + l * p.KP;
+    V* const down = z + (p.T - l) * p.KP;
+    const bool both = l > 0 && 2 * l < p.T;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const V a = x[k], m = x[(R1 - k) % R1];
+        if (k == 0) {
+            up[k] = a;
+            if (both) down[k] = sine ? neg(m) : m;
+        } else {
+            const V r = w.template at<V>(k);
+            up[k] = cmul(a, r);
+            const V d = cmul(m, conj(r));
+            if (both) down[k] = sine ? neg(d) : d;
+        }
+    }
+}
+
+// One Stockham stage over the K columns: thread beta takes butterfly b = beta / K of
+// column beta mod K.  Every read of the stage precedes its first write (block-wide
+// barriers: all threads call it).  The last stage writes X[k], k <= L / 2, to z[k].
+template <int R, bool FIXED, typename V>
+__device__ __forceinline__ void fft_stage(V* z, const FftPlan& p, unsigned word, unsigned span_inv,
+                                          bool last, bool sine, const double2* tw) {
+    const int span = fft_word_span(word), stride = fft_word_stride(word);
+    const int beta = threadIdx.x;
+    const bool act = beta < p.K * stride;
+    const int b = FIXED ? (int)((unsigned)beta / (unsigned)p.K) : div_by(beta, p.k_inv);
+    const int kap = beta - b * p.K;
+    const int k = span == 1 ? 0
+                  : FIXED   ? (int)((unsigned)b % (unsigned)span)
+                            : b - div_by(b, span_inv) * span;
+    V v[R];
+    if (act) {
+        if (span == 1) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) v[q] = z[(b + q * stride) * p.KP + kap];
+        } else {
+            Roots<R> w;
+            w.load(tw, span, k);
+#pragma unroll
+            for (int q = 0; q < R; ++q) v[q] = z[(b + q * stride) * p.KP + kap];
+#pragma unroll
+            for (int q = 1; q < R; ++q) v[q] = cmul(v[q], w.template at<V>(q));
+        }
+        Dft<R, V>::run(v);
+    }
+    __syncthreads();
+    if (act) {
+        if (last) {
+            const bool edge = kap == 0 || 2 * kap == p.R1;   // mirrored into itself
 #pragma unroll
             for (int q = 0; q < R; ++q) {
-                V x = z[zi(b + q * T)];
-                if (q && k) x = cmul(x, twiddle<V>(ct, q * k * tw, L));
-                v[it][q] = x;
+                const int i = kap + p.R1 * (b + q * span);
+                if (2 * i <= p.L) z[i] = v[q];
+                else if (!edge) z[p.L - i] = sine ? neg(v[q]) : v[q];
             }
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const int b = t + it * Tp;
-        if (b < T) {
-            Dft<R, V>::run(v[it]);
-            const int k = b % span;
+        } else {
             const int j = (b - k) * R + k;
 #pragma unroll
-            for (int q = 0; q < R; ++q) z[zi(j + q * span)] = v[it][q];
+            for (int q = 0; q < R; ++q) z[(j + q * span) * p.KP + kap] = v[q];
         }
     }
     __syncthreads();
 }
 
-// In-place forward FFT of every pair's buffer (block-wide barriers inside:
-// every thread of the block must call it).
 template <typename V>
-__device__ void fft_lds(V* z, const FftPlan& plan, const decltype(V::x)* ct,
-                        int t, int Tp) {
-    int span = 1;
-    for (int s = 0; s < plan.nstages; ++s) {
-        const int R = plan.radix[s];
+__device__ __forceinline__ void run_stages(V* z, const FftPlan& p, bool sine, const double2* tw) {
+    // the stages' descriptors, all read at once: a stage shifts them down
+    unsigned word[kMaxStages], inv[kMaxStages];
+#pragma unroll
+    for (int s = 0; s < kMaxStages; ++s) {
+        word[s] = p.word[s];
+        inv[s] = p.span_inv[s];
+    }
+    __syncthreads();   // the first stage's rows
+    for (int s = 0; s < p.nst; ++s) {
+        const unsigned w = word[0], v = inv[0];
+        const bool last = s == p.nst - 1;
+        const int R = fft_word_radix(w);
         switch (R) {
-            case 4: fft_stage<4>(z, ct, plan.L, span, t, Tp); break;
-            case 2: fft_stage<2>(z, ct, plan.L, span, t, Tp); break;
-            case 3: fft_stage<3>(z, ct, plan.L, span, t, Tp); break;
-            default: fft_stage<5>(z, ct, plan.L, span, t, Tp); break;
+            case 2: fft_stage<2, false>(z, p, w, v, last, sine, tw); break;
+            case 3: fft_stage<3, false>(z, p, w, v, last, sine, tw); break;
+            case 4: fft_stage<4, false>(z, p, w, v, last, sine, tw); break;
+            case 5: fft_stage<5, false>(z, p, w, v, last, sine, tw); break;
+            case 6: fft_stage<6, false>(z, p, w, v, last, sine, tw); break;
+            case 8: fft_stage<8, false>(z, p, w, v, last, sine, tw); break;
+            case 9: fft_stage<9, false>(z, p, w, v, last, sine, tw); break;
+            case 10: fft_stage<10, false>(z, p, w, v, last, sine, tw); break;
+            case 12: fft_stage<12, false>(z, p, w, v, last, sine, tw); break;
+            case 15: fft_stage<15, false>(z, p, w, v, last, sine, tw); break;
+            default: fft_stage<16, false>(z, p, w, v, last, sine, tw); break;
         }
-        span *= R;
+        if (s > 0) tw += fft_word_span(w) * root_count(R);
+#pragma unroll
+        for (int u = 0; u + 1 < kMaxStages; ++u) {
+            word[u] = word[u + 1];
+            inv[u] = inv[u + 1];
+        }
     }
 }
 
-// ---------------------------------------------------------------------------
-// Compile-time plans for the common transform lengths: the radix of each
-// stage and its span are constants, so the index arithmetic folds away.
-// A stage with span s and radix R needs the twiddles w^q, 1 <= q < R, of
-// w = exp(-2 pi i k / (s R)) for k < s: the table holds w alone, at
-// tw[tw_offset(L, s) + k] (the spans of the earlier stages summed; 341
-// entries for L = 1280 instead of L - 1 for every power), and the stage
-// forms w^2 = w w, w^3 = w^2 w, w^4 = w^2 w^2 in registers.
-// ---------------------------------------------------------------------------
-
-// Radix of the next static stage (build option LCODE_FFT_RADIX8: radix 8
-// first where it divides; measured at 641^2: pass B 44.6 us with
-// 8-8-4-5, 41.8 us with 4-4-4-4-5, so off by default).
-#ifndef LCODE_FFT_RADIX8
-#define LCODE_FFT_RADIX8 0
-#endif
-__host__ __device__ constexpr int next_radix(int rem) {
-    return (LCODE_FFT_RADIX8 && rem % 8 == 0) ? 8
-           : rem % 4 == 0 ? 4 : rem % 2 == 0 ? 2 : rem % 3 == 0 ? 3 : 5;
-}
-
-__host__ __device__ constexpr int tw_offset(int L, int span) {
-    int off = 0;
-    for (int sp = 1; sp < span && sp < L; sp *= next_radix(L / sp)) off += sp;
-    return off;
-}
-
-__host__ __device__ constexpr int tw_count(int L) { return tw_offset(L, L); }
-
-// Threads of one line pair: enough for the L / 4 butterflies of a radix-4
-// stage (the runtime plans need it: two butterflies per thread at most).
-__host__ __device__ constexpr int threads_per_pair(int L) {
-    return ((L + 3) / 4 + 63) / 64 * 64;
-}
-
-// LCODE_FFT_PAIR_WAVES_F32 / _F64 (0: threads_per_pair): waves per line
-// pair of the static plans; each thread then takes up to two butterflies of
-// a stage.  Kept at or above four input points per thread and three
-// twiddle-table entries per thread.  Fewer waves per pair let more pairs
-// share a CU's 32 wave slots (at 641^2, 5 waves per pair leave 966 blocks
-// for 768 slots); measured at 641^2, six-field solve: FP64 92.6 us with
-// 5 waves, 84.2 with 4; FP32 83.6 with 5, 72.0 with 4, 70.9 with 3 (two
-// pairs per block); with one pair per block FP64 76.8 / 71.9 / 77.7 us with
-// 5 / 4 / 3 waves, FP32 60.6 / 59.3 us with 4 / 3.
-#ifndef LCODE_FFT_PAIR_WAVES_F32
-#define LCODE_FFT_PAIR_WAVES_F32 3
-#endif
-#ifndef LCODE_FFT_PAIR_WAVES_F64
-#define LCODE_FFT_PAIR_WAVES_F64 4
-#endif
-__host__ __device__ constexpr int static_threads_per_pair(int L, bool fp32) {
-    const int d = threads_per_pair(L);
-    const int w = fp32 ? LCODE_FFT_PAIR_WAVES_F32 : LCODE_FFT_PAIR_WAVES_F64;
-    if (w <= 0) return d;
-    const int lo = ((L / 2 + 1 + 3) / 4 + 63) / 64 * 64;   // <= 4 input points
-    int t = 64 * w;
-    if (t < lo) t = lo;
-    if (t > d) t = d;
-    if (2 * t < (L + 3) / 4 || 3 * t < tw_count(L)) t = d;
-    return t;
-}
-
-// Input points per thread of a pair: a transform input has at most
-// L / 2 + 1 points.
-__host__ __device__ constexpr int points_per_thread(int L, bool fp32) {
-    return (L / 2 + 1 + static_threads_per_pair(L, fp32) - 1) /
-           static_threads_per_pair(L, fp32);
-}
-
-template <int L, int SPAN, typename V>
-__device__ __forceinline__ void fft_static(V* z, const double2* __restrict__ tw,
-                                           int t) {
-    if constexpr (SPAN < L) {
-        constexpr int R = next_radix(L / SPAN);
-        constexpr int T = L / R;
-        constexpr int Tp = static_threads_per_pair(L, sizeof(V) == sizeof(float2));
-        constexpr int ITER = (T + Tp - 1) / Tp;
-        constexpr int OFF = tw_offset(L, SPAN);
-        V v[ITER][R];
-#pragma unroll
-        for (int it = 0; it < ITER; ++it) {
-            const int b = t + it * Tp;
-            if (b < T) {
-                const int k = b % SPAN;
-                // the root in FP64 and its powers formed in FP64, each
-                // rounded once to the transform's precision
-                double2 w[R];
-                if constexpr (SPAN > 1) {
-                    w[1] = tw[OFF + k];
-                    if constexpr (R > 2) w[2] = cmul(w[1], w[1]);
-                    if constexpr (R > 3) w[3] = cmul(w[2], w[1]);
-                    if constexpr (R > 4) w[4] = cmul(w[2], w[2]);
-                    if constexpr (R > 5) w[5] = cmul(w[4], w[1]);
-                    if constexpr (R > 6) w[6] = cmul(w[4], w[2]);
-                    if constexpr (R > 7) w[7] = cmul(w[4], w[3]);
-                }
-#pragma unroll
-                for (int q = 0; q < R; ++q) {
-                    V x = z[zi(b + q * T)];
-                    if (SPAN > 1 && q) x = cmul(x, mk<V>(w[q].x, w[q].y));
-                    v[it][q] = x;
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < ITER; ++it) {
-            const int b = t + it * Tp;
-            if (b < T) {
-                Dft<R, V>::run(v[it]);
-                const int k = b % SPAN;
-                const int j = (b - k) * R + k;
-#pragma unroll
-                for (int q = 0; q < R; ++q) z[zi(j + q * SPAN)] = v[it][q];
-            }
-        }
-        __syncthreads();
-        fft_static<L, SPAN * R>(z, tw, t);
+template <int L, int STAGE, typename V>
+__device__ __forceinline__ void static_stages(V* z, bool sine, const double2* tw) {
+    constexpr StaticFft f = kStaticFft[static_fft(L)];
+    constexpr FftPlan p = make_plan(L, f.R1, f.nst, f.r);
+    if constexpr (STAGE < f.nst) {
+        constexpr int R = f.r[STAGE], span = fft_word_span(p.word[STAGE]);
+        fft_stage<R, true>(z, p, p.word[STAGE], 0, STAGE == f.nst - 1, sine, tw);
+        static_stages<L, STAGE + 1>(z, sine, tw + (STAGE > 0 ? span * root_count(R) : 0));
     }
 }
 
-// Twiddle source of a block: for L == 0 (runtime plan) the quarter-wave
-// cosine table, copied to LDS; for a static L the stage twiddle roots (FP64
-// in both precisions), copied to LDS when TW_LDS, else read from global
-// memory.
-template <typename S>
-struct Tw {
-    const S* ct;
-    const double2* tw;
-};
-
-template <typename S> struct TwSrc;
-template <> struct TwSrc<double> {
-    static __device__ const double* ct(const SolverGeom& g) { return g.costab; }
-};
-template <> struct TwSrc<float> {
-    static __device__ const float* ct(const SolverGeom& g) { return g.costab32; }
-};
-
-template <int L, bool TW_LDS, typename S>
-__device__ __forceinline__ Tw<S> load_twiddles(typename Vec<S>::T* lds,
-                                               const SolverGeom& g) {
-    Tw<S> r{nullptr, nullptr};
-    if constexpr (L == 0) {
-        S* ct = reinterpret_cast<S*>(lds + (size_t)g.P * padded_len(g.fft.L));
-        const S* src = TwSrc<S>::ct(g);
-        for (int k = threadIdx.x; k <= (g.fft.L >> 2); k += blockDim.x) ct[k] = src[k];
-        r.ct = ct;
-    } else if constexpr (TW_LDS) {
-        // at most three entries per thread (static_threads_per_pair keeps
-        // P * Tp >= tw_count / 3), all loaded before the LDS stores
-        constexpr int n = tw_count(L);
-        static_assert(n <= 3 * static_threads_per_pair(L, std::is_same<S, float>::value),
-                      "twiddle table larger than three per thread");
-        // (the data end is 16-byte aligned: an even number of points)
-        double2* d = reinterpret_cast<double2*>(lds + (size_t)g.P * padded_len(L));
-        const double2* src = g.stage_tw;
-        const int nt = blockDim.x;
-        double2 v[3];
-#pragma unroll
-        for (int u = 0; u < 3; ++u) v[u] = src[min((int)threadIdx.x + u * nt, n - 1)];
-#pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            const int k = threadIdx.x + u * nt;
-            if (k < n) d[k] = v[u];
-        }
-        r.tw = d;
+template <int L, typename V>
+__device__ __forceinline__ void fft_stages(V* z, const FftPlan& p, bool sine, const double2* tw) {
+    if constexpr (L != 0) {
+        __syncthreads();   // the first stage's rows
+        static_stages<L, 0>(z, sine, tw);
     } else {
-        r.tw = g.stage_tw;
+        run_stages(z, p, sine, tw);
     }
-    return r;
 }
 
-template <int L, typename S>
-__device__ __forceinline__ void fft_any(typename Vec<S>::T* z,
-                                        const SolverGeom& g, const Tw<S>& tw,
-                                        int t) {
-    if constexpr (L == 0) {
-        fft_lds(z, g.fft, tw.ct, t, g.Tp);
+// The block's plan: the constant of L, or (0) the geometry's.
+template <int L>
+__device__ __forceinline__ FftPlan plan_of(const SolverGeom& g) {
+    if constexpr (L != 0) {
+        constexpr StaticFft f = kStaticFft[static_fft(L)];
+        return make_plan(L, f.R1, f.nst, f.r);
     } else {
-        fft_static<L, 1>(z, tw.tw, t);
+        return g.fft;
     }
 }
 
-// Extension writers/readers.  Cosine (DCT-I, n points): z[k] and z[L-k]
-// hold input k.  Sine (DST-I, n points): z[k+1] = input k, z[L-1-k] =
-// -input k, z[0] = z[n+1] = 0.  For a pair (a real, b imaginary) the FFT
-// gives DCT(a) = Re Z[k], DCT(b) = Im Z[k]; DST(a) = -Im Z[k+1],
-// DST(b) = Re Z[k+1].
+// Outputs of the pair's two lines at column j of the grid, 0 <= j <= L / 2:
+// cosine Re and Im of X[j], sine -Im and Re.
 template <typename V>
-__device__ __forceinline__ void put_ext(V* z, int xf, int n, int len, int L,
-                                        double a, double b) {
-    using S = decltype(V::x);
-    const V v = mk<V>((S)a, (S)b);
-    if (xf == XF_DCT) {
-        z[zi(n)] = v;
-        if (n >= 1 && n <= len - 2) z[zi(L - n)] = v;
-    } else {
-        z[zi(n + 1)] = v;
-        z[zi(L - 1 - n)] = mk<V>(-v.x, -v.y);
+__device__ __forceinline__ void get_pair(const V* z, bool sine, int j, double& a, double& c) {
+    const V v = z[j];
+    a = sine ? -(double)v.y : (double)v.x;
+    c = sine ? (double)v.x : (double)v.y;
+}
+
+// Grid column of point l + T m: itself up to L / 2, its mirror image above.
+template <int R1>
+__device__ __forceinline__ int point_column(const FftPlan& p, int l, int m) {
+    const int n = l + p.T * m;
+    return 2 * m < R1 ? n : p.L - n;
+}
+
+// The extension's points l + T m of a lane from the values v(m, column) of the two
+// lines (sine: odd, 0 at both ends).
+template <int R1, typename V, typename F>
+__device__ __forceinline__ void extend(V (&x)[R1], const FftPlan& p, bool sine, int l, F&& v) {
+#pragma unroll
+    for (int m = 0; m < R1; ++m) {
+        x[m] = v(m, point_column<R1>(p, l, m));
+        if (sine && 2 * m >= R1) x[m] = neg(x[m]);
+        if ((m == 0 || 2 * m == R1) && sine && l == 0) x[m] = mk<V>(0, 0);
     }
 }
 
-template <typename V>
-__device__ __forceinline__ void put_ext_zeros(V* z, int xf, int len, int t) {
-    if (xf == XF_DST && t == 0) {
-        z[zi(0)] = mk<V>(0, 0);
-        z[zi(len + 1)] = mk<V>(0, 0);
-    }
-}
-
-template <typename V>
-__device__ __forceinline__ void get_ext(const V* z, int xf, int k, double& a,
-                                        double& b) {
-    if (xf == XF_DCT) {
-        const V v = z[zi(k)];
-        a = v.x;
-        b = v.y;
-    } else {
-        const V v = z[zi(k + 1)];
-        a = -v.y;
-        b = v.x;
-    }
-}
-
+// Right-hand sides of rows i and i + 1 (clamped to the grid: a row outside it, or
+// without data, is dropped by the caller) at column j; the values of rhs_value_k.  Row bases are uniform, the lane adds a 32-bit byte offset, and a
+// derivative along i takes the sources of its four rows once.
 template <typename G>
-__device__ __forceinline__ double rhs_value(int kind, int i, int j, int N,
-                                            const RhsInputs& in) {
-    return rhs_value_dev<G>(kind, i, j, N, in);
+__device__ __forceinline__ double at_byte(const G* row, unsigned off) {
+    return (double)*reinterpret_cast<const G*>(reinterpret_cast<const char*>(row) + off);
 }
 
-// LCODE_RHS_BATCH (build option, the FP64 wave pass A only; the other pass
-// A kernels keep 0, which their register budgets need): 0, each
-// right-hand-side value loads and combines its inputs in one expression, and
-// the compiler streams the loads (about a dozen in flight per wave); B > 0,
-// the inputs of B columns of both rows are loaded (rhs_load_k) before any is
-// combined (rhs_combine_k, the same arithmetic as rhs_value_k), so that up
-// to 18 B loads are in flight.
-#ifndef LCODE_RHS_BATCH
-#define LCODE_RHS_BATCH 0
-#endif
-
-// The loads of rhs_value_k<KIND>(i, j): r[0..2] and r[3..5] the source
-// (density or jz, its previous-pass value, beam) at the forward and backward
-// neighbour, r[6..8] the previous-slice current, the current and the trick
-// field at the point (Ex, Ey, Bx, By); r[0..3] the four current neighbours
-// (Ez, Bz).
 template <int KIND, typename G>
-__device__ __forceinline__ void rhs_load_k(int i, int j, int N, const RhsInputs& in,
-                                           double* r) {
-    const size_t idx = (size_t)i * N + j;
-    const bool inner = i >= 1 && i <= N - 2 && j >= 1 && j <= N - 2;
-    const size_t oi = inner ? (size_t)N : 0, oj = inner ? 1 : 0;
+__device__ __forceinline__ void rhs_pair_k(int i, int j, int N, const RhsInputs& in, double& a,
+                                           double& c) {
+    const int i1 = min(i + 1, N - 1);
+    const int rows[4] = {max(i - 1, 0), i, i1, min(i1 + 1, N - 1)};
+    const bool in0 = i >= 1 && i <= N - 2, in1 = i1 >= 1 && i1 <= N - 2;
+    auto over_h2 = [&](double x) { return quotient(x, in.h * 2, in.inv_h2); };
+    auto over_dxi = [&](double x) { return quotient(x, in.dxi, in.inv_dxi); };
     const G *jx = gp<G>(in.jx), *jy = gp<G>(in.jy);
+    auto row = [&](const auto* base, int r) { return base + (size_t)r * N; };
+    const bool jin = j >= 1 && j <= N - 2;
+    const int oj = jin ? 1 : 0;
+    const unsigned o = (unsigned)j * sizeof(G), op = (unsigned)(j + oj) * sizeof(G),
+                   om = (unsigned)(j - oj) * sizeof(G);
     if constexpr (KIND == F_EZ) {
-        r[0] = (double)jx[idx + oi];
-        r[1] = (double)jx[idx - oi];
-        r[2] = (double)jy[idx + oj];
-        r[3] = (double)jy[idx - oj];
+        // the interior only carries this right-hand side (zero elsewhere)
+        const double x0 = at_byte(row(jx, rows[0]), o), x1 = at_byte(row(jx, rows[1]), o),
+                     x2 = at_byte(row(jx, rows[2]), o), x3 = at_byte(row(jx, rows[3]), o);
+        const double ya = at_byte(row(jy, i), op) - at_byte(row(jy, i), om);
+        const double yc = at_byte(row(jy, i1), op) - at_byte(row(jy, i1), om);
+        a = over_h2(-((x2 - x0) + ya));
+        c = over_h2(-((x3 - x1) + yc));
     } else if constexpr (KIND == F_BZ) {
-        r[0] = (double)jx[idx + oj];
-        r[1] = (double)jx[idx - oj];
-        r[2] = (double)jy[idx + oi];
-        r[3] = (double)jy[idx - oi];
+        const double x0 = at_byte(row(jy, rows[0]), o), x1 = at_byte(row(jy, rows[1]), o),
+                     x2 = at_byte(row(jy, rows[2]), o), x3 = at_byte(row(jy, rows[3]), o);
+        const double ya = at_byte(row(jx, i), op) - at_byte(row(jx, i), om);
+        const double yc = at_byte(row(jx, i1), op) - at_byte(row(jx, i1), om);
+        const bool n0 = in0 && jin, n1 = in1 && jin;
+        a = over_h2(-((n0 ? ya : 0.) - (n0 ? x2 - x0 : 0.)));
+        c = over_h2(-((n1 ? yc : 0.) - (n1 ? x3 - x1 : 0.)));
     } else {
         constexpr bool rho = KIND == F_EX || KIND == F_EY;
         constexpr bool along_i = KIND == F_EX || KIND == F_BY;
-        const size_t o = along_i ? oi : oj;
+        constexpr bool xcur = along_i;
+        constexpr int ft = KIND == F_EX ? 0 : KIND == F_EY ? 1 : KIND == F_BX ? 2 : 3;
         const G* src = gp<G>(rho ? in.ro : in.jz);
         const double* sp0 = rho ? in.ro_prev : in.jz_prev;
         const G* prev = sp0 ? gp<G>(sp0) : src;
         const double* dummy = std::is_same<G, double>::value ? in.ro : in.zero64;
-        const double* b = in.beam ? in.beam : dummy;
-        r[0] = (double)src[idx + o];
-        r[1] = (double)prev[idx + o];
-        r[2] = b[idx + o];
-        r[3] = (double)src[idx - o];
-        r[4] = (double)prev[idx - o];
-        r[5] = b[idx - o];
-        constexpr bool xcur = KIND == F_EX || KIND == F_BY;
+        const double* beam = in.beam ? in.beam : dummy;
+        const double on = in.beam ? 1. : 0., off = in.beam ? 0. : in.beam_scalar;
+        // (a beam is added to the source of every derivative: lcode.py:862-863)
+        auto source = [&](int r, unsigned ob, int jj) {
+            const double s = (at_byte(row(src, r), ob) + at_byte(row(prev, r), ob)) / 2;
+            return s + (at_byte(row(beam, r), (unsigned)jj * 8u) * on + off);
+        };
+        double da, dc;
+        if constexpr (along_i) {
+            const double s0 = source(rows[0], o, j), s1 = source(rows[1], o, j);
+            const double s2 = source(rows[2], o, j), s3 = source(rows[3], o, j);
+            da = s2 - s0;
+            dc = s3 - s1;
+        } else {
+            da = source(i, op, j + oj) - source(i, om, j - oj);
+            dc = source(i1, op, j + oj) - source(i1, om, j - oj);
+        }
         const G* jp = gp<G>(xcur ? in.jx_prev : in.jy_prev);
         const G* jc = xcur ? jx : jy;
-        constexpr int ft = KIND == F_EX ? 0 : KIND == F_EY ? 1 : KIND == F_BX ? 2 : 3;
-        r[6] = (double)jp[idx];
-        r[7] = (double)jc[idx];
-        r[8] = (double)gp<G>(in.Ftrick[ft])[idx];
-    }
-}
-
-// rhs_value_k<KIND>(i, j) from the values rhs_load_k loaded.
-template <int KIND>
-__device__ __forceinline__ double rhs_combine_k(int i, int j, int N, const RhsInputs& in,
-                                                const double* r) {
-    const bool inner = i >= 1 && i <= N - 2 && j >= 1 && j <= N - 2;
-    const double h2 = in.h * 2;
-    if constexpr (KIND == F_EZ) {
-        return -((r[0] - r[1]) + (r[2] - r[3])) / h2;
-    } else if constexpr (KIND == F_BZ) {
-        const double djx_dy = r[0] - r[1];
-        const double djy_dx = r[2] - r[3];
-        return -((inner ? djx_dy : 0.) - (inner ? djy_dx : 0.)) / h2;
-    } else {
-        auto source = [&](double v, double p, double b) {
-            const double s = (v + p) / 2;
-            return s + (b * (in.beam ? 1. : 0.) + (in.beam ? 0. : in.beam_scalar));
-        };
-        const double d = (source(r[0], r[1], r[2]) - source(r[3], r[4], r[5])) / h2;
-        const double dj = (r[6] - r[7]) / in.dxi;
-        if constexpr (KIND == F_BX) return +(((inner ? d : 0.) - dj) + r[8] * in.trick);
-        else return -(((inner ? d : 0.) - dj) - r[8] * in.trick);
-    }
-}
-
-// Right-hand sides of rows ia and ib at columns j0 + t + u Tp, u < K, as
-// straight-line code: columns clamped to [j0, j0 + len), so all loads of
-// the thread are issued before their values are used.
-template <int KIND, int K, typename G, int B>
-__device__ __forceinline__ void rhs_rows_k(int ia, int ib, int j0, int len,
-                                           int t, int Tp, int N,
-                                           const RhsInputs& in, double* a,
-                                           double* c) {
-    if constexpr (B > 0) {
-#pragma unroll
-        for (int u0 = 0; u0 < K; u0 += B) {
-            double ra[B][9], rc[B][9];
-#pragma unroll
-            for (int u = u0; u < u0 + B && u < K; ++u) {
-                const int j = j0 + min(t + u * Tp, len - 1);
-                rhs_load_k<KIND, G>(ia, j, N, in, ra[u - u0]);
-                rhs_load_k<KIND, G>(ib, j, N, in, rc[u - u0]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = u0; u < u0 + B && u < K; ++u) {
-                const int j = j0 + min(t + u * Tp, len - 1);
-                a[u] = rhs_combine_k<KIND>(ia, j, N, in, ra[u - u0]);
-                c[u] = rhs_combine_k<KIND>(ib, j, N, in, rc[u - u0]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const int j = j0 + min(t + u * Tp, len - 1);
-            a[u] = rhs_value_k<KIND, G>(ia, j, N, in);
-            c[u] = rhs_value_k<KIND, G>(ib, j, N, in);
+        const G* tr = gp<G>(in.Ftrick[ft]);
+        const double ja = over_dxi(at_byte(row(jp, i), o) - at_byte(row(jc, i), o));
+        const double jc1 = over_dxi(at_byte(row(jp, i1), o) - at_byte(row(jc, i1), o));
+        const double ta = at_byte(row(tr, i), o) * in.trick;
+        const double tc = at_byte(row(tr, i1), o) * in.trick;
+        const double fa = (in0 && jin ? over_h2(da) : 0.) - ja;
+        const double fc = (in1 && jin ? over_h2(dc) : 0.) - jc1;
+        if constexpr (KIND == F_BX) {
+            a = fa + ta;
+            c = fc + tc;
+        } else {
+            a = -(fa - ta);
+            c = -(fc - tc);
         }
     }
 }
 
-template <int K, typename G, int B = 0>
-__device__ __forceinline__ void rhs_rows(int kind, int ia, int ib, int j0,
-                                         int len, int t, int Tp, int N,
-                                         const RhsInputs& in, double* a,
-                                         double* c) {
+template <typename G>
+__device__ __forceinline__ void rhs_pair(int kind, int i, int j, int N, const RhsInputs& in,
+                                         double& a, double& c) {
     switch (kind) {
-        case F_EX: rhs_rows_k<F_EX, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
-        case F_EY: rhs_rows_k<F_EY, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
-        case F_BX: rhs_rows_k<F_BX, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
-        case F_BY: rhs_rows_k<F_BY, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
-        case F_EZ: rhs_rows_k<F_EZ, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
-        default: rhs_rows_k<F_BZ, K, G, B>(ia, ib, j0, len, t, Tp, N, in, a, c); break;
+        case F_EX: rhs_pair_k<F_EX, G>(i, j, N, in, a, c); break;
+        case F_EY: rhs_pair_k<F_EY, G>(i, j, N, in, a, c); break;
+        case F_BX: rhs_pair_k<F_BX, G>(i, j, N, in, a, c); break;
+        case F_BY: rhs_pair_k<F_BY, G>(i, j, N, in, a, c); break;
+        case F_EZ: rhs_pair_k<F_EZ, G>(i, j, N, in, a, c); break;
+        default: rhs_pair_k<F_BZ, G>(i, j, N, in, a, c); break;
     }
 }
 
@@ -602,10 +632,22 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// Sum over the block, to every thread (scratch: one double per wave).
+__device__ __forceinline__ double block_sum(double v, double* scratch) {
+    v = wave_sum(v);
+    if (blockDim.x == 64) return v;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += scratch[w];
+    return t;
+}
+
 // XCD-aware block order.  Workgroups go to the 8 XCDs round-robin by
-// linear id and each XCD has its own L2; neighbouring line blocks touch the
-// same 128-B lines of the transposed spectra, so give every XCD a
-// contiguous range of (field, line block) pairs.  A bijection on the grid.
+// linear id and each XCD has its own L2; neighbouring row pairs share the
+// 128-B lines of their sources, so give every XCD a
+// contiguous range of (field, row pair)s.  A bijection on the grid.
 struct BlockPos {
     int field, block;
 };
@@ -616,14 +658,10 @@ __device__ __forceinline__ BlockPos xcd_block() {
     return BlockPos{logical / gx, logical % gx};
 }
 
-// Pass A's order: the fields of one line block get consecutive logical
+// Pass A's order: the fields of one row pair get consecutive logical
 // ids, so one XCD assembles all six right-hand sides of its rows and reads
 // their shared sources (densities, currents, beam) into its L2 once.
-#ifndef LCODE_PASS_A_FIELDS_INTERLEAVED
-#define LCODE_PASS_A_FIELDS_INTERLEAVED 1
-#endif
 __device__ __forceinline__ BlockPos xcd_block_rows() {
-    if (!LCODE_PASS_A_FIELDS_INTERLEAVED) return xcd_block();
     const int gx = gridDim.x, nf = gridDim.y, total = gx * nf;
     const int logical = xcd_logical(blockIdx.y * gx + blockIdx.x, total);
     return BlockPos{logical % nf, logical / nf};
@@ -633,71 +671,70 @@ __device__ __forceinline__ BlockPos xcd_block_rows() {
 // Passes
 // ---------------------------------------------------------------------------
 
-// LCODE_PASS_A_WAVES, LCODE_PASS_C_WAVES (0: the compiler's choice): waves
-// per SIMD the register allocation of passes A and C must allow.
-#ifndef LCODE_PASS_A_WAVES
-#define LCODE_PASS_A_WAVES 0
-#endif
-#ifndef LCODE_PASS_C_WAVES
-#define LCODE_PASS_C_WAVES 0
-#endif
-#if LCODE_PASS_A_WAVES > 0
-#define LCODE_PASS_A_ATTR __attribute__((amdgpu_waves_per_eu(LCODE_PASS_A_WAVES)))
-#else
-#define LCODE_PASS_A_ATTR
-#endif
-#if LCODE_PASS_C_WAVES > 0
-#define LCODE_PASS_C_ATTR __attribute__((amdgpu_waves_per_eu(LCODE_PASS_C_WAVES)))
-#else
-#define LCODE_PASS_C_ATTR
-#endif
+// Reads the first word of each 64-byte line of a kernel argument, so that the lines come
+// in together and not one by one where their members are first used (pass A 10.8 -> 10.1 us
+// at 257^2, 8.1 -> 7.4 at 129^2).
+template <typename T>
+__device__ __forceinline__ void fetch_lines(const T& v) {
+    const unsigned* w = reinterpret_cast<const unsigned*>(&v);
+    constexpr int n = (sizeof(T) + 63) / 64;
+    unsigned t[n + 1];
+#pragma unroll
+    for (int k = 0; k < n; ++k) t[k] = w[16 * k];
+    t[n] = w[sizeof(T) / 4 - 1];
+#pragma unroll
+    for (int k = 0; k <= n; ++k) asm volatile("" ::"s"(t[k]));
+}
 
+// Pass A: a block takes one field's grid rows ga (even) and ga + 1.  All its threads
+// assemble right-hand sides, a column of both rows at a time (at 641^2 21.8 us; two and three
+// columns in flight 24.4 and 23.9: more registers; the first stage's lanes alone, at their own points,
+// 30.3), and the first stage reads them back from LDS.
 // G: storage type of the source grids (FP64 arithmetic in both).
-template <int L_, bool TW_LDS, typename S, typename G>
-__global__ void __launch_bounds__(1024) LCODE_PASS_A_ATTR
+template <int R1, int L_, typename S, typename G>
+__global__ void __launch_bounds__(512)
 pass_a_kernel(SolverGeom g, SolveBatch b) {
     using V = typename Vec<S>::T;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    V* lds = reinterpret_cast<V*>(lds_raw);
     if (!gate_open(b.gate)) return;
     const BlockPos bp = xcd_block_rows();
     const FieldPlan& fp = b.f[bp.field];
-    const int Tp = g.Tp, L = g.fft.L, N = g.N;
-    const int lines = fp.rowsA;
-    if (bp.block * g.P * 2 >= lines) return;
-    const int pair = threadIdx.x / Tp, t = threadIdx.x - pair * Tp;
-    V* z = lds + (size_t)pair * padded_len(L);
-    const Tw<S> tw = load_twiddles<L_, TW_LDS, S>(lds, g);
-    const int ra = (bp.block * g.P + pair) * 2, rb = ra + 1;
-    const bool va = ra < lines, vb = rb < lines;
-    if constexpr (L_ != 0) {
-        // rows without data read row rowsA0 (in bounds) and are dropped
-        constexpr int kPer = points_per_thread(L_, std::is_same<S, float>::value);
-        double a[kPer], c[kPer];
-        rhs_rows<kPer, G>(fp.kind, fp.rowsA0 + (va ? ra : 0), fp.rowsA0 + (vb ? rb : 0),
-                       fp.colA0, fp.lenA, t, Tp, N, b.in, a, c);
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = t + u * Tp;
-            if (n < fp.lenA) put_ext(z, fp.xfA, n, fp.lenA, L, va ? a[u] : 0., vb ? c[u] : 0.);
-        }
-    } else {
-        for (int n = t; n < fp.lenA; n += Tp) {
-            const int j = fp.colA0 + n;
-            const double a = va ? rhs_value<G>(fp.kind, fp.rowsA0 + ra, j, N, b.in) : 0.;
-            const double c = vb ? rhs_value<G>(fp.kind, fp.rowsA0 + rb, j, N, b.in) : 0.;
-            put_ext(z, fp.xfA, n, fp.lenA, L, a, c);
-        }
-    }
-    put_ext_zeros(z, fp.xfA, fp.lenA, t);
-    __syncthreads();
-    fft_any<L_, S>(z, g, tw, t);
-    S* T = static_cast<S*>(fp.T);
-    for (int k = t; k < fp.lenA; k += Tp) {
+    const FftPlan p = plan_of<L_>(g);
+    double2* const tw = reinterpret_cast<double2*>(lds_raw);
+    V* const z = reinterpret_cast<V*>(tw + p.nroots);
+    const int N = g.N, ga = bp.block * 2, gb = ga + 1;
+    auto has = [&](int r) { return r >= fp.rowsA0 && r < fp.rowsA0 + fp.rowsA; };
+    fetch_lines(g);
+    fetch_lines(fp);
+    fetch_lines(b.in);
+    const bool va = has(ga), vb = has(gb);
+    if (!va && !vb) return;
+    const bool sine = fp.xfA == XF_DST;
+    StageRoots sr;
+    sr.load(p, g.tw);
+    const int l = threadIdx.x, nt = L_ ? p.threads : (int)blockDim.x;
+    Roots<R1 / 2 + 1> w;
+    w.load(g.tw, p.lanes, min(l, p.lanes - 1));
+    for (int j = l; j < N; j += nt) {
         double a, c;
-        get_ext(z, fp.xfA, k, a, c);
-        if (va) T[(size_t)(fp.rowsA0 + ra) * g.ld + k] = (S)a;
-        if (vb) T[(size_t)(fp.rowsA0 + rb) * g.ld + k] = (S)c;
+        rhs_pair<G>(fp.kind, ga, j, N, b.in, a, c);
+        z[j] = mk<V>(va ? (S)a : (S)0, vb ? (S)c : (S)0);
+    }
+    sr.store(p, g.tw, tw);
+    __syncthreads();
+    V x[R1];
+    if (l < p.lanes) extend<R1>(x, p, sine, l, [&](int, int j) { return z[j]; });
+    __syncthreads();
+    if (l < p.lanes) fft_first<R1>(x, z, p, sine, l, w);
+    fft_stages<L_>(z, p, sine, tw);
+    S* const Ta = static_cast<S*>(fp.T) + (size_t)ga * g.ld;
+    S* const Tb = Ta + g.ld;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < fp.lenA; k += blockDim.x) {
+        double a, c;
+        get_pair(z, sine, fp.colA0 + k, a, c);
+        if (va) Ta[k] = (S)a;
+        if (vb) Tb[k] = (S)c;
     }
 }
 
@@ -889,173 +926,129 @@ pass_b_kernel(SolverGeom g, SolveBatch b) {
     }
 }
 
+// Pass C: a block takes one field's rows ra (even) and ra + 1.  The first stage's lanes
+// load their points directly.  (Prev and guess values loaded ahead of the FFT
+// cost a wave per SIMD: 641^2 18.8 -> 24.7 us.)
 // G: storage type of the fields, averages and guess (FP64 epilogue
 // arithmetic in both).
-template <int L_, bool TW_LDS, typename S, typename G>
-__global__ void __launch_bounds__(1024) LCODE_PASS_C_ATTR
+template <int R1, int L_, typename S, typename G>
+__global__ void __launch_bounds__(512)
 pass_c_kernel(SolverGeom g, SolveBatch b) {
     using V = typename Vec<S>::T;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    V* lds = reinterpret_cast<V*>(lds_raw);
-    __shared__ double red[16];
+    __shared__ double red[8];
     if (!gate_open(b.gate)) return;
     const BlockPos bp = xcd_block();
     const FieldPlan& fp = b.f[bp.field];
-    const int Tp = g.Tp, L = g.fft.L, N = g.N;
-    if (bp.block * g.P * 2 >= N) {
-        if (b.resid && threadIdx.x == 0) {    // no rows: a zero partial
-            const int lin = blockIdx.y * gridDim.x + blockIdx.x;
-            b.resid_part[2 * lin] = b.resid_part[2 * lin + 1] = 0.;
-        }
-        return;
-    }
-    const int pair = threadIdx.x / Tp, t = threadIdx.x - pair * Tp;
-    V* z = lds + (size_t)pair * padded_len(L);
-    const Tw<S> tw = load_twiddles<L_, TW_LDS, S>(lds, g);
-    const int ra = (bp.block * g.P + pair) * 2, rb = ra + 1;
-    const int ca = ra - fp.rowsA0, cb = rb - fp.rowsA0;
-    const bool ha = ra < N && ca >= 0 && ca < fp.rowsA;
-    const bool hb = rb < N && cb >= 0 && cb < fp.rowsA;
-    // (rows without data read a valid row, and are dropped)
-    const S* Ta = static_cast<const S*>(fp.T) + (size_t)(ha ? ra : fp.rowsA0) * g.ld;
-    const S* Tb = static_cast<const S*>(fp.T) + (size_t)(hb ? rb : fp.rowsA0) * g.ld;
-    if constexpr (L_ != 0) {
-        // every load of the thread first (columns clamped in bounds, unused
-        // values dropped), then the LDS stores
-        constexpr int kPer = points_per_thread(L_, std::is_same<S, float>::value);
-        S xa[kPer], xb[kPer];
+    const FftPlan p = plan_of<L_>(g);
+    double2* const tw = reinterpret_cast<double2*>(lds_raw);
+    V* const z = reinterpret_cast<V*>(tw + p.nroots);
+    const int N = g.N, ra = bp.block * 2, rb = ra + 1;
+    auto has = [&](int r) { return r >= fp.rowsA0 && r < fp.rowsA0 + fp.rowsA; };
+    fetch_lines(g);
+    fetch_lines(fp);
+    const bool ha = has(ra), hb = has(rb);
+    const bool sine = fp.xfA == XF_DST;
+    const int l = threadIdx.x;
+    StageRoots sr;
+    sr.load(p, g.tw);
+    if (l < p.lanes) {
+        // (rows without data read a valid row, and are dropped; so is what the
+        // ends of a sine line read)
+        const S* Ta = static_cast<const S*>(fp.T) + (size_t)(ha ? ra : fp.rowsA0) * g.ld;
+        const S* Tb = static_cast<const S*>(fp.T) + (size_t)(hb ? rb : fp.rowsA0) * g.ld;
+        S a[R1], c[R1];
 #pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = min(t + u * Tp, fp.lenA - 1);
-            xa[u] = Ta[n];
-            xb[u] = Tb[n];
+        for (int m = 0; m < R1; ++m) {
+            const int k = min(max(point_column<R1>(p, l, m) - fp.colA0, 0), fp.lenA - 1);
+            a[m] = Ta[k];
+            c[m] = Tb[k];
         }
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = t + u * Tp;
-            if (n < fp.lenA)
-                put_ext(z, fp.xfA, n, fp.lenA, L, ha ? (double)xa[u] : 0.,
-                        hb ? (double)xb[u] : 0.);
-        }
-    } else {
-        for (int n = t; n < fp.lenA; n += Tp)
-            put_ext(z, fp.xfA, n, fp.lenA, L, ha ? (double)Ta[n] : 0., hb ? (double)Tb[n] : 0.);
+        Roots<R1 / 2 + 1> w;
+        w.load(g.tw, p.lanes, l);
+        V x[R1];
+        extend<R1>(x, p, sine, l, [&](int m, int) {
+            return mk<V>(ha ? a[m] : (S)0, hb ? c[m] : (S)0);
+        });
+        fft_first<R1>(x, z, p, sine, l, w);
     }
-    put_ext_zeros(z, fp.xfA, fp.lenA, t);
-    __syncthreads();
-    fft_any<L_, S>(z, g, tw, t);
-
+    sr.store(p, g.tw, tw);
     double mean = 0.;
     if (fp.partial) {
         double s = 0.;
         for (int k = threadIdx.x; k < fp.lenA; k += blockDim.x) s += fp.partial[k];
-        s = wave_sum(s);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-        __syncthreads();
-        double tot = 0.;
-        const int nw = blockDim.x >> 6;
-        for (int w = 0; w < nw; ++w) tot += red[w];
-        mean = tot / ((double)N * N);
+        mean = block_sum(s, red) / ((double)N * N);
     }
+
+    const int nt = L_ ? p.threads : (int)blockDim.x;
+    const G* guess = b.resid ? gp<G>(b.guess[fp.kind]) : nullptr;
+    const G* prevF = gp<G>(fp.prevF);
+    const size_t oa = (size_t)ra * N, ob = (size_t)min(rb, N - 1) * N;
+    // prev and guess values of kCols columns of both rows (columns clamped in
+    // bounds), all on their way before the first is used
+    constexpr int kCols = 4;
+    G qa[kCols], qb[kCols], ga[kCols], gb[kCols];
+    auto fetch = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < kCols; ++u) {
+            const int j = min(j0 + u * nt, N - 1);
+            qa[u] = qb[u] = ga[u] = gb[u] = (G)0;
+            if (prevF) {
+                qa[u] = prevF[oa + j];
+                qb[u] = prevF[ob + j];
+            }
+            if (guess) {
+                ga[u] = guess[oa + j];
+                gb[u] = guess[ob + j];
+            }
+        }
+    };
+    fft_stages<L_>(z, p, sine, tw);
 
     const bool transverse = fp.kind == F_EX || fp.kind == F_EY ||
                             fp.kind == F_BX || fp.kind == F_BY;
     const bool varA = b.variantA && transverse;
-    const G* guess = b.resid ? gp<G>(b.guess[fp.kind]) : nullptr;
-    const G* prevF = gp<G>(fp.prevF);
     G* const outF = gp<G>(fp.outF);
     G* const outAvg = gp<G>(fp.outAvg);
     double r_num = 0., r_den = 0.;
-    // one output point (i, j) of this pair: F from the spectrum value v,
-    // prev and guess values p, q of that point
-    auto emit = [&](int i, int j, double v, double p, double q) {
-        const size_t idx = (size_t)i * N + j;
+    // one output point: F from the spectrum value v, prev and guess values q, r
+    auto emit = [&](size_t idx, double v, double q, double r) {
         double F = v;
         if (fp.partial) F -= mean;                         // lcode.py:362
-        if (varA) F = 2 * F - p;                           // lcode.py:869-871
+        if (varA) F = 2 * F - q;                           // lcode.py:869-871
         if (outF) outF[idx] = (G)F;
-        if (outAvg) outAvg[idx] = (G)((F + p) / 2);        // lcode.py:876-881
+        if (outAvg) outAvg[idx] = (G)((F + q) / 2);        // lcode.py:876-881
         if (guess) {
-            const double d = F - q;
+            const double d = F - r;
             r_num += d * d;
             r_den += F * F;
         }
     };
-    // the field value at column j: a row without data shares its FFT with
-    // a partner row; keep it an exact zero instead of the partner's noise
-    auto spec = [&](int j, double& va, double& vb) {
-        va = vb = 0.;
-        const int k = j - fp.colA0;
-        if (k >= 0 && k < fp.lenA) get_ext(z, fp.xfA, k, va, vb);
-        if (!ha) va = 0.;
-        if (!hb) vb = 0.;
-    };
-    if constexpr (L_ != 0) {
-        // the prev and guess loads of every point of the thread first
-        // (rows and columns clamped in bounds), then the stores
-        constexpr int kPer = points_per_thread(L_, std::is_same<S, float>::value);
-        const size_t oa = (size_t)min(ra, N - 1) * N, ob = (size_t)min(rb, N - 1) * N;
-        double pa[kPer], pb[kPer], qa[kPer], qb[kPer];
+    for (int j0 = threadIdx.x; j0 < N; j0 += kCols * nt) {
+        fetch(j0);
 #pragma unroll
-        for (int u = 0; u < kPer; ++u) pa[u] = pb[u] = qa[u] = qb[u] = 0.;
-        if (prevF) {
-#pragma unroll
-            for (int u = 0; u < kPer; ++u) {
-                const int jc = min(t + u * Tp, N - 1);
-                pa[u] = prevF[oa + jc];
-                pb[u] = prevF[ob + jc];
-            }
-        }
-        if (guess) {
-#pragma unroll
-            for (int u = 0; u < kPer; ++u) {
-                const int jc = min(t + u * Tp, N - 1);
-                qa[u] = guess[oa + jc];
-                qb[u] = guess[ob + jc];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int j = t + u * Tp;
-            if (j >= N) continue;
-            double va, vb;
-            spec(j, va, vb);
-            if (ra < N) emit(ra, j, va, pa[u], qa[u]);
-            if (rb < N) emit(rb, j, vb, pb[u], qb[u]);
-        }
-    } else {
-        for (int j = t; j < N; j += Tp) {
-            double va, vb;
-            spec(j, va, vb);
-            const size_t ia = (size_t)ra * N + j, ib = (size_t)rb * N + j;
-            if (ra < N)
-                emit(ra, j, va, prevF ? (double)prevF[ia] : 0., guess ? (double)guess[ia] : 0.);
-            if (rb < N)
-                emit(rb, j, vb, prevF ? (double)prevF[ib] : 0., guess ? (double)guess[ib] : 0.);
+        for (int u = 0; u < kCols; ++u) {
+            const int j = j0 + u * nt;
+            if (j >= N) break;
+            // columns outside the transform are exact zeros, and so is a row without
+            // data (not the noise of the row that shares its transform)
+            double a, c;
+            get_pair(z, sine, j, a, c);
+            const bool inside = j >= fp.colA0 && j < fp.colA0 + fp.lenA;
+            emit(oa + j, inside && ha ? a : 0., qa[u], ga[u]);
+            if (rb < N) emit(ob + j, inside && hb ? c : 0., qb[u], gb[u]);
         }
     }
     if (b.resid) {
         // guided step: this block's share of the corrector's residual against
         // the guess, summed over its waves; one reduction kernel adds the
         // blocks' partials afterwards (no same-address atomics)
-        r_num = wave_sum(r_num);
-        r_den = wave_sum(r_den);
-        __shared__ double rs[2][16];
-        const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-        if ((threadIdx.x & 63) == 0) {
-            rs[0][w] = r_num;
-            rs[1][w] = r_den;
-        }
-        __syncthreads();
+        r_num = block_sum(r_num, red);
+        r_den = block_sum(r_den, red);
         if (threadIdx.x == 0) {
-            double a = 0., d = 0.;
-            for (int k = 0; k < nw; ++k) {
-                a += rs[0][k];
-                d += rs[1][k];
-            }
             const int lin = blockIdx.y * gridDim.x + blockIdx.x;
-            b.resid_part[2 * lin] = a;
-            b.resid_part[2 * lin + 1] = d;
+            b.resid_part[2 * lin] = r_num;
+            b.resid_part[2 * lin + 1] = r_den;
         }
     }
 }
@@ -1104,422 +1097,6 @@ guess_kernel(GuessArgs p) {
     }
 }
 
-
-// ---------------------------------------------------------------------------
-// Wave FFT (L = 1280 and 2560): one line pair per T = L / 20 lanes (one
-// wave at L = 1280, two at 2560), one pair per block (four in pass C at
-// L = 1280).  With n = l + T m and k = k1 + 20 k2,
-//   X[k1 + 20 k2] = sum_l W_T^(l k2) W_L^(l k1) sum_m x[l + T m] W_20^(m k1):
-// lane l holds the 20 points x[l + T m] in registers and transforms them
-// there (a Good-Thomas 4 x 5 DFT, no internal twiddles), multiplies by
-// W_L^(l k1), and the 20 transforms of length T across the lanes run as
-// Stockham radix-4 (and a last radix-2) stages through LDS, batched over k1
-// with k1 fastest: z[row * 20 + (k1 ^ swz(row))], lanes taking butterflies
-// beta = k1 + 20 b in order, so every LDS access of an instruction is a run
-// of consecutive 16-B points (the XOR spreads the first exchange's
-// stride-20 stores over the banks).  The last stage keeps its outputs in
-// registers: lane l's output (r, q) is X[l + T r + q L / R], consecutive
-// across lanes, so the passes read and write global memory coalesced.
-// Against the radix-4/5 plan above: four LDS exchanges per transform instead
-// of six, no barrier across waves at L = 1280, a quarter less VALU work.
-// ---------------------------------------------------------------------------
-
-// LCODE_FFT_WAVE_POINTS_1280: points per lane at L = 1280, 20 (one wave per
-// line pair) or 10 (two waves: a Good-Thomas 2 x 5 DFT-10 per lane, stages
-// 4, 4, 4, 2 across 128 lanes, four waves per SIMD).  L = 2560 takes 20.
-#ifndef LCODE_FFT_WAVE_POINTS_1280
-#define LCODE_FFT_WAVE_POINTS_1280 20
-#endif
-
-template <int L> struct WaveLanes {
-    static constexpr int R1 = L == 1280 ? LCODE_FFT_WAVE_POINTS_1280 : 20;   // points per lane
-    static constexpr int T = L / R1;                                          // lanes per pair
-    static_assert(R1 == 20 || R1 == 10, "wave FFT: 20 or 10 points per lane");
-    static_assert(T == 64 || T == 128, "wave FFT: one or two waves per line pair");
-};
-
-// LDS address of point (row, k1) of the batched transforms: rows of R1
-// points, k1 XOR-swizzled within the row (20: by (row >> 1) & 3, 10: by
-// (row >> 2) & 1) so that the first exchange's stride-R1 stores of eight
-// consecutive lanes hit eight different 16-byte bank groups.
-template <int R1>
-__device__ __forceinline__ int waddr(int row, int k1) {
-    const int sw = R1 == 20 ? (row >> 1) & 3 : (row >> 2) & 1;
-    return row * R1 + (k1 ^ sw);
-}
-
-// In-place DFT of R1 = N1 N2 points (gcd 1) by Good-Thomas: n = (N2 n1 + N1
-// n2) mod R1, k = (N2 (N2^-1 mod N1) k1 + N1 (N1^-1 mod N2) k2) mod R1, so
-// W_R1^(nk) = W_N1^(n1 k1) W_N2^(n2 k2) and no twiddles are needed: 20 = 4
-// x 5 (k = 5 k1 + 16 k2), 10 = 2 x 5 (k = 5 k1 + 6 k2).
-template <int R1, typename V>
-__device__ __forceinline__ void dft_lane(V (&x)[R1]) {
-    constexpr int N1 = R1 == 20 ? 4 : 2, N2 = 5;
-    constexpr int K1 = R1 == 20 ? 5 : 5, K2 = R1 == 20 ? 16 : 6;
-    V a[N2][N1];
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) {
-#pragma unroll
-        for (int n1 = 0; n1 < N1; ++n1) a[n2][n1] = x[(N2 * n1 + N1 * n2) % R1];
-        Dft<N1, V>::run(a[n2]);
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) {
-        V b[N2];
-#pragma unroll
-        for (int n2 = 0; n2 < N2; ++n2) b[n2] = a[n2][k1];
-        Dft<N2, V>::run(b);
-#pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) x[(K1 * k1 + K2 * k2) % R1] = b[k2];
-    }
-}
-
-// Lane l's extension points x[l + T m] of the type-1 transform whose n
-// inputs (pairs) are e[0 .. n) in LDS: cosine x[p] = e[p] (p <= L/2),
-// e[L - p] above; sine x[p] = e[p - 1] below L/2, -e[L - 1 - p] above,
-// 0 at p = 0 and L/2.
-template <int L, typename V>
-__device__ __forceinline__ void wext_load(const V* e, int xf, int lane,
-                                          V (&x)[WaveLanes<L>::R1]) {
-    constexpr int T = WaveLanes<L>::T, R1 = WaveLanes<L>::R1, H = L / 2;
-#pragma unroll
-    for (int m = 0; m < R1; ++m) {
-        const int p = lane + T * m;        // p < H exactly for m < R1 / 2
-        if (xf == XF_DCT) {
-            x[m] = e[m < R1 / 2 ? p : L - p];
-        } else if (m < R1 / 2) {
-            const V v = e[max(p - 1, 0)];
-            x[m] = p == 0 ? mk<V>(0, 0) : v;
-        } else {
-            const V v = e[min(L - 1 - p, H - 2)];
-            x[m] = p == H ? mk<V>(0, 0) : mk<V>(-v.x, -v.y);
-        }
-    }
-}
-
-// One Stockham stage of radix R and span SPAN over the R1 transforms of
-// length T in z: lane l takes butterflies beta = l + T r, r < ceil(R1 / R),
-// of the R1 T / R (the last r partial when R does not divide R1); the last
-// stage (R dividing R1) leaves output (r, q) in x[r * R + q].
-template <int L, int R, int SPAN, bool LAST, typename V>
-__device__ __forceinline__ void wstage(V* z, V (&x)[WaveLanes<L>::R1],
-                                       const double2* __restrict__ tw, int lane) {
-    constexpr int T = WaveLanes<L>::T, R1 = WaveLanes<L>::R1;
-    constexpr int NB = (R1 + R - 1) / R, NBT = R1 * T / R, STRIDE = T / R;
-    static_assert(!LAST || R1 % R == 0, "the last stage's radix divides R1");
-    V v[NB][R];
-    double2 w[NB];   // W_(SPAN R)^k = W_L^(k L / (SPAN R)) of each butterfly
-#pragma unroll
-    for (int r = 0; r < NB; ++r) {
-        const int beta = min(lane + T * r, NBT - 1);   // a partial r repeats the last
-        const int k1 = beta % R1, b = beta / R1, k = b % SPAN;
-        if constexpr (SPAN > 1) w[r] = tw[k * (L / (SPAN * R))];
-#pragma unroll
-        for (int q = 0; q < R; ++q) v[r][q] = z[waddr<R1>(b + q * STRIDE, k1)];
-    }
-    __syncthreads();   // every read of the stage before its first write
-#pragma unroll
-    for (int r = 0; r < NB; ++r) {
-        const int beta = lane + T * r;
-        if (NBT % T != 0 && beta >= NBT) continue;   // (only in a partial r)
-        if constexpr (SPAN > 1) {
-            // the powers formed in FP64, each rounded once to the transform's
-            // precision
-            double2 wq = w[r];
-#pragma unroll
-            for (int q = 1; q < R; ++q) {
-                if (q > 1) wq = cmul(wq, w[r]);
-                v[r][q] = cmul(v[r][q], mk<V>(wq.x, wq.y));
-            }
-        }
-        Dft<R, V>::run(v[r]);
-        if constexpr (LAST) {
-#pragma unroll
-            for (int q = 0; q < R; ++q) x[r * R + q] = v[r][q];
-        } else {
-            const int k1 = beta % R1, b = beta / R1, k = b % SPAN;
-            const int j = (b - k) * R + k;
-#pragma unroll
-            for (int q = 0; q < R; ++q) z[waddr<R1>(j + q * SPAN, k1)] = v[r][q];
-        }
-    }
-    if constexpr (!LAST) __syncthreads();
-}
-
-// Forward FFT of length L of the extension points in x (from wext_load).
-// z: T * R1 points of LDS, free on entry (the caller synchronised after its
-// last read).  On return x[r * R + q] = X[lane + T r + q L / R], R the last
-// radix (4 for one wave per pair at L = 1280, 2 otherwise), and z is free
-// again.
-template <int L, typename V>
-__device__ __forceinline__ void wave_fft(V* z, V (&x)[WaveLanes<L>::R1],
-                                         const double2* __restrict__ tw, int lane) {
-    constexpr int T = WaveLanes<L>::T, R1 = WaveLanes<L>::R1;
-    // W_L^(lane k1) = W_L^(lane 4a) W_L^(lane c) for k1 = 4a + c: a few
-    // table entries, one FP64 product each
-    constexpr int NA = (R1 + 3) / 4;
-    double2 lo[4], hi[NA];
-#pragma unroll
-    for (int c = 1; c < 4; ++c) lo[c] = tw[lane * c];
-#pragma unroll
-    for (int a = 1; a < NA; ++a) hi[a] = tw[lane * 4 * a];
-    dft_lane<R1>(x);
-#pragma unroll
-    for (int k1 = 1; k1 < R1; ++k1) {
-        const int a = k1 / 4, c = k1 % 4;
-        const double2 w = a == 0 ? lo[c] : c == 0 ? hi[a] : cmul(hi[a], lo[c]);
-        x[k1] = cmul(x[k1], mk<V>(w.x, w.y));
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < R1; ++k1) z[waddr<R1>(lane, k1)] = x[k1];
-    __syncthreads();
-    wstage<L, 4, 1, false>(z, x, tw, lane);
-    wstage<L, 4, 4, false>(z, x, tw, lane);
-    if constexpr (T == 64) {
-        wstage<L, 4, 16, true>(z, x, tw, lane);
-    } else {
-        wstage<L, 4, 16, false>(z, x, tw, lane);
-        wstage<L, 2, 64, true>(z, x, tw, lane);
-    }
-}
-
-template <int L> struct WaveOut {
-    static constexpr int R = WaveLanes<L>::T == 64 ? 4 : 2;   // last radix
-};
-
-#define LCODE_WAVE_R1 WaveLanes<L>::R1
-
-// The outputs of the type-1 transform held by this lane: f(u, k) for each
-// (register u, output k).
-template <int L, typename F>
-__device__ __forceinline__ void wext_index(int xf, int lane, F&& f) {
-    constexpr int T = WaveLanes<L>::T, R = WaveOut<L>::R, H = L / 2;
-#pragma unroll
-    for (int u = 0; u < LCODE_WAVE_R1; ++u) {
-        const int r = u / R, q = u % R;
-        if (q >= R / 2) continue;
-        const int idx = lane + T * r + q * (L / R);
-        if (xf == XF_DCT) f(u, idx);
-        else if (idx >= 1) f(u, idx - 1);
-    }
-    if (xf == XF_DCT && lane == 0) f(R / 2, H);
-}
-
-// Calls f(u, k, a, b) for every output k of the type-1 transform held by
-// this lane (register u; wext_index gives the (u, k) pairs alone): cosine
-// (L / 2 + 1 outputs) a = Re X[k], b = Im X[k]; sine (L / 2 - 1 outputs)
-// a = -Im X[k + 1], b = Re X[k + 1].  The registers with q < R / 2 hold
-// X[idx] for idx < L / 2; X[L / 2] is lane 0's register R / 2.
-template <int L, typename V, typename F>
-__device__ __forceinline__ void wext_out(const V (&x)[LCODE_WAVE_R1], int xf,
-                                         int lane, F&& f) {
-    wext_index<L>(xf, lane, [&](int u, int k) {
-        if (xf == XF_DCT) f(u, k, (double)x[u].x, (double)x[u].y);
-        else f(u, k, -(double)x[u].y, (double)x[u].x);
-    });
-}
-
-// Waves per SIMD the LDS allows (160 KiB per CU, L points per block of T
-// lanes): 40 / R1 with FP64 points (two at 20 points per lane, four at 10),
-// twice that with FP32 (three asked for: 168 registers, where the FP32
-// passes of L = 1280 spill at most 6; those of L = 2560 are not launched).
-#define LCODE_WAVE_ATTR(S) \
-    __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? 40 / WaveLanes<L>::R1 : 3)))
-
-__device__ __forceinline__ double block_sum_waves(double v, double* scratch) {
-    v = wave_sum(v);
-    if (blockDim.x == 64) return v;
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) scratch[w] = v;
-    __syncthreads();
-    double t = 0.;
-    for (int k = 0; k < (int)(blockDim.x >> 6); ++k) t += scratch[k];
-    __syncthreads();
-    return t;
-}
-
-template <int L, typename S, typename G>
-__global__ void __launch_bounds__(WaveLanes<L>::T) LCODE_WAVE_ATTR(S)
-pass_a_wave_kernel(SolverGeom g, SolveBatch b) {
-    using V = typename Vec<S>::T;
-    constexpr int T = WaveLanes<L>::T;
-    constexpr int kPer = (L / 2 + 1 + T - 1) / T;   // inputs per lane
-    __shared__ V z[T * LCODE_WAVE_R1];
-    if (!gate_open(b.gate)) return;
-    const BlockPos bp = xcd_block_rows();
-    const FieldPlan& fp = b.f[bp.field];
-    const int N = g.N, lane = threadIdx.x;
-    // grid rows ga (even) and ga + 1
-    const int ga = bp.block * 2, gb = ga + 1;
-    const int ta = ga - fp.rowsA0, tb = gb - fp.rowsA0;   // rows of the transform
-    const bool va = ta >= 0 && ta < fp.rowsA, vb = tb >= 0 && tb < fp.rowsA;
-    if (!va && !vb) return;
-    {
-        double a[kPer], c[kPer];
-        const int gc = va ? ga : gb;   // rows without data read a valid one
-        rhs_rows<kPer, G, sizeof(S) == 8 ? LCODE_RHS_BATCH : 0>(fp.kind, gc, vb ? gb : gc,
-                                                                fp.colA0, fp.lenA, lane, T, N,
-                                                                b.in, a, c);
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = lane + u * T;
-            if (n < fp.lenA) z[n] = mk<V>(va ? (S)a[u] : (S)0, vb ? (S)c[u] : (S)0);
-        }
-    }
-    __syncthreads();
-    V x[LCODE_WAVE_R1];
-    wext_load<L>(z, fp.xfA, lane, x);
-    __syncthreads();
-    wave_fft<L>(z, x, g.wave_tw, lane);
-    S* const Ta = static_cast<S*>(fp.T) + (size_t)ga * g.ld;
-    S* const Tb = Ta + g.ld;
-    wext_out<L>(x, fp.xfA, lane, [&](int, int k, double a, double c) {
-        if (va) Ta[k] = (S)a;
-        if (vb) Tb[k] = (S)c;
-    });
-}
-
-// Waves per SIMD of the FP32 wave pass C (build option; 3 as the other
-// FP32 passes: at 2 the mixed six-field solve measured the same).
-#ifndef LCODE_WAVE_C_F32_WAVES
-#define LCODE_WAVE_C_F32_WAVES 3
-#endif
-#define LCODE_WAVE_C_ATTR(S) \
-    __attribute__((amdgpu_waves_per_eu(sizeof(S) == 8 ? 40 / WaveLanes<L>::R1 : LCODE_WAVE_C_F32_WAVES)))
-
-template <int L, typename S, typename G>
-__global__ void __launch_bounds__(WaveLanes<L>::T) LCODE_WAVE_C_ATTR(S)
-pass_c_wave_kernel(SolverGeom g, SolveBatch b) {
-    using V = typename Vec<S>::T;
-    constexpr int T = WaveLanes<L>::T;
-    constexpr int kPer = (L / 2 + 1 + T - 1) / T;
-    __shared__ V z[T * LCODE_WAVE_R1];
-    if (!gate_open(b.gate)) return;
-    const BlockPos bp = xcd_block();
-    const FieldPlan& fp = b.f[bp.field];
-    const int N = g.N, lane = threadIdx.x;
-    const int ra = bp.block * 2, rb = ra + 1;
-    auto has = [&](int r) { return r < N && r - fp.rowsA0 >= 0 && r - fp.rowsA0 < fp.rowsA; };
-    const bool ha = has(ra), hb = has(rb);
-    {
-        // (rows without data read a valid row, and are dropped)
-        const S* Ta = static_cast<const S*>(fp.T) + (size_t)(ha ? ra : fp.rowsA0) * g.ld;
-        const S* Tb = static_cast<const S*>(fp.T) + (size_t)(hb ? rb : fp.rowsA0) * g.ld;
-        S xa[kPer], xb[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = min(lane + u * T, fp.lenA - 1);
-            xa[u] = Ta[n];
-            xb[u] = Tb[n];
-        }
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int n = lane + u * T;
-            if (n < fp.lenA) z[n] = mk<V>(ha ? xa[u] : (S)0, hb ? xb[u] : (S)0);
-        }
-    }
-    __syncthreads();
-    V x[LCODE_WAVE_R1];
-    wext_load<L>(z, fp.xfA, lane, x);
-    __syncthreads();
-    wave_fft<L>(z, x, g.wave_tw, lane);
-
-    double mean = 0.;
-    if (fp.partial) {
-        double s = 0.;
-        for (int k = lane; k < fp.lenA; k += T) s += fp.partial[k];
-        mean = block_sum_waves(s, reinterpret_cast<double*>(z)) / ((double)N * N);
-    }
-    const bool transverse = fp.kind == F_EX || fp.kind == F_EY ||
-                            fp.kind == F_BX || fp.kind == F_BY;
-    const bool varA = b.variantA && transverse;
-    const G* guess = b.resid ? gp<G>(b.guess[fp.kind]) : nullptr;
-    const G* prevF = gp<G>(fp.prevF);
-    G* const outF = gp<G>(fp.outF);
-    G* const outAvg = gp<G>(fp.outAvg);
-    double r_num = 0., r_den = 0.;
-    auto emit = [&](int i, int j, double v, double p, double q) {
-        const size_t idx = (size_t)i * N + j;
-        double F = v;
-        if (fp.partial) F -= mean;                         // lcode.py:362
-        if (varA) F = 2 * F - p;                           // lcode.py:869-871
-        if (outF) outF[idx] = (G)F;
-        if (outAvg) outAvg[idx] = (G)((F + p) / 2);        // lcode.py:876-881
-        if (guess) {
-            const double d = F - q;
-            r_num += d * d;
-            r_den += F * F;
-        }
-    };
-    // output column j of the lane's register u: j = lane + T r + q L / R
-    // (the cosine transform's index, 1 + the sine transform's), below L / 2
-    // for q < R / 2; column L / 2 = N - 1 is lane 0's register R / 2.
-    // Columns outside [colA0, colA0 + lenA) are exact zeros.
-    constexpr int R = WaveOut<L>::R, H = L / 2;
-    const size_t oa = (size_t)ra * N, ob = (size_t)min(rb, N - 1) * N;
-    auto value = [&](int u, int j, double& va, double& vb) {
-        va = vb = 0.;
-        const int k = j - fp.colA0;
-        if (k >= 0 && k < fp.lenA) {
-            if (fp.xfA == XF_DCT) {
-                va = x[u].x;
-                vb = x[u].y;
-            } else {
-                va = -(double)x[u].y;
-                vb = x[u].x;
-            }
-        }
-        if (!ha) va = 0.;
-        if (!hb) vb = 0.;
-    };
-    {
-        constexpr int kOut = LCODE_WAVE_R1 / 2;   // registers with q < R / 2
-        G pa[kOut], pb[kOut], qa[kOut], qb[kOut];
-#pragma unroll
-        for (int s = 0; s < kOut; ++s) {
-            const int r = s / (R / 2), q = s % (R / 2), u = r * R + q;
-            (void)u;
-            const int j = lane + T * r + q * (L / R);
-            pa[s] = pb[s] = qa[s] = qb[s] = (G)0;
-            if (prevF) {
-                pa[s] = prevF[oa + j];
-                pb[s] = prevF[ob + j];
-            }
-            if (guess) {
-                qa[s] = guess[oa + j];
-                qb[s] = guess[ob + j];
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < kOut; ++s) {
-            const int r = s / (R / 2), q = s % (R / 2), u = r * R + q;
-            const int j = lane + T * r + q * (L / R);
-            double va, vb;
-            value(u, j, va, vb);
-            emit(ra, j, va, pa[s], qa[s]);
-            if (rb < N) emit(rb, j, vb, pb[s], qb[s]);
-        }
-    }
-    if (lane == 0) {
-        double va, vb;
-        value(R / 2, H, va, vb);
-        emit(ra, H, va, prevF ? (double)prevF[oa + H] : 0., guess ? (double)guess[oa + H] : 0.);
-        if (rb < N)
-            emit(rb, H, vb, prevF ? (double)prevF[ob + H] : 0., guess ? (double)guess[ob + H] : 0.);
-    }
-    if (b.resid) {
-        double* scratch = reinterpret_cast<double*>(z);
-        r_num = block_sum_waves(r_num, scratch);
-        r_den = block_sum_waves(r_den, scratch);
-        if (threadIdx.x == 0) {
-            const int lin = blockIdx.y * gridDim.x + blockIdx.x;
-            b.resid_part[2 * lin] = r_num;
-            b.resid_part[2 * lin + 1] = r_den;
-        }
-    }
-}
-
 }  // namespace
 
 // Pass B's shape: 8 lines per block (a wave reads runs of 64 bytes) and 12
@@ -1556,14 +1133,15 @@ static int launch_pass_b(const SolverGeom& g, const SolveBatch& b, hipStream_t s
     return LCODE_OK;
 }
 
-template <int L_, bool TW_LDS, typename S, typename G>
-static int launch_passes(const SolverGeom& g, const SolveBatch& b,
-                         hipStream_t s, Profiler* prof, size_t lds,
-                         dim3 ga, dim3 gc) {
-    const dim3 block(g.P * g.Tp);
+template <int R1, int L_, typename S, typename G>
+static int launch_passes(const SolverGeom& g, const SolveBatch& b, hipStream_t s,
+                         Profiler* prof) {
+    // one block per field and pair of grid rows
+    const dim3 grid((g.N + 1) / 2, b.nfields), block(g.fft.threads);
+    const size_t lds = (size_t)solver_lds_bytes(g);
     {
         ProfScope ps(prof, "solve_pass_a", s, true);
-        launch_timed(ps, pass_a_kernel<L_, TW_LDS, S, G>, ga, block, lds, s, g, b);
+        launch_timed(ps, pass_a_kernel<R1, L_, S, G>, grid, block, lds, s, g, b);
     }
     LCODE_HIP(hipGetLastError());
     {
@@ -1572,129 +1150,123 @@ static int launch_passes(const SolverGeom& g, const SolveBatch& b,
     }
     {
         ProfScope ps(prof, "solve_pass_c", s, true);
-        launch_timed(ps, pass_c_kernel<L_, TW_LDS, S, G>, gc, block, lds, s, g, b);
+        launch_timed(ps, pass_c_kernel<R1, L_, S, G>, grid, block, lds, s, g, b);
     }
     LCODE_HIP(hipGetLastError());
     if (b.resid) {
         ProfScope ps(prof, "resid_reduce", s);
-        resid_reduce_kernel<<<1, 256, 0, s>>>(b.resid_part, (int)(gc.x * gc.y), b.resid);
+        resid_reduce_kernel<<<1, 256, 0, s>>>(b.resid_part, (int)(grid.x * grid.y), b.resid);
         LCODE_HIP(hipGetLastError());
     }
     return LCODE_OK;
 }
 
 int solver_lds_bytes(const SolverGeom& g) {
-    const size_t cplx = g.fp32 ? sizeof(float2) : sizeof(double2);
-    const size_t data = (size_t)g.P * padded_len(g.fft.L) * cplx;
-    if (g.static_L == 0) return (int)(data + ((size_t)g.fft.L / 4 + 1) * cplx / 2);
-    if (g.tw_lds) return (int)(data + (size_t)tw_count(g.fft.L) * sizeof(double2));
-    return (int)data;
+    return g.fft.nroots * (int)sizeof(double2) +
+           g.fft.T * g.fft.KP * (int)(g.fp32 ? sizeof(float2) : sizeof(double2));
 }
 
-int solver_padded_len(int L) { return padded_len(L); }
-
-int solver_tw_count(int L) { return tw_count(L); }
-
-int solver_threads_per_pair(int L, bool fp32, bool static_plan) {
-    return static_plan ? static_threads_per_pair(L, fp32) : threads_per_pair(L);
+std::vector<double2> solver_fft_roots(const FftPlan& p) {
+    std::vector<double2> t;
+    auto add = [&](int R, int n, int step) {   // W_L^(step k q), [root][k < n]
+        for (int q = 1; q < R; q += q < 4 ? 1 : 4)
+            for (int k = 0; k < n; ++k) {
+                const long double a = 2.0L * 3.14159265358979323846264338327950288L *
+                                      ((long)step * k * q % p.L) / p.L;
+                t.push_back(make_double2((double)std::cos(a), (double)-std::sin(a)));
+            }
+    };
+    add(p.K, p.lanes, 1);
+    for (int s = 1; s < p.nst; ++s) {
+        const int R = fft_word_radix(p.word[s]), span = fft_word_span(p.word[s]);
+        add(R, span, p.L / (span * R));
+    }
+    return t;
 }
 
-int solver_static_radix(int rem) { return next_radix(rem); }
-
-#ifndef LCODE_FFT_STATIC_PLANS
-#define LCODE_FFT_STATIC_PLANS 1
-#endif
-
-// LCODE_FFT_WAVE (1): the wave FFT passes for the FP64 transforms of L = 1280
-// and 2560 (grids of 641^2 and 1281^2); 0 keeps the radix-4/5 plan there too.
-#ifndef LCODE_FFT_WAVE
-#define LCODE_FFT_WAVE 1
-#endif
-
-bool solver_static_length(int L) {
-    if (!LCODE_FFT_STATIC_PLANS) return false;
-    switch (L) {
-        case 32: case 64: case 128: case 256: case 512: case 640:
-        case 1024: case 1280: case 2048: case 2560:
-            return true;
-        default:
-            return false;
+// The plan of a length without one of its own: the cheapest of all factorisations
+// under
+//   (sum of the radices + 8 per stage + 4 per 64 w columns) x rounds,
+// a block's chain (DFTs in registers, an LDS exchange per stage, columns per thread in the
+// assembly and the stores; a unit is about 0.1 us a pass) times how often the CU's
+// wave slots are filled: w waves per block, 16 resident per CU (128 registers), rounds =
+// the mean of the exact and the rounded-up number, at least 1.  Passes A + C,
+// six fields, us, with the plan's cost in brackets:
+//   301^2  4;5,5,6 21.5 (64)     4;15,10 22.0 (65)    10;6,10 23.7 (70)
+//   361^2  4;4,5,9 24.3 (62)     12;6,10 24.7 (64)    8;9,10 27.2 (75)
+//   451^2  20;5,9 30.0 (74)      12;5,15 31.0 (72)    4;5,5,9 37.0 (103)
+//   801^2  10;10,16 64.8 (140)   8;5,5,8 68.7 (198)
+//   901^2  8;15,15 82.1 (156)    20;9,10 84.7 (158)   4;5,9,10 128.7 (286)
+//   1081^2 12;12,15 116 (178)    16;9,15 129 (244)    8;5,6,9 168 (350)
+bool solver_fft_plan(int L, FftPlan* out) {
+    if (const int k = static_fft(L); k >= 0) {
+        const StaticFft& f = kStaticFft[k];
+        *out = make_plan(L, f.R1, f.nst, f.r);
+        return true;
     }
-}
-
-template <int L, typename S, typename G>
-static int launch_wave_passes(const SolverGeom& g, const SolveBatch& b,
-                              hipStream_t s, Profiler* prof) {
-    const dim3 block(WaveLanes<L>::T);
-    {
-        ProfScope ps(prof, "solve_pass_a", s, true);
-        // one block per pair of grid rows
-        launch_timed(ps, pass_a_wave_kernel<L, S, G>, dim3((g.N + 1) / 2, b.nfields),
-                     block, 0, s, g, b);
+    constexpr int kCUs = 256, kSlots = 16, kMaxThreads = 512;
+    const int N = L / 2 + 1;
+    const double blocks = 6. * ((N + 1) / 2) / kCUs;
+    double best = 0;
+    bool found = false;
+    int r[kMaxStages];
+    for (int R1 : {4, 8, 10, 12, 16, 20}) {
+        if (L % R1) continue;
+        auto search = [&](auto&& self, int depth, int rest, int sum) -> void {
+            if (rest == 1) {
+                const FftPlan p = make_plan(L, R1, depth, r);
+                if (p.threads > kMaxThreads) return;
+                const int w = p.threads / 64;
+                const double x = blocks / (kSlots / w);
+                const double rounds = std::max(1., (x + std::ceil(x)) / 2);
+                const double cost =
+                    (sum + 8 * (depth + 1) + 4 * ((N + p.threads - 1) / p.threads)) * rounds;
+                if (found && cost >= best) return;
+                found = true;
+                best = cost;
+                *out = p;
+                return;
+            }
+            if (depth == kMaxStages) return;
+            for (int R : {2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16}) {
+                if (rest % R) continue;
+                r[depth] = R;
+                self(self, depth + 1, rest / R, sum + R);
+            }
+        };
+        search(search, 0, L / R1, R1);
     }
-    LCODE_HIP(hipGetLastError());
-    {
-        const int rc = launch_pass_b<S>(g, b, s, prof);
-        if (rc) return rc;
-    }
-    const dim3 gc((g.N + 1) / 2, b.nfields);
-    {
-        ProfScope ps(prof, "solve_pass_c", s, true);
-        launch_timed(ps, pass_c_wave_kernel<L, S, G>, gc, block, 0, s,
-                     g, b);
-    }
-    LCODE_HIP(hipGetLastError());
-    if (b.resid) {
-        ProfScope ps(prof, "resid_reduce", s);
-        resid_reduce_kernel<<<1, 256, 0, s>>>(b.resid_part, (int)(gc.x * gc.y), b.resid);
-        LCODE_HIP(hipGetLastError());
-    }
-    return LCODE_OK;
-}
-
-bool solver_wave_length(int L) {
-    return LCODE_FFT_WAVE && (L == 1280 || L == 2560);
+    return found;
 }
 
 template <typename S, typename G>
 static int launch_solve_t(const SolverGeom& g, const SolveBatch& b,
                           hipStream_t s, Profiler* prof) {
-    const size_t lds = (size_t)solver_lds_bytes(g);
-    const int per_block = 2 * g.P;
-    int max_a = 0;
-    for (int f = 0; f < b.nfields; ++f) max_a = max_a > b.f[f].rowsA ? max_a : b.f[f].rowsA;
-    // the wave FFT runs the FP64 transforms and, with LCODE_FFT_WAVE_FP32, the
-    // FP32 ones of L = 1280 (the workspace sets wave_tw only then)
-    if constexpr (std::is_same<S, double>::value || LCODE_FFT_WAVE_FP32) if (g.wave_tw) {
-        // the wave passes take a cosine transform of N points from column
-        // (or line) 0 and a sine transform of N - 2 from 1
-        for (int f = 0; f < b.nfields; ++f) {
-            const FieldPlan& p = b.f[f];
-            const bool ok = p.xfA == XF_DCT ? p.lenA == g.N && p.colA0 == 0
-                                            : p.lenA == g.N - 2 && p.colA0 == 1;
-            if (!ok) {
-                set_error("internal: field plan outside the wave FFT layout");
-                return LCODE_E_INVALID;
-            }
+    // a cosine line has the N points from column 0, a sine line the N - 2 from 1
+    for (int f = 0; f < b.nfields; ++f) {
+        const FieldPlan& p = b.f[f];
+        const bool ok = p.xfA == XF_DCT ? p.lenA == g.N && p.colA0 == 0
+                                        : p.lenA == g.N - 2 && p.colA0 == 1;
+        if (!ok) {
+            set_error("internal: field plan outside the transform's layout");
+            return LCODE_E_INVALID;
         }
-        if (g.fft.L == 1280) return launch_wave_passes<1280, S, G>(g, b, s, prof);
-        if (g.fft.L == 2560) return launch_wave_passes<2560, S, G>(g, b, s, prof);
     }
-    const dim3 ga((max_a + per_block - 1) / per_block, b.nfields);
-    const dim3 gc((g.N + per_block - 1) / per_block, b.nfields);
-#define LCODE_CASE(LL)                                                          \
-    case LL:                                                                    \
-        return g.tw_lds                                                         \
-                   ? launch_passes<LL, true, S, G>(g, b, s, prof, lds, ga, gc) \
-                   : launch_passes<LL, false, S, G>(g, b, s, prof, lds, ga, gc);
-    switch (g.static_L) {
-        LCODE_CASE(32) LCODE_CASE(64) LCODE_CASE(128) LCODE_CASE(256)
-        LCODE_CASE(512) LCODE_CASE(640) LCODE_CASE(1024) LCODE_CASE(1280)
-        LCODE_CASE(2048) LCODE_CASE(2560)
-        default:
-            return launch_passes<0, false, S, G>(g, b, s, prof, lds, ga, gc);
-    }
+    switch (g.fft.L) {
+#define LCODE_CASE(LL) \
+    case LL: return launch_passes<kStaticFft[static_fft(LL)].R1, LL, S, G>(g, b, s, prof);
+        LCODE_CASE(64) LCODE_CASE(128) LCODE_CASE(256) LCODE_CASE(512) LCODE_CASE(640)
+        LCODE_CASE(1024) LCODE_CASE(1280) LCODE_CASE(2048) LCODE_CASE(2560)
 #undef LCODE_CASE
+    }
+    switch (g.fft.R1) {
+        case 4: return launch_passes<4, 0, S, G>(g, b, s, prof);
+        case 8: return launch_passes<8, 0, S, G>(g, b, s, prof);
+        case 10: return launch_passes<10, 0, S, G>(g, b, s, prof);
+        case 12: return launch_passes<12, 0, S, G>(g, b, s, prof);
+        case 16: return launch_passes<16, 0, S, G>(g, b, s, prof);
+        default: return launch_passes<20, 0, S, G>(g, b, s, prof);
+    }
 }
 
 int launch_guess(const GuessArgs& p, hipStream_t s, Profiler* prof) {
