@@ -130,6 +130,21 @@ __device__ __forceinline__ int xcd_logical(int lin, int total) {
     return xcd < r ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
 }
 
+// Reads the first word of each 64-byte line of a kernel argument, so that the lines come
+// in together and not one by one where their members are first used (pass A 10.8 -> 10.1 us
+// at 257^2, 8.1 -> 7.4 at 129^2).
+template <typename T>
+__device__ __forceinline__ void fetch_lines(const T& v) {
+    const unsigned* w = reinterpret_cast<const unsigned*>(&v);
+    constexpr int n = (sizeof(T) + 63) / 64;
+    unsigned t[n + 1];
+#pragma unroll
+    for (int k = 0; k < n; ++k) t[k] = w[16 * k];
+    t[n] = w[sizeof(T) / 4 - 1];
+#pragma unroll
+    for (int k = 0; k <= n; ++k) asm volatile("" ::"s"(t[k]));
+}
+
 // ---------------------------------------------------------------------------
 // TSC-2D shape (lcode.py:396-418)
 // ---------------------------------------------------------------------------
@@ -505,6 +520,8 @@ struct FieldPlan {
     const double* table;      // dense solvers: [lenA][rowsA] spectral multiplier
     const double* tri;        // FFT solvers: s = 1 - l of the tridiagonal
                               // elimination, [rowsA][ld] (pass B)
+    const int* tri_last;      // [lenA]: the row from which a line of it is constant,
+                              // or NULL
     double tri_scale;         // h^2 / (2 (N - 1)): of the right-hand side there
     int zero_mode;            // Bz: drop the zero mode
     void* T;                  // scratch spectra (S), [N][ld] by grid row

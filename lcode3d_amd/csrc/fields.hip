@@ -671,21 +671,6 @@ __device__ __forceinline__ BlockPos xcd_block_rows() {
 // Passes
 // ---------------------------------------------------------------------------
 
-// Reads the first word of each 64-byte line of a kernel argument, so that the lines come
-// in together and not one by one where their members are first used (pass A 10.8 -> 10.1 us
-// at 257^2, 8.1 -> 7.4 at 129^2).
-template <typename T>
-__device__ __forceinline__ void fetch_lines(const T& v) {
-    const unsigned* w = reinterpret_cast<const unsigned*>(&v);
-    constexpr int n = (sizeof(T) + 63) / 64;
-    unsigned t[n + 1];
-#pragma unroll
-    for (int k = 0; k < n; ++k) t[k] = w[16 * k];
-    t[n] = w[sizeof(T) / 4 - 1];
-#pragma unroll
-    for (int k = 0; k <= n; ++k) asm volatile("" ::"s"(t[k]));
-}
-
 // Pass A: a block takes one field's grid rows ga (even) and ga + 1.  All its threads
 // assemble right-hand sides, a column of both rows at a time (at 641^2 21.8 us; two and three
 // columns in flight 24.4 and 23.9: more registers; the first stage's lanes alone, at their own points,
@@ -764,6 +749,11 @@ pass_a_kernel(SolverGeom g, SolveBatch b) {
 // Six fields, us per launch, against the transform along i, multiplier and
 // transform back that this replaced: 361^2 28.6 -> 9.4, 641^2 23.4 -> 13.7,
 // 1281^2 122 -> 62, 641^2 with FP32 spectra 17.5 -> 12.9.
+//
+// All but the smoothest lines' multipliers are constant after a few rows (the
+// elimination has converged to the last bit): on large grids the rows behind that
+// one read it again (tri_last), which keeps most of the tables out of the traffic:
+// 1281^2 62.4 -> 54.1 us, 641^2 14.0 -> 13.8, with FP32 spectra 13.4 -> 12.6.
 template <int R, int CB, typename S>
 __global__ void __launch_bounds__(1024)
 pass_b_kernel(SolverGeom g, SolveBatch b) {
@@ -775,6 +765,8 @@ pass_b_kernel(SolverGeom g, SolveBatch b) {
     // same multipliers
     const BlockPos bp = xcd_block_rows();
     const FieldPlan& fp = b.f[bp.field];
+    fetch_lines(g);
+    fetch_lines(fp);
     const int n = fp.rowsA, k0 = bp.block * CB;
     if (k0 >= fp.lenA) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
@@ -789,12 +781,16 @@ pass_b_kernel(SolverGeom g, SolveBatch b) {
     // all loads first, rows clamped in bounds; the rows from n on become
     // zero rows (s = 1) whose solution is 0
     double y[R], s[R];
+    const int last = fp.tri_last ? fp.tri_last[kc] : n - 1;
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-        y[i] = (double)T[at(r0 + i)];
-        s[i] = tab[at(r0 + i)];
-    }
-    const double s_before = tab[at(r0 - 1)];
+    for (int i = 0; i < R; ++i) y[i] = (double)T[at(r0 + i)];
+    // the multipliers are constant from row `last` on (but for the cosine's last row)
+    auto tri_at = [&](int row) {
+        return tab[at(neumann && row >= n - 1 ? n - 1 : min(row, last))];
+    };
+#pragma unroll
+    for (int i = 0; i < R; ++i) s[i] = tri_at(r0 + i);
+    const double s_before = tri_at(r0 - 1);
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         const int row = r0 + i;
