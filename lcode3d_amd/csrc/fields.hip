@@ -262,9 +262,9 @@ template <typename V> struct Dft<16, V> {
 // wavefronts per SIMD on small grids, memory on large ones (1281^2: pass C 320 MB in
 // 67 us).  Six fields, passes A / C, us per launch, transforms of the whole extension
 // (radix 4 in LDS; 20 points per lane at 641^2 and 1281^2) -> of half of it:
-// 129^2 6.4 / 6.4 -> 6.2 / 6.2, 257^2 9.7 / 9.2 -> 8.8 / 8.2, 361^2 19.2 / 19.0 ->
-// 13.0 / 11.3, 641^2 23.8 / 21.2 -> 21.8 / 17.0, with FP32 transforms and grids 18.4 / 20.2
-// -> 15.1 / 15.0, 1281^2 96.8 / 80.3 -> 81.0 / 66.8.
+// 129^2 6.4 / 6.4 -> 6.3 / 6.2, 257^2 9.7 / 9.2 -> 8.6 / 8.2, 361^2 19.2 / 19.0 ->
+// 12.3 / 11.3, 641^2 23.8 / 21.2 -> 21.2 / 17.0, with FP32 transforms and grids 18.4 / 20.2
+// -> 14.0 / 15.0, 1281^2 96.8 / 80.3 -> 80.5 / 66.3.
 // ---------------------------------------------------------------------------
 
 // Roots held per butterfly of radix R: w^q, q = 1, 2, 3, 4, 8, 12 (below R).
@@ -531,11 +531,15 @@ __device__ __forceinline__ void extend(V (&x)[R1], const FftPlan& p, bool sine, 
 }
 
 // Right-hand sides of rows i and i + 1 (clamped to the grid: a row outside it, or
-// without data, is dropped by the caller) at column j; the values of rhs_value_k.  Row bases are uniform, the lane adds a 32-bit byte offset, and a
-// derivative along i takes the sources of its four rows once.
+// without data, is dropped by the caller) at column j; the values of rhs_value_k.  The
+// grids' bases are uniform and the lane holds one 32-bit offset per row, for all grids (a base
+// per row and grid took more scalar registers than there are: 641^2 22.4 us against 21.2,
+// 1281^2 86.7 against 80.5); a derivative along i takes the
+// sources of its four rows once.
 template <typename G>
-__device__ __forceinline__ double at_byte(const G* row, unsigned off) {
-    return (double)*reinterpret_cast<const G*>(reinterpret_cast<const char*>(row) + off);
+__device__ __forceinline__ double at(const G* base, unsigned e) {
+    return (double)*reinterpret_cast<const G*>(reinterpret_cast<const char*>(base) +
+                                               e * (unsigned)sizeof(G));
 }
 
 template <int KIND, typename G>
@@ -547,24 +551,24 @@ __device__ __forceinline__ void rhs_pair_k(int i, int j, int N, const RhsInputs&
     auto over_h2 = [&](double x) { return quotient(x, in.h * 2, in.inv_h2); };
     auto over_dxi = [&](double x) { return quotient(x, in.dxi, in.inv_dxi); };
     const G *jx = gp<G>(in.jx), *jy = gp<G>(in.jy);
-    auto row = [&](const auto* base, int r) { return base + (size_t)r * N; };
     const bool jin = j >= 1 && j <= N - 2;
-    const int oj = jin ? 1 : 0;
-    const unsigned o = (unsigned)j * sizeof(G), op = (unsigned)(j + oj) * sizeof(G),
-                   om = (unsigned)(j - oj) * sizeof(G);
+    const unsigned oj = jin ? 1 : 0;
+    unsigned o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (unsigned)(rows[r] * N + j);
     if constexpr (KIND == F_EZ) {
         // the interior only carries this right-hand side (zero elsewhere)
-        const double x0 = at_byte(row(jx, rows[0]), o), x1 = at_byte(row(jx, rows[1]), o),
-                     x2 = at_byte(row(jx, rows[2]), o), x3 = at_byte(row(jx, rows[3]), o);
-        const double ya = at_byte(row(jy, i), op) - at_byte(row(jy, i), om);
-        const double yc = at_byte(row(jy, i1), op) - at_byte(row(jy, i1), om);
+        const double x0 = at(jx, o[0]), x1 = at(jx, o[1]),
+                     x2 = at(jx, o[2]), x3 = at(jx, o[3]);
+        const double ya = at(jy, o[1] + oj) - at(jy, o[1] - oj);
+        const double yc = at(jy, o[2] + oj) - at(jy, o[2] - oj);
         a = over_h2(-((x2 - x0) + ya));
         c = over_h2(-((x3 - x1) + yc));
     } else if constexpr (KIND == F_BZ) {
-        const double x0 = at_byte(row(jy, rows[0]), o), x1 = at_byte(row(jy, rows[1]), o),
-                     x2 = at_byte(row(jy, rows[2]), o), x3 = at_byte(row(jy, rows[3]), o);
-        const double ya = at_byte(row(jx, i), op) - at_byte(row(jx, i), om);
-        const double yc = at_byte(row(jx, i1), op) - at_byte(row(jx, i1), om);
+        const double x0 = at(jy, o[0]), x1 = at(jy, o[1]),
+                     x2 = at(jy, o[2]), x3 = at(jy, o[3]);
+        const double ya = at(jx, o[1] + oj) - at(jx, o[1] - oj);
+        const double yc = at(jx, o[2] + oj) - at(jx, o[2] - oj);
         const bool n0 = in0 && jin, n1 = in1 && jin;
         a = over_h2(-((n0 ? ya : 0.) - (n0 ? x2 - x0 : 0.)));
         c = over_h2(-((n1 ? yc : 0.) - (n1 ? x3 - x1 : 0.)));
@@ -580,27 +584,27 @@ __device__ __forceinline__ void rhs_pair_k(int i, int j, int N, const RhsInputs&
         const double* beam = in.beam ? in.beam : dummy;
         const double on = in.beam ? 1. : 0., off = in.beam ? 0. : in.beam_scalar;
         // (a beam is added to the source of every derivative: lcode.py:862-863)
-        auto source = [&](int r, unsigned ob, int jj) {
-            const double s = (at_byte(row(src, r), ob) + at_byte(row(prev, r), ob)) / 2;
-            return s + (at_byte(row(beam, r), (unsigned)jj * 8u) * on + off);
+        auto source = [&](unsigned e) {
+            const double s = (at(src, e) + at(prev, e)) / 2;
+            return s + (at(beam, e) * on + off);
         };
         double da, dc;
         if constexpr (along_i) {
-            const double s0 = source(rows[0], o, j), s1 = source(rows[1], o, j);
-            const double s2 = source(rows[2], o, j), s3 = source(rows[3], o, j);
+            const double s0 = source(o[0]), s1 = source(o[1]);
+            const double s2 = source(o[2]), s3 = source(o[3]);
             da = s2 - s0;
             dc = s3 - s1;
         } else {
-            da = source(i, op, j + oj) - source(i, om, j - oj);
-            dc = source(i1, op, j + oj) - source(i1, om, j - oj);
+            da = source(o[1] + oj) - source(o[1] - oj);
+            dc = source(o[2] + oj) - source(o[2] - oj);
         }
         const G* jp = gp<G>(xcur ? in.jx_prev : in.jy_prev);
         const G* jc = xcur ? jx : jy;
         const G* tr = gp<G>(in.Ftrick[ft]);
-        const double ja = over_dxi(at_byte(row(jp, i), o) - at_byte(row(jc, i), o));
-        const double jc1 = over_dxi(at_byte(row(jp, i1), o) - at_byte(row(jc, i1), o));
-        const double ta = at_byte(row(tr, i), o) * in.trick;
-        const double tc = at_byte(row(tr, i1), o) * in.trick;
+        const double ja = over_dxi(at(jp, o[1]) - at(jc, o[1]));
+        const double jc1 = over_dxi(at(jp, o[2]) - at(jc, o[2]));
+        const double ta = at(tr, o[1]) * in.trick;
+        const double tc = at(tr, o[2]) * in.trick;
         const double fa = (in0 && jin ? over_h2(da) : 0.) - ja;
         const double fc = (in1 && jin ? over_h2(dc) : 0.) - jc1;
         if constexpr (KIND == F_BX) {
@@ -672,9 +676,9 @@ __device__ __forceinline__ BlockPos xcd_block_rows() {
 // ---------------------------------------------------------------------------
 
 // Pass A: a block takes one field's grid rows ga (even) and ga + 1.  All its threads
-// assemble right-hand sides, a column of both rows at a time (at 641^2 21.8 us; two and three
-// columns in flight 24.4 and 23.9: more registers; the first stage's lanes alone, at their own points,
-// 30.3), and the first stage reads them back from LDS.
+// assemble right-hand sides, a column of both rows at a time (at 641^2 21.2 us; two
+// columns in flight 22.6: more registers; the first stage's lanes alone, at their own
+// points, 30.3), and the first stage reads them back from LDS.
 // G: storage type of the source grids (FP64 arithmetic in both).
 template <int R1, int L_, typename S, typename G>
 __global__ void __launch_bounds__(512)
