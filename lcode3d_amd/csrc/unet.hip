@@ -46,65 +46,122 @@ __device__ __forceinline__ float bf2f(uint16_t b) {
 // Convolution (forward, and input gradient with transposed weights)
 // ---------------------------------------------------------------------------
 
-// Output channels of the block: mt * 16 (mt = 1, 2 or 4).
-template <int MT>
-__global__ void __launch_bounds__(256)
+constexpr int kHalo = kHaloR * kHaloC;              // 204 pixels of a tile with its halo
+constexpr int kTileThreads = 256;
+// 16-byte quarters of a 32-channel input tile per thread
+constexpr int kTileLoads = (kHalo * 4 + kTileThreads - 1) / kTileThreads;
+
+// 2 x 2 mean of a finer tensor from its four pixels (those outside it zero).
+__device__ __forceinline__ uint4 pool4(const uint4* u) {
+    float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t w4[4] = {u[d].x, u[d].y, u[d].z, u[d].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[2 * e] += bf2f((uint16_t)(w4[e] & 0xFFFFu));
+            f[2 * e + 1] += bf2f((uint16_t)(w4[e] >> 16));
+        }
+    }
+    uint32_t w4[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        w4[e] = (uint32_t)f2bf(f[2 * e] * .25f) | ((uint32_t)f2bf(f[2 * e + 1] * .25f) << 16);
+    return make_uint4(w4[0], w4[1], w4[2], w4[3]);
+}
+
+// The thread's quarters of the input tile at (r0 - 1, c0 - 1) (zeros outside the
+// plane), all loads issued before one is used.  mode: UnetConvArgs::in_mode.
+__device__ __forceinline__ void load_tile(const uint16_t* in, int mode, int in_h, int in_w, int H,
+                                          int W, int r0, int c0, uint4* v) {
+    const uint4 zero = make_uint4(0, 0, 0, 0);
+    auto place = [&](int i, int& gr, int& gc, int& q) {
+        const int k = min((int)threadIdx.x + i * kTileThreads, kHalo * 4 - 1), pix = k >> 2;
+        q = k & 3;
+        gr = r0 - 1 + pix / kHaloC;
+        gc = c0 - 1 + pix % kHaloC;
+        return gr >= 0 && gr < H && gc >= 0 && gc < W;
+    };
+    auto at = [&](int row, int col, int w, int q) {
+        return *reinterpret_cast<const uint4*>(in + ((size_t)row * w + col) * kC + q * 8);
+    };
+    int gr, gc, q;
+    if (mode != 1) {
+        const int sh = mode == 2 ? 1 : 0, w = mode == 2 ? in_w : W;
+#pragma unroll
+        for (int i = 0; i < kTileLoads; ++i) {
+            place(i, gr, gc, q);
+            v[i] = at(min(max(gr, 0), H - 1) >> sh, min(max(gc, 0), W - 1) >> sh, w, q);
+        }
+#pragma unroll
+        for (int i = 0; i < kTileLoads; ++i)
+            if (!place(i, gr, gc, q)) v[i] = zero;
+    } else {
+        uint4 u[kTileLoads][4];
+#pragma unroll
+        for (int i = 0; i < kTileLoads; ++i) {
+            place(i, gr, gc, q);
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                u[i][d] = at(min(max(2 * gr + d / 2, 0), in_h - 1),
+                             min(max(2 * gc + d % 2, 0), in_w - 1), in_w, q);
+        }
+#pragma unroll
+        for (int i = 0; i < kTileLoads; ++i) {
+            const bool in_plane = place(i, gr, gc, q);
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                if (2 * gr + d / 2 >= in_h || 2 * gc + d % 2 >= in_w) u[i][d] = zero;
+            v[i] = in_plane ? pool4(u[i]) : zero;
+        }
+    }
+}
+
+// Output channels of the block: MT * 16 (MT = 1, 2 or 4); input chunks NIN.  Bound: the
+// chain of one block (246 of them at 161 x 161 pixels, fewer below): its loads, then
+// 9 NIN taps.  The weights (18 to 37 KB) and the tile are therefore loaded by
+// all threads at once into registers, one round trip, before they go to LDS; a loop
+// of load and store took one per 16 bytes of a thread.  us per launch, mean over
+// the levels of S = 161: inference 13.9 -> 8.5, training 10.4 -> 7.3 (MT = 4: 11.2 -> 7.7).
+// (Three taps unrolled against one: 8.5 and 8.7.)
+template <int MT, int NIN>
+__global__ void __launch_bounds__(kTileThreads)
 unet_conv_kernel(UnetConvArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    uint16_t* sx = reinterpret_cast<uint16_t*>(lds_raw);          // [nin][6][34][40]
-    const int cin = kC * a.nin;
-    const int wrow = cin + 8;                                       // packed row stride
-    uint16_t* sw = sx + (size_t)a.nin * kHaloR * kHaloC * kPix;     // [9][MT*16][cin+8]
+    uint16_t* sx = reinterpret_cast<uint16_t*>(lds_raw);          // [NIN][6][34][40]
+    constexpr int cin = kC * NIN;
+    constexpr int wrow = cin + 8;                                   // packed row stride
+    uint16_t* sw = sx + (size_t)NIN * kHalo * kPix;                 // [9][MT*16][cin+8]
     const int tiles_x = (a.W + kTC - 1) / kTC;
     const int r0 = (blockIdx.x / tiles_x) * kTR, c0 = (blockIdx.x % tiles_x) * kTC;
 
-    // stage the input tile with its halo (zeros outside the plane), 16 B
-    // per thread and step
-    const int chunks = a.nin * kHaloR * kHaloC * 4;
-    for (int k = threadIdx.x; k < chunks; k += blockDim.x) {
-        const int q = k & 3, pix = k >> 2;
-        const int ch = pix / (kHaloR * kHaloC), rem = pix % (kHaloR * kHaloC);
-        const int rr = rem / kHaloC, cc = rem % kHaloC;
-        const int gr = r0 - 1 + rr, gc = c0 - 1 + cc;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (gr >= 0 && gr < a.H && gc >= 0 && gc < a.W) {
-            const int mode = a.in_mode[ch];
-            if (mode == 0) {
-                v = *reinterpret_cast<const uint4*>(a.in[ch] + ((size_t)gr * a.W + gc) * kC + q * 8);
-            } else if (mode == 2) {       // nearest upsampling of a coarser tensor
-                v = *reinterpret_cast<const uint4*>(
-                    a.in[ch] + ((size_t)(gr / 2) * a.in_w[ch] + gc / 2) * kC + q * 8);
-            } else {                      // 2 x 2 mean of a finer tensor
-                float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                for (int da = 0; da < 2; ++da)
-                    for (int db = 0; db < 2; ++db) {
-                        const int ii = 2 * gr + da, jj = 2 * gc + db;
-                        if (ii >= a.in_h[ch] || jj >= a.in_w[ch]) continue;
-                        const uint4 u = *reinterpret_cast<const uint4*>(
-                            a.in[ch] + ((size_t)ii * a.in_w[ch] + jj) * kC + q * 8);
-                        const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
+    // the packed weights [9][MT*16][cin], 16 B per thread and step
+    constexpr int wchunks = 9 * MT * 16 * (cin / 8);
+    constexpr int kW = (wchunks + kTileThreads - 1) / kTileThreads;
+    uint4 wv[kW], xv[NIN][kTileLoads];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            f[2 * e] += bf2f((uint16_t)(w4[e] & 0xFFFFu));
-                            f[2 * e + 1] += bf2f((uint16_t)(w4[e] >> 16));
-                        }
-                    }
-                uint32_t w4[4];
+    for (int i = 0; i < kW; ++i)
+        wv[i] = *reinterpret_cast<const uint4*>(
+            a.w + 8 * (size_t)min((int)threadIdx.x + i * kTileThreads, wchunks - 1));
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    w4[e] = (uint32_t)f2bf(f[2 * e] * .25f) | ((uint32_t)f2bf(f[2 * e + 1] * .25f) << 16);
-                v = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-            }
-        }
-        *reinterpret_cast<uint4*>(sx + (size_t)pix * kPix + q * 8) = v;
-    }
-    // stage the packed weights [9][MT*16][cin] into rows of cin + 8
-    const int wchunks = 9 * MT * 16 * (cin / 8);
-    for (int k = threadIdx.x; k < wchunks; k += blockDim.x) {
+    for (int ch = 0; ch < NIN; ++ch)
+        load_tile(a.in[ch], a.in_mode[ch], a.in_h[ch], a.in_w[ch], a.H, a.W, r0, c0, xv[ch]);
+    // rows of cin + 8 in LDS
+#pragma unroll
+    for (int i = 0; i < kW; ++i) {
+        const int k = threadIdx.x + i * kTileThreads;
         const int q = k % (cin / 8), row = k / (cin / 8);
-        *reinterpret_cast<uint4*>(sw + (size_t)row * wrow + q * 8) =
-            *reinterpret_cast<const uint4*>(a.w + (size_t)row * cin + q * 8);
+        if (k < wchunks) *reinterpret_cast<uint4*>(sw + (size_t)row * wrow + q * 8) = wv[i];
     }
+#pragma unroll
+    for (int ch = 0; ch < NIN; ++ch)
+#pragma unroll
+        for (int i = 0; i < kTileLoads; ++i) {
+            const int k = threadIdx.x + i * kTileThreads;
+            if (k < kHalo * 4)
+                *reinterpret_cast<uint4*>(sx + (size_t)(ch * kHalo + (k >> 2)) * kPix +
+                                          (k & 3) * 8) = xv[ch][i];
+        }
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -114,9 +171,9 @@ unet_conv_kernel(UnetConvArgs a) {
     for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[n][m] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int ch = 0; ch < a.nin; ++ch) {
-        const uint16_t* xc = sx + (size_t)ch * kHaloR * kHaloC * kPix;
-#pragma unroll 1
+    for (int ch = 0; ch < NIN; ++ch) {
+        const uint16_t* xc = sx + (size_t)ch * kHalo * kPix;
+#pragma unroll 3
         for (int tap = 0; tap < 9; ++tap) {
             const int ty = tap / 3, tx = tap % 3;
             bf8 b[2];
@@ -185,31 +242,60 @@ unet_conv_kernel(UnetConvArgs a) {
 // Per block: the output gradient of its 4 x 32 pixels transposed into
 // gT[co][128] and the input tile (with halo) into xT[ci][6 * 34]; wave w
 // takes taps w, w + 4 (and 8 for wave 0); MT output-channel tiles of 16,
-// NN = cin / 16 input-channel tiles.
+// NN = cin / 16 input-channel tiles.  Bound: the chain of a block; its 30 to 60 KB came in by
+// single channels, one round trip per 512 of them: S = 161, us per launch, <2, 4> 36.7 -> 10.7,
+// <2, 2> 18.7 -> 7.1, <1, 2> 14.4 -> 7.2.
 template <int MT, int NN>
 __global__ void __launch_bounds__(256)
 unet_wgrad_kernel(UnetWgradArgs a) {
     constexpr int kTile = kTR * kTC;                 // 128 pixels
     constexpr int kCin = NN * 16;
-    constexpr int kHalo = kHaloR * kHaloC;           // 204 pixels
     __shared__ __align__(16) uint16_t gT[MT * 16][kTile + 8];
     __shared__ __align__(16) uint16_t xT[kCin][kHalo + 4];
     const int tiles_x = (a.W + kTC - 1) / kTC;
     const int r0 = (blockIdx.x / tiles_x) * kTR, c0 = (blockIdx.x % tiles_x) * kTC;
-    for (int k = threadIdx.x; k < kTile * MT * 16; k += blockDim.x) {
-        const int co = k % (MT * 16), px = k / (MT * 16);
-        const int gr = r0 + px / kTC, gc = c0 + px % kTC;
-        uint16_t v = 0;
-        if (gr < a.H && gc < a.W) v = a.g[((size_t)gr * a.W + gc) * kC + co];
-        gT[co][px] = v;
-    }
-    for (int k = threadIdx.x; k < kHalo * kCin; k += blockDim.x) {
-        const int ci = k % kCin, px = k / kCin;
-        const int gr = r0 - 1 + px / kHaloC, gc = c0 - 1 + px % kHaloC;
-        uint16_t v = 0;
-        if (gr >= 0 && gr < a.H && gc >= 0 && gc < a.W)
-            v = a.in[ci / kC][((size_t)gr * a.W + gc) * kC + ci % kC];
-        xT[ci][px] = v;
+    // 16 bytes (8 channels of a pixel) per thread and step, all loads first; adjacent
+    // threads take adjacent pixels, which the transposed stores write side by side
+    {
+        constexpr int kG = kTile * MT * 2, kX = kHalo * NN * 2;
+        constexpr int nG = (kG + 255) / 256, nX = (kX + 255) / 256;
+        uint4 gv[nG], xv[nX];
+#pragma unroll
+        for (int i = 0; i < nG; ++i) {
+            const int k = min((int)threadIdx.x + i * 256, kG - 1), px = k % kTile, q = k / kTile;
+            const int gr = min(r0 + px / kTC, a.H - 1), gc = min(c0 + px % kTC, a.W - 1);
+            gv[i] = *reinterpret_cast<const uint4*>(a.g + ((size_t)gr * a.W + gc) * kC + q * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < nX; ++i) {
+            const int k = min((int)threadIdx.x + i * 256, kX - 1), px = k % kHalo, q = k / kHalo;
+            const int gr = min(max(r0 - 1 + px / kHaloC, 0), a.H - 1);
+            const int gc = min(max(c0 - 1 + px % kHaloC, 0), a.W - 1);
+            const uint16_t* in = NN > 2 && q >= 4 ? a.in[1] : a.in[0];
+            xv[i] = *reinterpret_cast<const uint4*>(in + ((size_t)gr * a.W + gc) * kC + q % 4 * 8);
+        }
+        auto put = [](uint16_t* row, int stride, uint4 v) {
+            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                row[(2 * e) * stride] = (uint16_t)(w4[e] & 0xFFFFu);
+                row[(2 * e + 1) * stride] = (uint16_t)(w4[e] >> 16);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < nG; ++i) {
+            const int k = threadIdx.x + i * 256, px = k % kTile, q = k / kTile;
+            const bool in_plane = r0 + px / kTC < a.H && c0 + px % kTC < a.W;
+            if (k < kG)
+                put(&gT[q * 8][px], kTile + 8, in_plane ? gv[i] : make_uint4(0, 0, 0, 0));
+        }
+#pragma unroll
+        for (int i = 0; i < nX; ++i) {
+            const int k = threadIdx.x + i * 256, px = k % kHalo, q = k / kHalo;
+            const int gr = r0 - 1 + px / kHaloC, gc = c0 - 1 + px % kHaloC;
+            const bool in_plane = gr >= 0 && gr < a.H && gc >= 0 && gc < a.W;
+            if (k < kX) put(&xT[q * 8][px], kHalo + 4, in_plane ? xv[i] : make_uint4(0, 0, 0, 0));
+        }
     }
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -253,10 +339,11 @@ unet_wgrad_kernel(UnetWgradArgs a) {
                 }
     }
     // bias gradient: the output gradient summed over the tile's pixels
-    if (threadIdx.x < MT * 16) {
+    // (by the last wave: the first has three taps)
+    if (const int co = (int)threadIdx.x - 192; co >= 0 && co < MT * 16) {
         float s = 0.f;
-        for (int px = 0; px < kTile; ++px) s += bf2f(gT[threadIdx.x][px]);
-        part[9 * MT * 16 * kCin + threadIdx.x] = s;
+        for (int px = 0; px < kTile; ++px) s += bf2f(gT[co][px]);
+        part[9 * MT * 16 * kCin + co] = s;
     }
 }
 
@@ -451,29 +538,36 @@ __device__ __forceinline__ double fld(const void* p, int f32, size_t idx) {
 // takes level-0 pixel p and plane group g (field g < 6: channels g and
 // 6 + g; 6: the beam; 7: the density and the zero channels), so adjacent
 // threads read adjacent 4-value row segments of one plane.
+template <typename G>
 __global__ void __launch_bounds__(256)
 unet_inputs_kernel(UnetIoArgs a) {
     const int S = a.S, N = a.N, P = S * S;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= 8 * P) return;
     const int g = k / P, p = k % P, I = p / S, J = p % S;
-    const void* src = g < 6 ? a.f1[g] : a.ro;
+    const G* src = static_cast<const G*>(g < 6 ? a.f1[g] : a.ro);
+    const G* src2 = static_cast<const G*>(a.f2[min(g, 5)]);
     double s1 = 0., s2 = 0.;
-    for (int a4 = 0; a4 < 4; ++a4) {
-        const int i = 4 * I + a4;
-        if (i >= N) break;
-        for (int b4 = 0; b4 < 4; ++b4) {
-            const int j = 4 * J + b4;
-            if (j >= N) break;
-            const size_t idx = (size_t)i * N + j;
-            if (g == 6) {
-                s1 += a.beam ? a.beam[idx] : a.beam_scalar;
-            } else {
-                const double x1 = fld(src, a.f32, idx);
-                s1 += x1;
-                if (g < 6) s2 += x1 - fld(a.f2[g], a.f32, idx);
-            }
-        }
+    // the 16 values of each source at once (clamped to the grid), those outside it
+    // dropped; a loop left at the edge waited for each (641^2 FP32 grids 16.4 -> 11.9 us)
+    auto sum = [&](auto&& value) {
+        double v[16], t = 0.;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            v[e] = value((size_t)min(4 * I + e / 4, N - 1) * N + min(4 * J + e % 4, N - 1));
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            t += 4 * I + e / 4 < N && 4 * J + e % 4 < N ? v[e] : 0.;
+        return t;
+    };
+    if (g == 6) {
+        if (a.beam) s1 = sum([&](size_t idx) { return a.beam[idx]; });
+        else s1 = sum([&](size_t) { return a.beam_scalar; });
+    } else if (g == 7) {
+        s1 = sum([&](size_t idx) { return (double)src[idx]; });
+    } else {
+        s1 = sum([&](size_t idx) { return (double)src[idx]; });
+        s2 = sum([&](size_t idx) { return (double)src[idx] - (double)src2[idx]; });
     }
     const int c1 = g < 6 ? g : (g == 6 ? 12 : 13);
     const float v1 = (float)(s1 / 16 / a.scale[c1]);
@@ -561,7 +655,7 @@ int launch_unet_conv(const UnetConvArgs& a, hipStream_t s) {
     const dim3 grid(unet_tiles(a.H, a.W));
     // blocks above 64 KiB of LDS (two input chunks) need the limit raised
     // once per instantiation (gfx950 has 160 KiB per CU)
-    static bool raised[3] = {false, false, false};
+    static bool raised[6] = {};
     auto launch = [&](auto kernel, int slot) {
         if (lds > 65536 && !raised[slot]) {
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -574,11 +668,12 @@ int launch_unet_conv(const UnetConvArgs& a, hipStream_t s) {
         return true;
     };
     bool ok;
-    switch (mt) {
-        case 1: ok = launch(unet_conv_kernel<1>, 0); break;
-        case 2: ok = launch(unet_conv_kernel<2>, 1); break;
-        case 4: ok = launch(unet_conv_kernel<4>, 2); break;
-        default: set_error("unet conv: cout_pad must be 16, 32 or 64"); return LCODE_E_INVALID;
+    if (mt == 1) ok = a.nin == 1 ? launch(unet_conv_kernel<1, 1>, 0) : launch(unet_conv_kernel<1, 2>, 1);
+    else if (mt == 2) ok = a.nin == 1 ? launch(unet_conv_kernel<2, 1>, 2) : launch(unet_conv_kernel<2, 2>, 3);
+    else if (mt == 4) ok = a.nin == 1 ? launch(unet_conv_kernel<4, 1>, 4) : launch(unet_conv_kernel<4, 2>, 5);
+    else {
+        set_error("unet conv: cout_pad must be 16, 32 or 64");
+        return LCODE_E_INVALID;
     }
     if (!ok) {
         set_error("hipFuncSetAttribute (dynamic LDS) failed for the unet convolution");
@@ -668,7 +763,10 @@ int launch_unet_mse(const float* y, const float* t, int P, uint16_t* g,
 
 int launch_unet_io(const UnetIoArgs& a, int which, hipStream_t s) {
     switch (which) {
-        case 0: unet_inputs_kernel<<<nblk(8L * a.S * a.S), 256, 0, s>>>(a); break;
+        case 0:
+            if (a.f32) unet_inputs_kernel<float><<<nblk(8L * a.S * a.S), 256, 0, s>>>(a);
+            else unet_inputs_kernel<double><<<nblk(8L * a.S * a.S), 256, 0, s>>>(a);
+            break;
         case 1: unet_targets_kernel<<<nblk((long)a.S * a.S * 6), 256, 0, s>>>(a); break;
         case 2: unet_guess_kernel<<<nblk((long)a.N * a.N), 256, 0, s>>>(a); break;
         default: return LCODE_E_INVALID;
