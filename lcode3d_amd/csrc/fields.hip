@@ -1081,19 +1081,30 @@ resid_reduce_kernel(const double* part, int nblocks, double* resid) {
 // Guided step set-up: guess = sum_t c[t] hist[t] for the six fields, the
 // predictor-pass averages (guess + prev) / 2 (lcode.py:876-881 with the
 // guess in place of the predicted fields), and zeroed residual sums.
-template <typename G>
+// Bound: memory, (6 NT + 6) grids in and 12 out; the number of terms is a template
+// parameter so that the loads of all fields are in flight at once (a loop over them:
+// 641^2 FP32 grids, three terms, 13.1 us; now 11.6).
+template <int NT, typename G>
 __global__ void __launch_bounds__(256)
 guess_kernel(GuessArgs p) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (p.acc_zero && k < 2) p.acc_zero[k] = 0.;
     if (k >= p.n) return;
+    G h[NT][6], prev[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) h[t][f] = gp<G>(p.h[t][f])[k];
+        prev[f] = gp<G>(p.prev[f])[k];
+    }
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
         double gsum = 0.;
-        for (int t = 0; t < p.nt; ++t) gsum += p.c[t] * (double)gp<G>(p.h[t][f])[k];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) gsum += p.c[t] * (double)h[t][f];
         const G gs = (G)gsum;
         gp<G>(p.guess[f])[k] = gs;
-        gp<G>(p.avg[f])[k] = (G)(((double)gs + (double)gp<G>(p.prev[f])[k]) / 2);
+        gp<G>(p.avg[f])[k] = (G)(((double)gs + (double)prev[f]) / 2);
     }
 }
 
@@ -1272,10 +1283,16 @@ static int launch_solve_t(const SolverGeom& g, const SolveBatch& b,
 int launch_guess(const GuessArgs& p, hipStream_t s, Profiler* prof) {
     {
         ProfScope ps(prof, "guess", s);
-        if (p.grid32)
-            guess_kernel<float><<<(p.n + 255) / 256, 256, 0, s>>>(p);
-        else
-            guess_kernel<double><<<(p.n + 255) / 256, 256, 0, s>>>(p);
+        auto go = [&](auto k32, auto k64) {
+            if (p.grid32) k32<<<(p.n + 255) / 256, 256, 0, s>>>(p);
+            else k64<<<(p.n + 255) / 256, 256, 0, s>>>(p);
+        };
+        switch (p.nt) {
+            case 1: go(guess_kernel<1, float>, guess_kernel<1, double>); break;
+            case 2: go(guess_kernel<2, float>, guess_kernel<2, double>); break;
+            case 3: go(guess_kernel<3, float>, guess_kernel<3, double>); break;
+            default: go(guess_kernel<4, float>, guess_kernel<4, double>); break;
+        }
     }
     LCODE_HIP(hipGetLastError());
     return LCODE_OK;
