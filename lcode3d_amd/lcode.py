@@ -42,14 +42,12 @@ def _device():
 def _as_device(array, dtype=None):
     """cp.asarray: host arrays are copied to the current device."""
     if isinstance(array, torch.Tensor):
-        t = array
-        if t.device.type != "cuda":
-            t = t.to(_device())
+        t = array if array.is_cuda else array.to(_device())
     else:
         t = torch.as_tensor(np.asarray(array), device=_device())
-    if dtype is not None:
+    if dtype is not None and t.dtype != dtype:
         t = t.to(dtype)
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 class GPUArrays:
@@ -154,7 +152,7 @@ def _stream():
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _check_grid(config, *arrays, dtype=_F64):
@@ -293,7 +291,7 @@ def calculate_Ex_Ey_Bx_By(config, Ex_avg, Ey_avg, Bx_avg, By_avg,
     beam, beam_scalar = _beam_arg(config, beam_ro)
     cs = _config_struct(config)
     outs = [torch.empty_like(grids[0]) for _ in range(4)]
-    out_pp, keep = _lib.ptr_array([o.data_ptr() for o in outs])
+    out_pp = _lib.ptr_array([o.data_ptr() for o in outs])
     g = [_ptr(t) for t in grids]
     _lib.check(lib.lcode_calculate_Ex_Ey_Bx_By(
         _workspace(cs), ctypes.byref(cs), g[0], g[1], g[2], g[3],
@@ -336,8 +334,8 @@ def move_smart(config, m, q, x_init, y_init, x_prev_offt, y_prev_offt,
     nc = parts[0].shape[0]
     cs = _config_struct(config, nc)
     outs = [torch.empty_like(parts[0]) for _ in range(5)]
-    f_pp, kf = _lib.ptr_array([f.data_ptr() for f in fields])
-    o_pp, ko = _lib.ptr_array([o.data_ptr() for o in outs])
+    f_pp = _lib.ptr_array([f.data_ptr() for f in fields])
+    o_pp = _lib.ptr_array([o.data_ptr() for o in outs])
     _lib.check(lib.lcode_move_smart(_workspace(cs), ctypes.byref(cs),
                                     *[_ptr(p) for p in parts], f_pp, o_pp,
                                     _stream()), "lcode_move_smart")
@@ -378,7 +376,7 @@ def deposit(config, ro_initial, x_offt, y_offt, m, q, px, py, pz,
     n = int(config.grid_steps)
     outs = [torch.empty((n, n), dtype=_F64, device=parts[0].device)
             for _ in range(4)]
-    o_pp, ko = _lib.ptr_array([o.data_ptr() for o in outs])
+    o_pp = _lib.ptr_array([o.data_ptr() for o in outs])
     _lib.check(lib.lcode_deposit(_workspace(cs), ctypes.byref(cs), ro0_ptr,
                                  *[_ptr(p) for p in parts], ctypes.byref(vp),
                                  o_pp, _stream()), "lcode_deposit")
