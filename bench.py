@@ -60,8 +60,8 @@ def kernel_bytes(name, nc, n):
 
     push           11 coarse inputs + 5 outputs, 6 gathered fields
     deposit_tile   7 coarse inputs, ro_initial, 4 grids out
-    solve_pass_a   13 RHS source grids in, 6 transposed spectra out
-    solve_pass_b   6 spectra + 6 eigenvalue tables in, 6 spectra out
+    solve_pass_a   13 RHS source grids in, 6 spectra out
+    solve_pass_b   6 spectra + 4 multiplier tables in, 6 spectra out
     solve_pass_c   6 spectra + 6 prev fields in, 6 averages out, plus the
                    6 fields on the corrector pass (mean: 9 grids out)
     """
@@ -70,7 +70,7 @@ def kernel_bytes(name, nc, n):
         "push": 16 * c2 + 6 * n2,
         "deposit_tile": 7 * c2 + 5 * n2,
         "solve_pass_a": 19 * n2,
-        "solve_pass_b": 18 * n2,
+        "solve_pass_b": 16 * n2,
         "solve_pass_c": 21 * n2,
     }
     return 8 * table[name] if name in table else None
