@@ -59,8 +59,8 @@ enum {
 enum {
     LCODE_SOLVER_FFT64 = 0, /* hand-written mixed-radix FFT in LDS, FP64 */
     LCODE_SOLVER_FFT32 = 1, /* the same in FP32 (mixed precision): the
-                               transforms, spectra and eigenvalue tables;
-                               RHS, Bz mean and zero mode, Variant A and
+                               transforms and spectra; RHS, solution
+                               along i, Bz mean and zero mode, Variant A and
                                averages stay FP64 */
     LCODE_SOLVER_DENSE64 = 2,      /* dense N x N sine/cosine matrices,
                                       FP64 MFMA (v_mfma_f64_16x16x4) */
@@ -134,7 +134,7 @@ const char *lcode_last_error(void);
 /* Library version string. */
 const char *lcode_version(void);
 
-/* Builds the eigenvalue and twiddle tables for cfg (N, h, trick, solver)
+/* Builds the solver's tables and roots of unity for cfg (N, h, trick, solver)
  * on the current device and allocates the step's scratch. */
 int lcode_workspace_create(const lcode_config *cfg, lcode_workspace **out);
 int lcode_workspace_destroy(lcode_workspace *ws);

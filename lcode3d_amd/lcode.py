@@ -129,7 +129,7 @@ def _solver_of(config):
     config.field_solver_transform: 'fft' (default; mixed-radix FFT in LDS)
     or 'dense' (N x N sine/cosine matrices on MFMA);
     config.field_solver_precision: 'fp64' (default, the plain path), 'fp32'
-    (FFT only: transforms, spectra and eigenvalue tables in FP32) or
+    (FFT only: transforms and spectra in FP32) or
     'bf16x3' (dense only: hi/lo BF16 splits, three MFMA products, FP32
     accumulation); in these three the RHS, Bz mean, Variant A and averages
     are FP64.  'mixed' (FFT only): the mixed-precision step - the ten grids
