@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/lcode3d_hip.h"
+#include "tile_order.hpp"
 
 namespace lcode {
 
@@ -331,12 +332,6 @@ struct DepositArgs {
                                    // arithmetic and ro_initial stay FP64)
     Gate gate;
 };
-
-// A block of the tile kernel: its tile, the slot of a split tile (or -1) and
-// which part of it.
-inline unsigned dep_entry(int tile, int slot, int part) {
-    return (unsigned)tile | (unsigned)(slot + 1) << 16 | (unsigned)part << 31;
-}
 
 int launch_estimate(const EstimateArgs& a, hipStream_t s, Profiler* prof);
 int launch_push(const PushArgs& a, hipStream_t s, Profiler* prof);

@@ -437,8 +437,8 @@ deposit_tile_kernel(DepositArgs a) {
     // tiles and light ones; its last nsplit entries are the second parts of the
     // split tiles)
     const int ntx = a.ntx, lin = blockIdx.x;
-    const unsigned entry = scalar(a.tile_order ? (int)a.tile_order[lin] : lin);
-    const int tile = entry & 0xFFFFu, slot = (int)((entry >> 16) & 0x7FFFu) - 1, part = entry >> 31;
+    const DepBlock blk = dep_block(a.tile_order, a.tile_order ? scalar((int)a.tile_order[lin]) : 0, lin);
+    const int tile = blk.tile, slot = blk.slot, part = blk.part;
     const int nparts = slot >= 0 ? 2 : 1;
     const int ty = tile / ntx, tx = tile - ty * ntx;
     const int ci0 = ty * T, cj0 = tx * T;
@@ -1107,6 +1107,8 @@ int launch_deposit(const DepositArgs& a, hipStream_t s, Profiler* prof) {
     LCODE_REQUIRE(a.nsplit >= 0 && a.nsplit <= a.ntx * a.ntx &&
                       (!a.nsplit || (a.tile_order && a.split_part && a.split_count)),
                   "deposition: inconsistent split tiles");
+    LCODE_REQUIRE(!a.tile_order || dep_entries_fit(a.ntx * a.ntx, a.nsplit),
+                  "deposition: more tiles than the block table holds");
     const DepKernel kernel = deposit_kernel_of(a.tile, a.waves, a.staged, a.grid32);
     LCODE_REQUIRE(kernel, "deposition: no kernel for this tile");
     {

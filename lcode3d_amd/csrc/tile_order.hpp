@@ -6,7 +6,34 @@
 #include <algorithm>
 #include <vector>
 
+#if defined(__HIP__)
+#define LCODE_TILE_FN __host__ __device__ __forceinline__
+#else
+#define LCODE_TILE_FN inline
+#endif
+
 namespace lcode {
+
+// What a block of the deposition's tile kernel takes: a tile, and of a split
+// tile its slot (else -1) and which of the two parts.
+struct DepBlock {
+    int tile, slot, part;
+};
+
+// A block's word of the host's table: 16 bits of tile, 15 of slot + 1, the part.
+inline unsigned dep_entry(int tile, int slot, int part) {
+    return (unsigned)tile | (unsigned)(slot + 1) << 16 | (unsigned)part << 31;
+}
+
+// Whether the tiles and slots of a launch fit the table's words.
+inline bool dep_entries_fit(int tiles, int nsplit) { return tiles <= 65536 && nsplit <= 32767; }
+
+// Block `lin`: its word, or without a table its own index as the tile (a grid
+// without a table may have more tiles than a word holds).
+LCODE_TILE_FN DepBlock dep_block(bool table, unsigned word, int lin) {
+    if (!table) return DepBlock{lin, -1, 0};
+    return DepBlock{(int)(word & 0xFFFFu), (int)(word >> 16 & 0x7FFFu) - 1, (int)(word >> 31)};
+}
 
 // Squared distance of tile t (row-major in an nt x nt grid of tiles) from
 // the grid centre, in tiles.
