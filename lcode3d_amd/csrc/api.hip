@@ -56,10 +56,13 @@ struct lcode_workspace {
     double* favg[6] = {};          // field averages of the current pass
     int* fault = nullptr;
     int* spill = nullptr;          // nf * nf spilled fine particle indices
-    int* spill_ctr = nullptr;      // [0], [1] spill counts, [2], [3] the
-                                   // pushes' displacement bound in cells,
-                                   // each pair of slots used in turn; [4]
-                                   // tile blocks done (the in-kernel spill)
+    int* spill_ctr = nullptr;      // kCounters ints: [0], [1] spill counts,
+                                   // [2], [3] the pushes' displacement bound
+                                   // in cells, each pair of slots used in
+                                   // turn; [4] tile blocks done (the in-kernel
+                                   // spill); [5], [6] the bound that a
+                                   // deposition on its own takes of its
+                                   // offsets, in turn
     int* regions = nullptr;        // the same bound per deposition tile:
                                    // two slots of region_n^2 ints
     int region_n = 0;              // tiles per side (0: no per-tile bounds)
@@ -73,6 +76,7 @@ struct lcode_workspace {
     double* split_part = nullptr;
     int* split_count = nullptr;
     int bound_slot = 0;            // slot the next push raises
+    int own_slot = 0;              // slot of the next deposition on its own
     int spill_slot = 0;            // count slot of the next deposition
     int grid_spill_left = 0;       // depositions still followed by the spill
                                    // kernel after spills were last seen
@@ -95,6 +99,8 @@ struct lcode_workspace {
 };
 
 namespace {
+
+constexpr int kCounters = 7;   // of lcode_workspace::spill_ctr
 
 // 1: per-tile displacement bounds size each deposition tile's halo; 0: the
 // largest bound over all particles sizes every tile's halo (build option)
@@ -540,7 +546,7 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     if ((rc = dev_alloc(ws, (void**)&ws->fault, sizeof(int)))) return fail(rc);
     const size_t nfp = (size_t)cfg->nf * cfg->nf;
     if ((rc = dev_alloc(ws, (void**)&ws->spill, (nfp ? nfp : 1) * sizeof(int)))) return fail(rc);
-    if ((rc = dev_alloc(ws, (void**)&ws->spill_ctr, 5 * sizeof(int)))) return fail(rc);
+    if ((rc = dev_alloc(ws, (void**)&ws->spill_ctr, kCounters * sizeof(int)))) return fail(rc);
     // per-tile displacement bounds: a deposition tile takes the largest of
     // its 3 x 3 neighbourhood, which holds every coarse particle a fine
     // particle within the largest halo + 1 cells of the tile interpolates
@@ -606,7 +612,7 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     }
     ws->host_flag[0] = ws->host_flag[1] = 0;
     if (hipMemset(ws->fault, 0, sizeof(int)) != hipSuccess ||
-        hipMemset(ws->spill_ctr, 0, 5 * sizeof(int)) != hipSuccess ||
+        hipMemset(ws->spill_ctr, 0, kCounters * sizeof(int)) != hipSuccess ||
         (ws->regions &&
          hipMemset(ws->regions, 0, 2 * (size_t)nt * nt * sizeof(int)) != hipSuccess) ||
         hipDeviceSynchronize() != hipSuccess) {
@@ -884,25 +890,31 @@ static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
     // after a push of this workspace: a halo of the pushes' displacement
     // bound, read from the slot the pushes raised; the deposition zeroes
     // the other slot, which the next pushes raise
-    if (halo != HALO_LARGEST) {
+    if (halo == HALO_OF_PUSHES) {
         a.halo_cells = ws->spill_ctr + 2 + ws->bound_slot;
         a.halo_next = ws->spill_ctr + 2 + (1 - ws->bound_slot);
         if (ws->regions) {
             const size_t nr = (size_t)ws->region_n * ws->region_n;
-            if (halo == HALO_OF_PUSHES) a.halo_regions = ws->regions + ws->bound_slot * nr;
+            a.halo_regions = ws->regions + ws->bound_slot * nr;
             a.halo_regions_next = ws->regions + (1 - ws->bound_slot) * nr;
         }
     }
+    // on its own: a slot that no push raises (it may hold the non-finite mark of
+    // a state that is not the one deposited here).  What a failed or a replayed call
+    // leaves in it is a bound of earlier offsets, which only makes halos larger.
+    int* const own = ws->spill_ctr + 5 + ws->own_slot;
+    if (halo == HALO_OF_OFFSETS) {
+        a.halo_cells = own;
+        a.halo_next = ws->spill_ctr + 5 + (1 - ws->own_slot);
+    }
     a.gate = gate;
     LCODE_REQUIRE(cfg->nf <= ws->nf, "workspace was built for fewer fine particles");
-    // (on top of what pushes may have raised the slot to: a larger bound only
-    // makes larger halos)
     int rc = LCODE_OK;
-    if (halo == HALO_OF_OFFSETS)
-        rc = launch_deposit_bound(a, ws->spill_ctr + 2 + ws->bound_slot, stream, &ws->prof);
+    if (halo == HALO_OF_OFFSETS) rc = launch_deposit_bound(a, own, stream, &ws->prof);
     if (rc == LCODE_OK) rc = launch_deposit(a, stream, &ws->prof);
     if (rc == LCODE_OK) ws->spill_slot = 1 - ws->spill_slot;
-    if (rc == LCODE_OK && halo != HALO_LARGEST) ws->bound_slot = 1 - ws->bound_slot;
+    if (rc == LCODE_OK && halo == HALO_OF_PUSHES) ws->bound_slot = 1 - ws->bound_slot;
+    if (rc == LCODE_OK && halo == HALO_OF_OFFSETS) ws->own_slot = 1 - ws->own_slot;
     return rc;
 }
 
