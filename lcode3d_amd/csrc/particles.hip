@@ -732,10 +732,13 @@ deposit_tile_kernel(DepositArgs a) {
                 const int ci = xi.z, cj = xj.z;   // initial cell
                 const bool home = ((unsigned)(ci - ci0) < (unsigned)T) &
                                   ((unsigned)(cj - cj0) < (unsigned)T);
-                // (NaN where the position is not finite)
-                const bool odd = __builtin_isunordered(xl, yl);
-                if (is_edge && !odd && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2)) {
-                    if (home) atomicAdd(a.fault, 1);
+                // (NaN where the position is not finite; further than kFarCells counts
+                // as that, which the halo test below finds but for a centre that is
+                // clamped first)
+                bool odd = __builtin_isunordered(xl, yl);
+                if (is_edge && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2)) {
+                    odd |= !(fabs(xh) <= kFarCells && fabs(yh) <= kFarCells);
+                    if (home && !odd) atomicAdd(a.fault, 1);
                     ti = min(max(ti, 1), N - 2);
                     tj = min(max(tj, 1), N - 2);
                 }
