@@ -143,6 +143,16 @@ constexpr int kDepOrder = LCODE_DEP_ORDER;
 constexpr int kDepResident = 3;   // tile blocks per CU (158 VGPRs, 4 waves) when
                                   // the runtime reports none
 
+// Per-tile displacement bounds: a deposition tile takes the largest of its 3 x 3
+// neighbourhood, which holds every coarse particle that a fine particle within the
+// largest halo + 1 cells of the tile interpolates from when 2 coarseness + 10 <= tile
+// side (a fine particle lies within 2 coarseness + 2 cells of its coarse
+// neighbours, at the plasma edge).  Asked for each call's plasma: one workspace may
+// serve several.
+bool regions_hold(const lcode_config* cfg, const DepositPlan& plan) {
+    return kDepRegions && 2 * cfg->plasma_coarseness + kDepositHalo + 4 <= plan.tile;
+}
+
 // Side of the XCD clusters of the tile order (tile_order.hpp).
 #ifndef LCODE_DEP_CLUSTER
 #define LCODE_DEP_CLUSTER 3
@@ -547,11 +557,6 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     const size_t nfp = (size_t)cfg->nf * cfg->nf;
     if ((rc = dev_alloc(ws, (void**)&ws->spill, (nfp ? nfp : 1) * sizeof(int)))) return fail(rc);
     if ((rc = dev_alloc(ws, (void**)&ws->spill_ctr, kCounters * sizeof(int)))) return fail(rc);
-    // per-tile displacement bounds: a deposition tile takes the largest of
-    // its 3 x 3 neighbourhood, which holds every coarse particle a fine
-    // particle within the largest halo + 1 cells of the tile interpolates
-    // from when 2 coarseness + 10 <= tile side (a fine particle lies within
-    // 2 coarseness + 2 cells of its coarse neighbours, at the plasma edge)
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws->device) !=
         hipSuccess) {
@@ -561,7 +566,7 @@ int lcode_workspace_create(const lcode_config* cfg, lcode_workspace** out) {
     ws->cus = cus;
     ws->dep_plan = deposit_plan(N, cfg->plasma_coarseness, cfg->plasma_fineness, cus);
     const int nt = ws->dep_plan.nt;
-    if (kDepRegions && 2 * cfg->plasma_coarseness + kDepositHalo + 4 <= ws->dep_plan.tile) {
+    if (regions_hold(cfg, ws->dep_plan)) {
         ws->region_n = nt;
         if ((rc = dev_alloc(ws, (void**)&ws->regions, 2 * (size_t)nt * nt * sizeof(int))))
             return fail(rc);
@@ -895,7 +900,7 @@ static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
         a.halo_next = ws->spill_ctr + 2 + (1 - ws->bound_slot);
         if (ws->regions) {
             const size_t nr = (size_t)ws->region_n * ws->region_n;
-            a.halo_regions = ws->regions + ws->bound_slot * nr;
+            if (regions_hold(cfg, plan)) a.halo_regions = ws->regions + ws->bound_slot * nr;
             a.halo_regions_next = ws->regions + (1 - ws->bound_slot) * nr;
         }
     }
