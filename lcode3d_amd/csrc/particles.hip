@@ -437,7 +437,8 @@ deposit_tile_kernel(DepositArgs a) {
     // tiles and light ones; its last nsplit entries are the second parts of the
     // split tiles)
     const int ntx = a.ntx, lin = blockIdx.x;
-    const DepBlock blk = dep_block(a.tile_order, a.tile_order ? scalar((int)a.tile_order[lin]) : 0, lin);
+    const unsigned word = scalar(a.tile_order ? (int)a.tile_order[lin] : 0);
+    const DepBlock blk = dep_block(a.tile_order, word, lin);
     const int tile = blk.tile, slot = blk.slot, part = blk.part;
     const int nparts = slot >= 0 ? 2 : 1;
     const int ty = tile / ntx, tx = tile - ty * ntx;

@@ -28,11 +28,11 @@ inline unsigned dep_entry(int tile, int slot, int part) {
 // Whether the tiles and slots of a launch fit the table's words.
 inline bool dep_entries_fit(int tiles, int nsplit) { return tiles <= 65536 && nsplit <= 32767; }
 
-// Block `lin`: its word, or without a table its own index as the tile (a grid
-// without a table may have more tiles than a word holds).
+// Block `lin` by its word, or without a table by the word 0 and its own index as the
+// tile (a grid without a table may have more tiles than a word holds).
 LCODE_TILE_FN DepBlock dep_block(bool table, unsigned word, int lin) {
-    if (!table) return DepBlock{lin, -1, 0};
-    return DepBlock{(int)(word & 0xFFFFu), (int)(word >> 16 & 0x7FFFu) - 1, (int)(word >> 31)};
+    return DepBlock{(int)(word & 0xFFFFu) + (table ? 0 : lin), (int)(word >> 16 & 0x7FFFu) - 1,
+                    (int)(word >> 31)};
 }
 
 // Squared distance of tile t (row-major in an nt x nt grid of tiles) from
