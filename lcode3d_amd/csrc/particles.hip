@@ -733,15 +733,17 @@ deposit_tile_kernel(DepositArgs a) {
                 const int ci = xi.z, cj = xj.z;   // initial cell
                 const bool home = ((unsigned)(ci - ci0) < (unsigned)T) &
                                   ((unsigned)(cj - cj0) < (unsigned)T);
-                // (NaN where the position is not finite; further than kFarCells counts
-                // as that, which the halo test below finds but for a centre that is
-                // clamped first)
-                bool odd = __builtin_isunordered(xl, yl);
-                if (is_edge && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2)) {
-                    odd |= !(fabs(xh) <= kFarCells && fabs(yh) <= kFarCells);
-                    if (home && !odd) atomicAdd(a.fault, 1);
-                    ti = min(max(ti, 1), N - 2);
-                    tj = min(max(tj, 1), N - 2);
+                // (NaN where the position is not finite)
+                const bool odd = __builtin_isunordered(xl, yl);
+                if (is_edge && !odd && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2)) {
+                    // (a centre further than kFarCells stays as it is: beyond the halo)
+                    constexpr int kFar = (int)kFarCells;
+                    if ((unsigned)ti - ih + kFar < 2u * kFar &&
+                        (unsigned)tj - ih + kFar < 2u * kFar) {
+                        if (home) atomicAdd(a.fault, 1);
+                        ti = min(max(ti, 1), N - 2);
+                        tj = min(max(tj, 1), N - 2);
+                    }
                 }
                 if (q == 0) swap = yl >= roomy;
                 if (odd | ((unsigned)(ti - ci + halo) > 2u * halo) |
