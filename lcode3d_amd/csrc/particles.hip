@@ -1100,11 +1100,17 @@ DepositPlan deposit_plan(int N, int coarseness, int fineness, int cus) {
     p.nt = (N + p.tile - 1) / p.tile;
     p.waves = p.tile == 24 && p.nt * p.nt > 3 * cus ? 4 : 3;
     const int ext = p.tile + 2 * kDepositHalo + 2;   // initial cells per side, at most
-    p.fine_max = std::max(fineness, 3) * ext;        // (a denser grid than configured fits too)
     // the coarse rectangle of a tile has at most ext / coarseness + 3 rows;
     // staged while three blocks share a CU's LDS
+    p.fine_max = std::max(fineness, 3) * ext;
     p.coarse_max = ext / coarseness + 3;
     p.staged = deposit_lds_bytes(p.tile, p.fine_max, p.coarse_max) <= 53 * 1024;
+    // The tables also take grids denser than the config says (the caller makes them):
+    // 18 coarse rows and 128 fine indices, or 15 and no more of these where four
+    // blocks share the LDS (more took a block of each CU: 1281^2 995 -> 1052 us a
+    // step).  A denser tile is a fault.
+    if (p.staged) p.coarse_max = std::max(p.coarse_max, p.waves == 4 ? 15 : 18);
+    if (!p.staged || p.waves == 3) p.fine_max = std::max(p.fine_max, 128);
     return p;
 }
 
