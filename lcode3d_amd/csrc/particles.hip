@@ -264,13 +264,28 @@ __device__ __forceinline__ void fine_particle(const DepositArgs& a, int fi, int 
 
 constexpr int kDepBlock = 256;   // threads of a deposition tile's block
 
+// x / h + .5, its product rounded before the sum as the reference rounds its
+// quotient (lcode.py:404): far from the axis a product left unrounded moves the
+// weights by 1e-14 against it.
+__device__ __forceinline__ double in_cells(double x, double inv_h) {
+#pragma clang fp contract(off)
+    const double q = x * inv_h;
+    return q + .5;
+}
+
+// The cell of a fine particle, at its initial position or displaced: one rule for both,
+// or a particle at rest on a cell's edge would seem to have moved.
+__device__ __forceinline__ int dep_cell(double x, int N, double inv_h) {
+    return (int)floor(in_cells(x, inv_h)) + N / 2;
+}
+
 // First fine index whose initial cell is >= c (fg is increasing).
 __device__ int first_fine_at_or_after(const double* fg, int nf, int c, int N,
-                                      double h) {
+                                      double inv_h) {
     int lo = 0, hi = nf;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (cell_of(fg[mid], N, h) < c) lo = mid + 1; else hi = mid;
+        if (dep_cell(fg[mid], N, inv_h) < c) lo = mid + 1; else hi = mid;
     }
     return lo;
 }
@@ -370,22 +385,13 @@ inline size_t deposit_lds_bytes(int T, int fine_max, int coarse_max) {
 // First fine index whose initial cell is >= c (fg is increasing), from this
 // lane's sample of a 64-entry window at w0 (the cell of entry w0 + lane), else
 // by search.  Every lane of the wave calls it.
-__device__ __forceinline__ int wave_first_fine(const double* fg, int nf, int c, int N, double h,
+__device__ __forceinline__ int wave_first_fine(const double* fg, int nf, int c, int N, double inv_h,
                                                int w0, int sample) {
     const int lane = threadIdx.x & 63;
     const int n = __popcll(__ballot(w0 + lane < nf && sample < c));
     const bool open_left = n > 0 || w0 == 0, open_right = n < 64 || w0 + 64 >= nf;
     if (open_left && open_right) return min(w0 + n, nf);
-    return first_fine_at_or_after(fg, nf, c, N, h);
-}
-
-// x / h + .5, its product rounded before the sum as the reference rounds its
-// quotient (lcode.py:404): far from the axis a product left unrounded moves the
-// weights by 1e-14 against it.
-__device__ __forceinline__ double in_cells(double x, double inv_h) {
-#pragma clang fp contract(off)
-    const double q = x * inv_h;
-    return q + .5;
+    return first_fine_at_or_after(fg, nf, c, N, inv_h);
 }
 
 // gamma = sqrt(s) and 1 / (gamma - pz) to about an ulp, without the compiler's
@@ -457,7 +463,7 @@ deposit_tile_kernel(DepositArgs a) {
     if (a.nf > 0) {
         const int k = min(w0 + lane, a.nf - 1);
         sample_c = (int)neighbour[k];
-        sample = cell_of(a.fg[k], N, a.h);
+        sample = dep_cell(a.fg[k], N, inv_h);
     }
     // halo: the displacement bound of the last pushes when one is given.
     // A fine particle's offset is a convex mix of coarse offsets, so its
@@ -499,7 +505,7 @@ deposit_tile_kernel(DepositArgs a) {
     const int ext = T + 2 * halo + 2;
     if (wave < 4) {
         const int lo = (wave < 2 ? ci0 : cj0) - 1 - halo;
-        const int r = wave_first_fine(a.fg, a.nf, lo + (last_end ? ext : 0), N, a.h, w0, sample);
+        const int r = wave_first_fine(a.fg, a.nf, lo + (last_end ? ext : 0), N, inv_h, w0, sample);
         // the coarse neighbour of the range's first (last) fine index
         const int at = min(max(last_end ? r - 1 : r, 0), max(a.nf - 1, 0));
         int c = __shfl(sample_c, at - w0, 64);
@@ -576,7 +582,7 @@ deposit_tile_kernel(DepositArgs a) {
             l.fi[s] = v.fg;
             l.xi[s] = make_int4(min(max(v.P - lo, 0), hi) * scale,
                                 min(max(v.Nn - lo, 0), hi) * scale,
-                                cell_of(v.fg, N, a.h), 0);
+                                dep_cell(v.fg, N, inv_h), 0);
         };
         // 16 x 16 threads over the rectangle; every thread's first entries of both
         // tables on their way together, the rest (large ranges) in turn
