@@ -271,9 +271,13 @@ template <typename V> struct Dft<16, V> {
 __host__ __device__ constexpr int root_count(int R) { return (R < 4 ? R : 4) - 1 + (R + 3) / 4 - 1; }
 
 // The plan of radices R1; r[0 .. nst).  A constant for the lengths with kernels of their
-// own (static_fft: powers of two and 5 times one, the usual grids), whose index
-// arithmetic then folds away.  A + C of six fields, us, the same plan from kernel
+// own (static_fft: the powers of two from 64 to 2048 and 640, 1280 and 2560, the grids
+// that a run is refined through by halving its step), whose index arithmetic then
+// folds away.  A + C of six fields, us, the same plan from kernel
 // arguments and as a constant: 129^2 14.8 and 12.4, 257^2 19.9 and 17.1, 641^2 41.5 and 38.9.
+// The rest of the two families gains nothing by it and has none: 80, 160 and 320 (their
+// grids are a block's chain; a step 81^2 81.8 and 81.9, 161^2 93.0 and 93.0) and 4096
+// (memory; six FP32 solves at 2049^2 440.8 and 440.7).
 __host__ __device__ constexpr FftPlan make_plan(int L, int R1, int nst, const int* r) {
     FftPlan p{};
     p.L = L;
