@@ -851,17 +851,18 @@ static DepositArgs deposit_args(const lcode_config* cfg,
     return a;
 }
 
-// What a deposition sizes its tiles' halo by: the bounds the workspace's pushes
-// raised, or the bound of its own offsets (a deposition on its own, whose
-// particles may come from anywhere).
-enum HaloBound { HALO_OF_PUSHES, HALO_OF_OFFSETS };
+// What a deposition sizes its tiles' halo by: the largest halo, the bounds the
+// workspace's pushes raised, or the bound of its own offsets (a deposition on
+// its own, whose particles may come from anywhere).
+enum HaloBound { HALO_LARGEST, HALO_OF_PUSHES, HALO_OF_OFFSETS };
 
 static int do_deposit(lcode_workspace* ws, const lcode_config* cfg,
                       const double* ro_initial, const double* xo,
                       const double* yo, const double* m, const double* q,
                       const double* px, const double* py, const double* pz,
                       const lcode_virt_params* vp, double* const out[4],
-                      hipStream_t stream, HaloBound halo, Gate gate = Gate{nullptr, 0.}) {
+                      hipStream_t stream, Gate gate = Gate{nullptr, 0.},
+                      HaloBound halo = HALO_LARGEST) {
     // (a workspace may serve other coarseness and fineness values than its own)
     const DepositPlan plan = deposit_plan(ws->N, cfg->plasma_coarseness, cfg->plasma_fineness,
                                           ws->cus);
@@ -972,7 +973,7 @@ int lcode_deposit(lcode_workspace* ws, const lcode_config* cfg,
     LCODE_REQUIRE(virt_params && out, "NULL virt_params/out");
     for (int k = 0; k < 4; ++k) LCODE_REQUIRE(out[k], "NULL output");
     return do_deposit(ws, cfg, ro_initial, x_offt, y_offt, m, q, px, py, pz,
-                      virt_params, out, stream, HALO_OF_OFFSETS);
+                      virt_params, out, stream, Gate{nullptr, 0.}, HALO_OF_OFFSETS);
 }
 
 }  // extern "C"
@@ -1184,7 +1185,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     // 3: deposit (lcode.py:856-859)
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p1[0], ws->p1[1], c->m,
                          c->q, ws->p1[2], ws->p1[3], ws->p1[4], vp, ws->dep,
-                         stream, HALO_OF_PUSHES)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     // 4: fields with prev fields in the trick term; only the averages are
     // used afterwards (lcode.py:862-881)
@@ -1207,7 +1208,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     // 6: deposit (lcode.py:890-891)
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, HALO_OF_PUSHES)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     // 7: fields with the pass-1 averages in the trick term; the solved
     // fields are the step's output (lcode.py:893-911, :927-928).  The
@@ -1231,7 +1232,7 @@ static int step_impl(lcode_workspace* ws, const lcode_config* cfg,
     double* const outD[4] = {out->ro, out->jx, out->jy, out->jz};
     return do_deposit(ws, cfg, c->ro_initial, out->x_offt, out->y_offt, c->m,
                       c->q, out->px, out->py, out->pz, vp, outD, stream,
-                      HALO_OF_PUSHES);
+                      Gate{nullptr, 0.}, HALO_OF_PUSHES);
 }
 
 static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
@@ -1290,7 +1291,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
         return rc;
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, HALO_OF_PUSHES)))
+                         stream, Gate{nullptr, 0.}, HALO_OF_PUSHES)))
         return rc;
     if ((rc = field_pass(ws, cfg, prev, trick_avg, beam_ro, beam_scalar,
                          ws->dep, outF, ws->favg, stream, Gate{nullptr, 0.},
@@ -1317,7 +1318,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
         return rc;
     if ((rc = do_deposit(ws, cfg, c->ro_initial, ws->p2[0], ws->p2[1], c->m,
                          c->q, ws->p2[2], ws->p2[3], ws->p2[4], vp, ws->dep,
-                         stream, HALO_OF_PUSHES, fallback)))
+                         stream, fallback, HALO_OF_PUSHES)))
         return rc;
     if ((rc = field_pass(ws, cfg, prev, trick_avg, beam_ro, beam_scalar,
                          ws->dep, outF, ws->favg, stream, fallback)))
@@ -1332,7 +1333,7 @@ static int guided_impl(lcode_workspace* ws, const lcode_config* cfg,
     double* const outD[4] = {out->ro, out->jx, out->jy, out->jz};
     return do_deposit(ws, cfg, c->ro_initial, out->x_offt, out->y_offt, c->m,
                       c->q, out->px, out->py, out->pz, vp, outD, stream,
-                      HALO_OF_PUSHES);
+                      Gate{nullptr, 0.}, HALO_OF_PUSHES);
 }
 
 // ws->grid32 for the duration of one call
