@@ -136,7 +136,12 @@ constexpr int kDepOrder = LCODE_DEP_ORDER;
 // once, at the tile blocks per CU the runtime reports for the kernel, or
 // kDepResident when it reports none; 0: none).  The tiles nearest the grid centre
 // are split: an axisymmetric beam's wake compresses and displaces the plasma
-// there, so those tiles have the largest halos and the most particles.
+// there, so those tiles have the largest halos and the most particles.  us per launch
+// in a step, displacements to 1.2 cells, split / not: 24-cell tiles 641^2 32.6 / 33.7
+// (in the developed wake 39.3 / 43.2 before the tiles' start was shortened), 601^2
+// 32.2 / 33.2; 16-cell tiles 217^2 15.0 / 16.6, 257^2 16.0 / 16.8, 361^2 19.9 / 18.4;
+// 8-cell tiles, all of them split, 129^2 11.5 / 10.4, 193^2 13.2 / 13.1: it does not
+// pay where a tile is little more than its start.
 #ifndef LCODE_DEP_SPLIT
 #define LCODE_DEP_SPLIT -1
 #endif

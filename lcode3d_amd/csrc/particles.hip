@@ -1109,9 +1109,22 @@ int deposit_blocks_per_cu(const DepositPlan& p) {
 }
 
 // Small grids take small tiles: 24-cell ones would leave CUs idle (36 tiles at
-// 129^2) and the launch as long as the chain of one tile.  us per launch, 24 /
-// 16 / 8 cells: 129^2 25.3 / - / 12.3, 361^2 28.8 / 20.5 / -, 641^2 34.7 / 46.6 /
-// -; larger tiles than 24 leave too few blocks at 641^2 or too few registers
+// 129^2) and the launch as long as the chain of one tile.  us per launch in a step,
+// fineness 2, displacements to 1.2 cells, 8 / 16 / 24 cells a side:
+//   coarseness 2 (24 cells: not staged)      coarseness 3
+//   129^2  11.5 / 13.6 / 23.3                181^2  11.6 / 13.2 / 17.5
+//   193^2  13.2 / 14.5 / 23.2                201^2  12.9 / 14.0 / 17.7
+//   217^2  12.3 / 15.0 / 24.8                217^2  12.4 / 14.2 / 18.2
+//   257^2  17.5 / 16.0 / 25.6                241^2  16.6 / 14.9 / 18.8
+//   321^2  24.5 / 18.3 / 27.3                385^2  31.8 / 19.3 / 23.0
+//   401^2  35.0 / 20.5 / 32.3                433^2  39.3 / 22.3 / 24.8
+//   541^2     - / 33.2 / 40.8                481^2     - / 28.6 / 27.1
+//   641^2     - / 43.7 / 46.8                641^2     - / 42.9 / 32.6
+// (coarseness 3 up to 433^2: 0.5 cells.)  The sides cross where the smaller tiles take
+// a second round of the block slots (8 cells beyond 216^2, 16 cells beyond 432^2 on
+// 256 CUs with three blocks each); the lines at 200 and 400 lie a little below, and
+// take no account of the CUs or the coarseness.
+// Tiles larger than 24 cells leave too few blocks at 641^2 or too few registers
 // for the waves (32 cells with 8 waves 34.8 - 52).  In launches of several
 // rounds four waves per SIMD hide more of a tile's start than three (1281^2,
 // fineness 3: 190 -> 178), in one round they leave the same waves and fewer
@@ -1123,7 +1136,8 @@ DepositPlan deposit_plan(int N, int coarseness, int fineness, int cus) {
     p.waves = p.tile == 24 && p.nt * p.nt > 3 * cus ? 4 : 3;
     const int ext = p.tile + 2 * kDepositHalo + 2;   // initial cells per side, at most
     // the coarse rectangle of a tile has at most ext / coarseness + 3 rows;
-    // staged while three blocks share a CU's LDS
+    // staged while three blocks share a CU's LDS (not with 24 cells at coarseness 2,
+    // 54.7 KB with tables for fineness 3)
     p.fine_max = std::max(fineness, 3) * ext;
     p.coarse_max = ext / coarseness + 3;
     p.staged = deposit_lds_bytes(p.tile, p.fine_max, p.coarse_max) <= 53 * 1024;
