@@ -271,11 +271,14 @@ template <typename V> struct Dft<16, V> {
 __host__ __device__ constexpr int root_count(int R) { return (R < 4 ? R : 4) - 1 + (R + 3) / 4 - 1; }
 
 // The plan of radices R1; r[0 .. nst).  A constant for the lengths with kernels of their
-// own (static_fft: every power of two and five times one from 64 to 4096, the
-// grids that a run is refined through by halving its step), whose index arithmetic
-// then folds away.  The same plan from kernel arguments and as a constant, us: A + C of
-// six fields 129^2 14.8 and 12.4, 257^2 19.9 and 17.1, 641^2 41.5 and 38.9; a step at
-// 81^2 81.9 and 81.8, 161^2 93.0 and 90.4; six FP32 solves at 2049^2 442 and 433.
+// own (static_fft: the powers of two from 64 to 2048 and 640, 1280 and 2560, the grids
+// that a run is refined through by halving its step), whose index arithmetic then
+// folds away.  The same plan from kernel arguments and as a constant, us: A + C of
+// six fields 129^2 14.8 and 12.4, 257^2 19.9 and 17.1, 641^2 41.5 and 38.9.  The rest of
+// the two families, 80, 160, 320 and 4096, has none: a step at 81^2 81.9 and 81.8, at
+// 161^2 93.0 and 90.4, six FP32 solves at 2049^2 442 and 433, but with their 18 kernels in
+// the library the steps of other sizes took longer (641^2 with FP32 grids 198.0 -> 200.9,
+// FP64 217.4 -> 218.4, 361^2 143.2 -> 143.8).
 __host__ __device__ constexpr FftPlan make_plan(int L, int R1, int nst, const int* r) {
     FftPlan p{};
     p.L = L;
@@ -306,10 +309,9 @@ struct StaticFft {
     int L, R1, nst, r[3];
 };
 constexpr StaticFft kStaticFft[] = {
-    {64, 4, 2, {4, 4}},     {80, 8, 1, {10}},       {128, 4, 2, {4, 8}},   {160, 4, 2, {5, 8}},
-    {256, 4, 3, {4, 4, 4}}, {320, 8, 2, {5, 8}},    {512, 4, 3, {4, 4, 8}}, {640, 4, 3, {4, 4, 10}},
-    {1024, 8, 2, {8, 16}},  {1280, 10, 2, {16, 8}}, {2048, 8, 2, {16, 16}}, {2560, 10, 2, {16, 16}},
-    {4096, 16, 2, {16, 16}},
+    {64, 4, 2, {4, 4}},    {128, 4, 2, {4, 8}},     {256, 4, 3, {4, 4, 4}},
+    {512, 4, 3, {4, 4, 8}}, {640, 4, 3, {4, 4, 10}}, {1024, 8, 2, {8, 16}},
+    {1280, 10, 2, {16, 8}}, {2048, 8, 2, {16, 16}},  {2560, 10, 2, {16, 16}},
 };
 constexpr int static_fft(int L) {   // index, or -1
     for (int k = 0; k < (int)(sizeof(kStaticFft) / sizeof(kStaticFft[0])); ++k)
@@ -1269,14 +1271,10 @@ static int launch_solve_t(const SolverGeom& g, const SolveBatch& b,
     switch (g.fft.L) {
 #define LCODE_CASE(LL) \
     case LL: return launch_passes<kStaticFft[static_fft(LL)].R1, LL, S, G>(g, b, s, prof);
-        LCODE_CASE(64) LCODE_CASE(80) LCODE_CASE(128) LCODE_CASE(160) LCODE_CASE(256)
-        LCODE_CASE(320) LCODE_CASE(512) LCODE_CASE(640) LCODE_CASE(1024) LCODE_CASE(1280)
-        LCODE_CASE(2048) LCODE_CASE(2560)
+        LCODE_CASE(64) LCODE_CASE(128) LCODE_CASE(256) LCODE_CASE(512) LCODE_CASE(640)
+        LCODE_CASE(1024) LCODE_CASE(1280) LCODE_CASE(2048) LCODE_CASE(2560)
 #undef LCODE_CASE
     }
-    if constexpr (std::is_same<S, float>::value)   // (FP64 lengths end at 3640)
-        if (g.fft.L == 4096)
-            return launch_passes<kStaticFft[static_fft(4096)].R1, 4096, S, G>(g, b, s, prof);
     switch (g.fft.R1) {
         case 4: return launch_passes<4, 0, S, G>(g, b, s, prof);
         case 8: return launch_passes<8, 0, S, G>(g, b, s, prof);
