@@ -774,9 +774,8 @@ deposit_tile_kernel(DepositArgs a) {
                             if (!is_edge && !(ti >= 1 && ti <= N - 2 && tj >= 1 && tj <= N - 2))
                                 atomicAdd(a.fault, 1);
                             if (may_spill) {
-                                __hip_atomic_store(a.spill + atomicAdd(a.spill_count, 1),
-                                                   (fi_a + li) * a.nf + fj_a + lj,
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                a.spill[atomicAdd(a.spill_count, 1)] =
+                                    (fi_a + li) * a.nf + fj_a + lj;
                                 if (a.host_spill)
                                     __hip_atomic_store(a.host_spill, 1, __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_SYSTEM);
@@ -850,16 +849,6 @@ deposit_tile_kernel(DepositArgs a) {
             __syncthreads();
         }
     }
-    // a particle may have spilled somewhere (the bound every block read exceeds the
-    // largest halo) and no spill kernel follows: the last block to finish deposits the
-    // list onto the others' cells, which therefore travel as the split tiles' sums do,
-    // as device-scope atomic stores.  (A device-scope fence in every block: lcode_deposit
-    // at 193^2 with offsets just beyond the halo 70 us, now 25.)
-    const bool listed = a.spill_in_tiles && global > a.halo && !nonfinite;
-    auto put = [&](G* p, double v) {
-        if (listed) __hip_atomic_store(p, (G)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else *p = (G)v;
-    };
     // store the tile, adding the ion background to ro last (lcode.py:687)
     if (store) {
 #pragma unroll
@@ -873,35 +862,38 @@ deposit_tile_kernel(DepositArgs a) {
             G* const jx = gp<G>(a.jx);
             G* const jy = gp<G>(a.jy);
             G* const jz = gp<G>(a.jz);
-            if (overfull || nonfinite || tile_nan) {
-                const double nan = __builtin_nan("");
-                put(ro + idx, nan);
-                put(jx + idx, nan);
-                put(jy + idx, nan);
-                put(jz + idx, nan);
-                continue;
-            }
+            const bool bad = overfull || nonfinite || tile_nan;
+            const double nan = __builtin_nan("");
             const double* s = l.acc + r * D::kPitch + c;
             // the FP64 ion background is added in FP64, then rounded once
-            put(ro + idx, a.ro_initial ? s[0] + base[u] : s[0]);
-            put(jx + idx, s[D::kComp]);
-            put(jy + idx, s[2 * D::kComp]);
-            put(jz + idx, s[3 * D::kComp]);
+            ro[idx] = (G)(bad ? nan : a.ro_initial ? s[0] + base[u] : s[0]);
+            jx[idx] = (G)(bad ? nan : s[D::kComp]);
+            jy[idx] = (G)(bad ? nan : s[2 * D::kComp]);
+            jz[idx] = (G)(bad ? nan : s[3 * D::kComp]);
         }
     }
-    if (listed) {
+    // a particle may have spilled somewhere (the bound every block read exceeds the
+    // largest halo) and no spill kernel follows: the last block to finish, after every
+    // block's stores are visible, deposits the list.  One thread makes the block's
+    // stores visible (they are complete at the barrier): a fence in every wave, which
+    // also drops the XCD's L2, took lcode_deposit at 193^2 with offsets just beyond the
+    // halo 71 us instead of 28.5, a step there with spills 282 instead of 146.
+    // (Device-scope atomic stores without a fence: 25.4 and 119, but 0.2 us more in
+    // every launch with 8- and 16-cell tiles, which take them by a branch.)
+    if (a.spill_in_tiles && global > a.halo && !nonfinite) {
         __builtin_amdgcn_s_waitcnt(0);   // this wave's stores are complete
         __syncthreads();
-        if (threadIdx.x == 0)
+        if (threadIdx.x == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             last_block = atomicAdd(a.done, 1) == (int)gridDim.x - 1;
+        }
         __syncthreads();
         if (last_block) {
-            __threadfence();   // nothing of the other blocks' cells from a stale line
+            __threadfence();
             const int count = __hip_atomic_load(a.spill_count, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
             for (int p = threadIdx.x; p < count; p += kDepBlock)
-                deposit_spill_one<G>(a, __hip_atomic_load(a.spill + p, __ATOMIC_RELAXED,
-                                                          __HIP_MEMORY_SCOPE_AGENT), N);
+                deposit_spill_one<G>(a, a.spill[p], N);
             if (threadIdx.x == 0) *a.done = 0;
         }
     }
