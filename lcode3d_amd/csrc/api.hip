@@ -1,5 +1,5 @@
-// C ABI of the gfx950 LCODE 3D step: workspace (the eigenvalue tables the
-// reference memoizes with cp.memoize, FFT twiddles, scratch), the
+// C ABI of the gfx950 LCODE 3D step: workspace (the solver's tables, which the
+// reference memoizes with cp.memoize, roots of unity, scratch), the
 // standalone operators and the fused xi step (lcode.py:828-931).
 
 #include <hip/hip_runtime.h>

@@ -335,8 +335,9 @@ __device__ __forceinline__ void deposit_spill_one(const DepositArgs& a, int fk, 
 // rectangle, then the stores - and the launch), the rest is the chain of a
 // particle: two rounds of LDS reads and about 60 dependent FP64 operations, with
 // three waves per SIMD to overlap it (VALU issue 62 % of that time, LDS 40 %).
-// us per launch before / now: 129^2 25.3 / 12.4, 361^2 28.8 / 20.8, 641^2 39.9 /
-// 34.8, 1281^2 with fineness 3 231 / 182.  Tried at 641^2 and slower: strips of
+// us per launch with 24-cell tiles everywhere and a longer start / now: 129^2 25.3 /
+// 12.3, 361^2 28.8 / 20.0, 641^2 39.9 / 33.6, 1281^2 with fineness 3 231 / 167 (VALU issue
+// 70 % there).  Tried at 641^2 and slower: strips of
 // particles along j whose sums slide with the centre (61 us: the lanes leave
 // their columns at different steps), 5 waves per block (44 - 65), 32-cell tiles
 // with 8 waves (35 - 52).
@@ -918,9 +919,10 @@ deposit_spill_kernel(DepositArgs a) {
 // *bound to the cells that the coarse offsets move a particle at most, or to
 // halo + 1 (which sends the deposition to its largest halo and the spill list)
 // when an offset is not finite or larger, or when an interpolation weight would
-// let a fine particle move further than its coarse ones.  4 us at 641^2,
-// against the largest halo's three times as many particles per tile and a
-// device-wide fence in every block (lcode_deposit 122 -> 39 us).
+// let a fine particle move further than its coarse ones.  At 641^2 it takes 7 of
+// lcode_deposit's 39 us, which took 122 with the largest halo's three times as many
+// particles per tile and a fence in every wave; with particles beyond that halo it is
+// what it costs (58 -> 63).
 __global__ void __launch_bounds__(kBlock)
 deposit_bound_kernel(DepositArgs a, int* bound) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
