@@ -151,8 +151,9 @@ int lcode_workspace_fault_count(lcode_workspace *ws, hipStream_t stream,
  * not synchronise: it reads a host-visible flag that the pushes and the
  * deposition set, so a kernel still running has not reported yet (after a
  * stream synchronisation every finished kernel has).  When the flag is set
- * the depositions that met it wrote NaN grids instead of depositing, and
- * everything computed from them is NaN.  reset != 0 clears it.  The
+ * the step depositions that met it wrote NaN grids instead of depositing
+ * (lcode_deposit: NaN in the tiles of the particles that interpolate from it),
+ * and everything computed from them is NaN.  reset != 0 clears it.  The
  * reference has no such check: a NaN particle there deposits at an
  * undefined cell or faults. */
 int lcode_workspace_nonfinite(lcode_workspace *ws, int32_t reset,
